@@ -1,5 +1,5 @@
 // diagonalize_hsp_and_H11(opt = 0) on the device (src/module_gradient.f90:158-453)
-// and the eigenvalue solver behind it.
+// (its eigenvalue solver is that of tg_eig.hip).
 //
 // For every resident state (U, V real):
 //   rho = V V^T, kappa = V U^T                       (calculate_densities_real)
@@ -14,16 +14,10 @@
 // upper triangles read), ascending.  The gradient recipes of calculate_gradient
 // (:97-120) turn the extreme eigenvalues into the step parameters eta, mu.
 //
-// Eigenvalues: one workgroup per symmetric matrix.  Householder reduction to
-// tridiagonal form (the reflector of each column from its sub-diagonal part,
-// p = tau A v, w = p - (tau/2)(p.v) v, A -= v w^T + w v^T), with the matrix in
-// LDS up to order EIG_NL and in global memory (L2) beyond; then every
-// eigenvalue by bisection on Sturm sequence counts of the tridiagonal matrix,
-// one thread per eigenvalue index, to the resolution of the floating-point
-// numbers.
+// Eigenvalues: the panel reduction of the eigen-solver and multisection on Sturm
+// counts (batched_sym_eigvals, tg_eig.hip).
 #include <algorithm>
 #include <cmath>
-#include <cfloat>
 #include <vector>
 
 #include "tg_internal.h"
@@ -31,149 +25,8 @@
 namespace {
 
 constexpr int NT = 256;
-constexpr int EIG_TH = 256;
-constexpr int EIG_NL = 112;          // matrices up to this order stay in LDS
 
 inline unsigned nblk(long long tot) { return (unsigned)((tot + NT - 1) / NT); }
-
-__device__ inline double wave_sum(double v) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-
-template <int TH>
-__device__ inline double block_sum(double v, double* red) {
-  v = wave_sum(v);
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  __syncthreads();
-  if (lane == 0) red[wid] = v;
-  __syncthreads();
-  double s = 0.0;
-#pragma unroll
-  for (int q = 0; q < TH / 64; ++q) s += red[q];
-  return s;
-}
-
-// number of eigenvalues of the tridiagonal (d, e2 = e^2) below x
-__device__ inline int sturm_count(int n, const double* d, const double* e2, double x, double pivmin) {
-  int cnt = 0;
-  double q = d[0] - x;
-  if (q <= pivmin) { ++cnt; q = fmin(q, -pivmin); }
-  for (int j = 1; j < n; ++j) {
-    q = d[j] - x - e2[j - 1] / q;
-    if (q <= pivmin) { ++cnt; q = fmin(q, -pivmin); }
-  }
-  return cnt;
-}
-
-// M: n x n symmetric matrix (leading dimension ldm; LDS or global), destroyed.
-// d, e2, v, p: LDS vectors of n.  Writes the n eigenvalues, ascending, to w.
-template <int TH>
-__device__ void sym_eigvals(int n, double* M, int ldm, double* d, double* e2, double* v, double* p,
-                            double* red, double* __restrict__ w) {
-  const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
-  constexpr int NW = TH / 64;
-  for (int k = 0; k + 2 < n; ++k) {
-    const int m = n - k - 1;
-    double s2 = 0.0;
-    for (int i = t; i < m; i += TH) {
-      const double x = M[(k + 1 + i) + (long long)k * ldm];
-      v[i] = x;
-      if (i > 0) s2 = fma(x, x, s2);
-    }
-    s2 = block_sum<TH>(s2, red);      // (barrier inside: v visible)
-    const double alpha = v[0];
-    if (t == 0) d[k] = M[k + (long long)k * ldm];
-    if (s2 == 0.0) {
-      if (t == 0) e2[k] = alpha * alpha;
-      __syncthreads();
-      continue;
-    }
-    const double beta = -copysign(sqrt(fma(alpha, alpha, s2)), alpha);
-    const double tau = (beta - alpha) / beta;
-    const double scale = 1.0 / (alpha - beta);
-    if (t == 0) e2[k] = beta * beta;
-    __syncthreads();
-    for (int i = t; i < m; i += TH) v[i] = (i == 0) ? 1.0 : v[i] * scale;
-    __syncthreads();
-    // p = tau A22 v (A22 symmetric: column j dotted with v, one wave per column)
-    for (int j = wid; j < m; j += NW) {
-      const double* col = M + (k + 1) + (long long)(k + 1 + j) * ldm;
-      double acc = 0.0;
-      for (int i = lane; i < m; i += 64) acc = fma(col[i], v[i], acc);
-      acc = wave_sum(acc);
-      if (lane == 0) p[j] = tau * acc;
-    }
-    __syncthreads();
-    double dot = 0.0;
-    for (int i = t; i < m; i += TH) dot = fma(p[i], v[i], dot);
-    dot = block_sum<TH>(dot, red);
-    const double K = 0.5 * tau * dot;
-    for (int i = t; i < m; i += TH) p[i] = fma(-K, v[i], p[i]);
-    __syncthreads();
-    // A22 -= v w^T + w v^T
-    const long long mm = (long long)m * m;
-    for (long long idx = t; idx < mm; idx += TH) {
-      const int i = (int)(idx % m), j = (int)(idx / m);
-      double* a = M + (k + 1 + i) + (long long)(k + 1 + j) * ldm;
-      *a = fma(-v[i], p[j], fma(-p[i], v[j], *a));
-    }
-    __syncthreads();
-  }
-  if (t == 0) {
-    if (n >= 2) {
-      d[n - 2] = M[(n - 2) + (long long)(n - 2) * ldm];
-      const double en = M[(n - 1) + (long long)(n - 2) * ldm];
-      e2[n - 2] = en * en;
-    }
-    d[n - 1] = M[(n - 1) + (long long)(n - 1) * ldm];
-  }
-  __syncthreads();
-  // Gershgorin interval and the pivot guard of the Sturm counts
-  double gl = DBL_MAX, gu = -DBL_MAX, emax2 = 0.0;
-  for (int i = 0; i < n; ++i) {
-    const double el = (i > 0) ? sqrt(e2[i - 1]) : 0.0, er = (i + 1 < n) ? sqrt(e2[i]) : 0.0;
-    gl = fmin(gl, d[i] - el - er);
-    gu = fmax(gu, d[i] + el + er);
-    if (i + 1 < n) emax2 = fmax(emax2, e2[i]);
-  }
-  const double pivmin = DBL_MIN * fmax(1.0, emax2);
-  const double span = fmax(fabs(gl), fabs(gu));
-  gl -= 2.0 * DBL_EPSILON * span * n + pivmin;
-  gu += 2.0 * DBL_EPSILON * span * n + pivmin;
-  for (int i = t; i < n; i += TH) {
-    double lo = gl, hi = gu;
-    for (int it = 0; it < 256; ++it) {
-      const double mid = 0.5 * (lo + hi);
-      if (!(mid > lo && mid < hi)) break;
-      if (sturm_count(n, d, e2, mid, pivmin) > i) hi = mid;
-      else lo = mid;
-    }
-    w[i] = 0.5 * (lo + hi);
-  }
-}
-
-// count matrices: A + b * sA (upper triangle read, ld lda), work + b * n * n
-// (global work for n > EIG_NL), eigenvalues at w + b * ws.
-template <int TH, bool LDSM>
-__global__ void __launch_bounds__(TH)
-sym_eigvals_kernel(int n, const double* __restrict__ A0, int lda, long long sA,
-                   double* __restrict__ work, double* __restrict__ w0, long long ws) {
-  __shared__ double Ml[LDSM ? EIG_NL * EIG_NL : 1];
-  __shared__ double vecs[4 * (LDSM ? EIG_NL : 512)];
-  __shared__ double red[TH / 64];
-  const double* A = A0 + blockIdx.x * sA;
-  double* M = LDSM ? Ml : work + (long long)blockIdx.x * n * n;
-  const long long nn = (long long)n * n;
-  for (long long idx = threadIdx.x; idx < nn; idx += TH) {
-    const int i = (int)(idx % n), j = (int)(idx / n);
-    M[idx] = (i <= j) ? A[i + (long long)j * lda] : A[j + (long long)i * lda];
-  }
-  __syncthreads();
-  const int cap = LDSM ? EIG_NL : 512;
-  sym_eigvals<TH>(n, M, n, vecs, vecs + cap, vecs + 2 * cap, vecs + 3 * cap, red,
-                  w0 + blockIdx.x * ws);
-}
 
 // ---- pieces of H11 and of the constraint terms ----------------------------
 
@@ -245,25 +98,6 @@ sub_f11_kernel(int n, int m, const double* __restrict__ lam0, const double* __re
 
 }  // namespace
 
-// batched eigenvalues of symmetric matrices (upper triangles read); work: count
-// n*n doubles when n > EIG_NL (else unused, may be null)
-int batched_sym_eigvals(hipStream_t s, int n, const double* A, int lda, long long sA, int count,
-                        double* work, double* w, long long ws) {
-  if (count <= 0 || n <= 0) return TG_OK;
-  if (n > 512) {
-    tg_set_error("batched_sym_eigvals: order above 512");
-    return TG_E_UNSUPPORTED;
-  }
-  if (n <= EIG_NL)
-    hipLaunchKernelGGL((sym_eigvals_kernel<EIG_TH, true>), dim3(count), dim3(EIG_TH), 0, s, n, A,
-                       lda, sA, work, w, ws);
-  else
-    hipLaunchKernelGGL((sym_eigvals_kernel<EIG_TH, false>), dim3(count), dim3(EIG_TH), 0, s, n, A,
-                       lda, sA, work, w, ws);
-  TG_HIP(hipGetLastError());
-  return TG_OK;
-}
-
 // Step parameters of calculate_gradient for gradient_type 1 (from the H11
 // spectrum) and 2 (from the h spectrum), module_gradient.f90:97-120; type 0 or
 // a failed diagonalisation keep the input eta, mu.
@@ -299,9 +133,9 @@ int tg_hsp_h11_device(tg_ctx* c, const double* lam, std::vector<double>& eig, do
   const double* U = c->d_U.as<double>();
   const double* V = c->d_V.as<double>();
   // complex: rho, kappa, Gamma, DeltaLR, DeltaRL, h (S nn each); real: h, Delta,
-  // H11, X, A2, A3 (S nn each), eigen work (2 S nn), eigenvalues (2 S n)
+  // H11, X, A2, A3 (S nn each), eigen work (2 S (nn + 3 n)), eigenvalues (2 S n)
   const size_t cb = sizeof(cplx) * 6 * S * nn;
-  const size_t rb = sizeof(double) * (8 * (size_t)S * nn + 2 * (size_t)S * n);
+  const size_t rb = sizeof(double) * (6 * (size_t)S * nn + sym_eigvals_work(n, 2 * S) + 2 * (size_t)S * n);
   TG_TRY(c->d_a19.ensure(cb + rb));
   cplx* zr = c->d_a19.as<cplx>();
   cplx* zk = zr + S * nn;
@@ -315,8 +149,8 @@ int tg_hsp_h11_device(tg_ctx* c, const double* lam, std::vector<double>& eig, do
   double* X = rD + S * nn;
   double* A2 = X + S * nn;
   double* A3 = A2 + S * nn;
-  double* ew = A3 + S * nn;          // 2 S nn
-  double* ev = ew + 2 * S * nn;      // 2 S n
+  double* ew = A3 + S * nn;          // eigen work (and two S nn scratch matrices before)
+  double* ev = ew + sym_eigvals_work(n, 2 * S);   // 2 S n
   // rho = V V^T, kappa = V U^T, as complex inputs of the contraction
   TG_TRY(gemm_dd(s, OP_N, OP_T, n, n, n, 1.0, V, n, nn, V, n, nn, 0.0, X, n, nn, S));
   hipLaunchKernelGGL(real_to_cplx_kernel, dim3(nblk(S * nn)), dim3(NT), 0, s, S * nn, X, zr);

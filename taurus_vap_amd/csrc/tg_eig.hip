@@ -82,6 +82,19 @@ __device__ inline double block_max(double v, double* red) {
   return s;
 }
 
+template <int TH>
+__device__ inline double block_max_signed(double v, double* red) {
+  v = wave_max(v);
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  __syncthreads();
+  if (lane == 0) red[wid] = v;
+  __syncthreads();
+  double s = red[0];
+#pragma unroll
+  for (int q = 1; q < TH / 64; ++q) s = fmax(s, red[q]);
+  return s;
+}
+
 // 1/x from the hardware reciprocal and two Newton steps (the secular sums only
 // need the terms to a few ulps; the quotients that fix the eigenvectors divide)
 __device__ inline double recip(double x) {
@@ -103,7 +116,8 @@ __device__ inline double recip(double x) {
 constexpr int TD_TH = 512;
 constexpr int TD_NS = 4;        // column slices of the row products
 
-template <int TH, int PB>
+// VECS = false leaves the reflectors out (eigenvalues only).
+template <int TH, int PB, bool VECS>
 __global__ void __launch_bounds__(TH)
 tridiag_kernel(int n, const double* __restrict__ Ain, int lda, long long sA, double* __restrict__ A,
                double* __restrict__ Vm, double* __restrict__ d, double* __restrict__ e,
@@ -132,7 +146,7 @@ tridiag_kernel(int n, const double* __restrict__ Ain, int lda, long long sA, dou
     for (int i = t; i < n; i += TH) {
       const long long o = i + (long long)j * n;
       A[o] = (i <= j) ? src[i + (long long)j * lda] : src[j + (long long)i * lda];
-      Vm[o] = 0.0;
+      if (VECS) Vm[o] = 0.0;
     }
   __syncthreads();
   const int nref = n - 2;
@@ -188,7 +202,7 @@ tridiag_kernel(int n, const double* __restrict__ Ain, int lda, long long sA, dou
         const double vr = (r == 1) ? 1.0 : col[r] * scale;
         v[r - 1] = vr;
         Vp[(i + r) + j * n] = vr;
-        Vm[(i + r) + (long long)i * n] = vr;
+        if (VECS) Vm[(i + r) + (long long)i * n] = vr;
       }
       __syncthreads();
       // p = A22 v by rows over TD_NS column slices; t1 = W^T v, t2 = V^T v (LDS)
@@ -773,6 +787,86 @@ const MergePlan& merge_plan(int n) {
   return plans.emplace(n, std::move(P)).first->second;
 }
 
+// Householder reduction of count matrices (panel width by the LDS it takes)
+template <bool VECS>
+int tridiag_launch(hipStream_t s, int n, const double* A, int lda, long long sA, int count, double* Aw,
+                   double* Vm, double* d, double* e, double* tau) {
+  const int pb = n <= 384 ? 16 : (n <= 640 ? 8 : 4);
+  const size_t lds = sizeof(double) * ((3 + 2 * (size_t)pb + TD_NS) * n + 2 * pb + TD_TH / 64);
+  if (pb == 16)
+    hipLaunchKernelGGL((tridiag_kernel<TD_TH, 16, VECS>), dim3(count), dim3(TD_TH), lds, s, n, A, lda,
+                       sA, Aw, Vm, d, e, tau);
+  else if (pb == 8)
+    hipLaunchKernelGGL((tridiag_kernel<TD_TH, 8, VECS>), dim3(count), dim3(TD_TH), lds, s, n, A, lda,
+                       sA, Aw, Vm, d, e, tau);
+  else
+    hipLaunchKernelGGL((tridiag_kernel<TD_TH, 4, VECS>), dim3(count), dim3(TD_TH), lds, s, n, A, lda,
+                       sA, Aw, Vm, d, e, tau);
+  TG_HIP(hipGetLastError());
+  return TG_OK;
+}
+
+// Eigenvalues of tridiagonal matrices by multisection on Sturm counts, to the
+// resolution of the floating-point numbers.  A group of SG lanes takes one
+// eigenvalue index: each lane counts at one of SG points inside the bracket, so
+// a pass over the matrix leaves 1/(SG+1) of it (4.1 bits for SG = 16 against one
+// for a bisection); the counts are a serial chain of divisions, so the time is
+// passes x n x the latency of one division whatever the number of lanes.  SG_W
+// eigenvalues per workgroup, the rest of the chip taking the other indices.
+constexpr int SG = 16, SG_W = 16;
+__global__ void __launch_bounds__(SG * SG_W)
+sturm_kernel(int n, const double* __restrict__ d0, const double* __restrict__ e0,
+             double* __restrict__ w0, long long ws) {
+  extern __shared__ double sh[];
+  double* d = sh;
+  double* e2 = sh + n;
+  __shared__ double red[SG * SG_W / 64];
+  const int t = threadIdx.x;
+  const long long o = (long long)blockIdx.y * n;
+  double gl = DBL_MAX, gu = -DBL_MAX, em = 0.0;
+  for (int i = t; i < n; i += SG * SG_W) {
+    const double el = (i > 0) ? e0[o + i - 1] : 0.0, er = (i + 1 < n) ? e0[o + i] : 0.0;
+    const double di = d0[o + i], r = fabs(el) + fabs(er);
+    d[i] = di;
+    e2[i] = er * er;
+    gl = fmin(gl, di - r);
+    gu = fmax(gu, di + r);
+    em = fmax(em, er * er);
+  }
+  // Gershgorin interval and the pivot guard of the counts
+  gl = -block_max_signed<SG * SG_W>(-gl, red);
+  gu = block_max_signed<SG * SG_W>(gu, red);
+  em = block_max_signed<SG * SG_W>(em, red);
+  const double pivmin = DBL_MIN * fmax(1.0, em);
+  const double slack = 2.0 * DBL_EPSILON * fmax(fabs(gl), fabs(gu)) * n + pivmin;
+  double lo = gl - slack, hi = gu + slack;
+  const int i = blockIdx.x * SG_W + t / SG, g = t % SG;
+  const int ic = min(i, n - 1);                    // surplus groups repeat the last index
+  const int base = (t & 63) / SG * SG;
+  for (int it = 0; it < 64; ++it) {
+    const double mid = 0.5 * (lo + hi);
+    if (!(mid > lo && mid < hi)) break;            // uniform over the group
+    const double x = fma(hi - lo, (g + 1) * (1.0 / (SG + 1)), lo);
+    int cnt = 0;
+    double q = d[0] - x;
+    if (q <= pivmin) { ++cnt; q = fmin(q, -pivmin); }
+    for (int j = 1; j < n; ++j) {
+      q = d[j] - x - e2[j - 1] / q;
+      if (q <= pivmin) { ++cnt; q = fmin(q, -pivmin); }
+    }
+    // first point with more than i eigenvalues below it; the one before is the new lo
+    const unsigned long long all = __ballot(cnt > ic);
+    const unsigned m = (unsigned)(all >> base) & ((1u << SG) - 1);
+    const int f = m ? __ffs(m) - 1 : SG;
+    const double xl = __shfl(x, base + max(f - 1, 0), 64), xh = __shfl(x, base + min(f, SG - 1), 64);
+    if (f > 0) lo = fmax(lo, xl);
+    if (f < SG) hi = fmin(hi, xh);
+  }
+  // the counts do not resolve values within the pivot guard: these are zero
+  const double wv = 0.5 * (lo + hi);
+  if (g == 0 && i < n) w0[blockIdx.y * ws + i] = (fabs(wv) <= 2.0 * pivmin) ? 0.0 : wv;
+}
+
 }  // namespace
 
 size_t sym_eigensystem_work_bytes(int n, int count) {
@@ -782,6 +876,29 @@ size_t sym_eigensystem_work_bytes(int n, int count) {
                                           (size_t)std::max(1, npan) * EG_NB * EG_NB);
   const size_t ints = (size_t)3 * n + (size_t)count;
   return sizeof(double) * doubles + sizeof(int) * ints + 256;
+}
+
+// Eigenvalues only (upper triangles read), work of sym_eigvals_work(n, count)
+// doubles.  Two matrices of order 224 (h and H11 of one state) take 2.4 ms with the
+// host copies, 9.1 ms by the unblocked reduction with a rank-2 update per column
+// and one bisection per thread; that reduction with the matrix in LDS (order 112:
+// 1.81 ms) loses to this one at every order from 24 (0.19 against 0.24 ms) up
+// (order 112: 0.87 ms).
+int batched_sym_eigvals(hipStream_t s, int n, const double* A, int lda, long long sA, int count,
+                        double* work, double* w, long long ws) {
+  if (count <= 0 || n <= 0) return TG_OK;
+  if (n > 512) {
+    tg_set_error("batched_sym_eigvals: order above 512");
+    return TG_E_UNSUPPORTED;
+  }
+  double* d = work + (long long)count * n * n;
+  double* e = d + (long long)count * n;
+  double* tau = e + (long long)count * n;
+  TG_TRY(tridiag_launch<false>(s, n, A, lda, sA, count, work, nullptr, d, e, tau));
+  hipLaunchKernelGGL(sturm_kernel, dim3((n + SG_W - 1) / SG_W, count), dim3(SG * SG_W),
+                     sizeof(double) * 2 * n, s, n, d, e, w, ws);
+  TG_HIP(hipGetLastError());
+  return TG_OK;
 }
 
 int batched_sym_eigensystem(hipStream_t s, int n, const double* A, int lda, long long sA, int count,
@@ -808,20 +925,7 @@ int batched_sym_eigensystem(hipStream_t s, int n, const double* A, int lda, long
   const MergePlan& P = merge_plan(n);
   if (!P.desc.empty())
     TG_HIP(hipMemcpyAsync(idesc, P.desc.data(), sizeof(int) * P.desc.size(), hipMemcpyHostToDevice, s));
-  {
-    const int pb = n <= 384 ? 16 : (n <= 640 ? 8 : 4);
-    const size_t lds1 = sizeof(double) * ((3 + 2 * (size_t)pb + TD_NS) * n + 2 * pb + TD_TH / 64);
-    if (pb == 16)
-      hipLaunchKernelGGL((tridiag_kernel<TD_TH, 16>), dim3(count), dim3(TD_TH), lds1, s, n, A, lda, sA,
-                         Aw, Vm, d, e, tau);
-    else if (pb == 8)
-      hipLaunchKernelGGL((tridiag_kernel<TD_TH, 8>), dim3(count), dim3(TD_TH), lds1, s, n, A, lda, sA,
-                         Aw, Vm, d, e, tau);
-    else
-      hipLaunchKernelGGL((tridiag_kernel<TD_TH, 4>), dim3(count), dim3(TD_TH), lds1, s, n, A, lda, sA,
-                         Aw, Vm, d, e, tau);
-  }
-  TG_HIP(hipGetLastError());
+  TG_TRY(tridiag_launch<true>(s, n, A, lda, sA, count, Aw, Vm, d, e, tau));
   const unsigned gi = (unsigned)std::min<long long>((nn + EG_TH - 1) / EG_TH, 1024);
   hipLaunchKernelGGL(dc_init_kernel, dim3(gi, count), dim3(EG_TH), 0, s, n, d, e, wi, Z, dinfo);
   TG_HIP(hipGetLastError());

@@ -331,8 +331,6 @@ int tg_hsp_h11_device(tg_ctx* c, const double* lam, std::vector<double>& eig, do
 // eta, mu of calculate_gradient for gradient_type (module_gradient.f90:97-120)
 void gradient_recipe(int type, int n, const double* eig_hsp, const double* eig_h11, double eta0,
                      double mu0, double* eta, double* mu);
-// eigenvalues (ascending) of count symmetric matrices A + b sA (upper triangle
-// read) to w + b ws; work: count n^2 doubles for orders above 112
 // Eigenvalues (ascending, stride ws) and eigenvectors (n x n, stride sE) of count
 // symmetric matrices (upper triangles read), n <= 1024; work of
 // sym_eigensystem_work_bytes(n, count) bytes; info[k] != 0 when a secular root of
@@ -350,8 +348,11 @@ int canonical_launch(tg_ctx* c, hipStream_t s, double eps);
 int canonical_finish(tg_ctx* c, hipStream_t s, double eps, int* nocc, int* nemp, double* ovacc,
                      double* voveru);
 int upload_overlap_setup(tg_ctx* c, hipStream_t s);
+// eigenvalues (ascending) of count symmetric matrices A + b sA (upper triangle
+// read) to w + b ws; work: sym_eigvals_work(n, count) doubles
 int batched_sym_eigvals(hipStream_t s, int n, const double* A, int lda, long long sA, int count,
                         double* work, double* w, long long ws);
+inline size_t sym_eigvals_work(int n, int count) { return (size_t)count * ((size_t)n * n + 3 * (size_t)n); }
 // The resident U, V, D and c->st of c->ns states are set: the tail of
 // tg_set_states (Z buffers, gauge grid, state marked for the set-up upload).
 int tg_states_ready(tg_ctx* c);

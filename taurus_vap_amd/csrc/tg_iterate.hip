@@ -1032,7 +1032,7 @@ int tg_sym_eigenvalues(int n, int count, const double* A, int lda, double* w) {
   double *dA = nullptr, *dW = nullptr, *dw = nullptr;
   int r = TG_OK;
   if (hipMalloc(&dA, sizeof(double) * m * count) != hipSuccess ||
-      hipMalloc(&dW, sizeof(double) * (size_t)n * n * count) != hipSuccess ||
+      hipMalloc(&dW, sizeof(double) * sym_eigvals_work(n, count)) != hipSuccess ||
       hipMalloc(&dw, sizeof(double) * (size_t)n * count) != hipSuccess) {
     tg_set_error("tg_sym_eigenvalues: hipMalloc failed");
     r = TG_E_NOMEM;

@@ -105,3 +105,23 @@ def test_density_of_emax6_state():
     rho = V @ V.T
     w, Z = gpu.sym_eigensystem(rho)
     _check(rho, w, Z, "emax6 rho")
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 15, 16, 17, 33, 64, 385, 512])
+def test_eigenvalues_at_group_edges(n):
+    """sym_eigenvalues (panel reduction, multisection in groups of 16 lanes) on a
+    random, a diagonal, a zero and a doubly degenerate matrix: backward stable
+    reduction and exact counts leave an error of a few n eps |A|."""
+    from taurus_vap_amd import gpu
+    rng = np.random.default_rng(n)
+    x = rng.normal(size=(n, n))
+    q, _ = np.linalg.qr(rng.normal(size=(n, n)))
+    pairs = np.repeat(np.arange((n + 1) // 2, dtype=float), 2)[:n]
+    mats = np.stack([x + x.T, np.diag(np.linspace(-3.0, 5.0, n)), np.zeros((n, n)),
+                     (q * pairs) @ q.T])
+    w = gpu.sym_eigenvalues(mats)
+    for k in range(4):
+        a = np.triu(mats[k]) + np.triu(mats[k], 1).T
+        ref = np.linalg.eigvalsh(a)
+        assert np.all(np.diff(w[k]) >= 0.0)
+        assert np.max(np.abs(w[k] - ref)) <= 8 * n * 2.2e-16 * max(1e-300, np.max(np.abs(ref))), k
