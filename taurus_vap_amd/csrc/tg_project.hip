@@ -1115,7 +1115,7 @@ int project_run(tg_ctx* c) {
   // overlaps <Phi|R|Phi> for the gauge rotation (rot_over) and, when printing,
   // for parity x gauge (rot_pari, :279-284).  R_n = D0^T R D0 = ep*Pa + en*Pb.
   // Items are processed in segments of one overlap shape: the whole chunk when
-  // every state has the same nocc / nemp, else one segment per state.
+  // every state has the same nocc / nemp, else one per run of such states.
   auto overlap_segment = [&](const double* Pa, const double* Pb, long long a0, long long b0, int cnt,
                              const OvlShape& o, cplx* dst) -> int {
     const RunPlan& P = *PP;
@@ -1198,10 +1198,17 @@ int project_run(tg_ctx* c) {
   auto overlap = [&](const double* Pa, const double* Pb, long long a0, int na, cplx* dst) -> int {
     const RunPlan& P = *PP;
     if (P.uniform) return overlap_segment(Pa, Pb, a0, a0, na, P.sh[0], dst);
-    for (int st = (int)(a0 / A); st <= (int)((a0 + na - 1) / A); ++st) {
+    // runs of neighbouring states of one shape share a segment (most states have
+    // the basis's usual shape: one odd state in 24 made 24 Pfaffian launches of 81
+    // matrices, each a chain of its own, one after the other)
+    const int s1 = (int)((a0 + na - 1) / A);
+    for (int st = (int)(a0 / A); st <= s1;) {
+      int e = st + 1;
+      while (e <= s1 && P.sh[e].nocc == P.sh[st].nocc && P.sh[e].nemp == P.sh[st].nemp) ++e;
       const long long b0 = std::max<long long>((long long)st * A, a0);
-      const long long b1 = std::min<long long>((long long)(st + 1) * A, a0 + na);
+      const long long b1 = std::min<long long>((long long)e * A, a0 + na);
       TG_TRY(overlap_segment(Pa, Pb, a0, b0, (int)(b1 - b0), P.sh[st], dst));
+      st = e;
     }
     return TG_OK;
   };
