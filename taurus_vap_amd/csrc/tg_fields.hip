@@ -11,12 +11,31 @@
 //   pp channel  Delta_xy = sum_{u>v} P[(x,y),(u,v)] kappa_uv  (x>y),
 //               blocks labelled by (2m_x+2m_y, 2t_x+2t_y, l_x+l_y mod 2).
 // W and P are filled by adding exactly the reference's 8 + 4 updates, so every
-// element keeps its value (FP32 when the TBMEs are FP32: no rounding added) and
-// the angles of a batch become the M dimension of one GEMM per block: the
-// scattered, atomic-prone loop turns into dense FP64 arithmetic with each
-// matrix element read once per batch.
+// element keeps its value, and the angles of a batch become the M dimension of one
+// GEMM per block: the scattered, atomic-prone loop turns into dense FP64 arithmetic.
+//
+// The blocks are reduced further by the symmetries the interaction has, each a signed
+// permutation of a block's elements:
+//   ph: time reversal with hermiticity, (a,c) -> (c~,a~);  pp: time reversal,
+//       (x,y) -> (x~,y~); the signs follow from the elements;
+//   charge reflection, proton <-> neutron of every state (+1 in ph; a stored pp pair
+//       changes its order, -1), and the product of the two.
+// One that maps a block to itself and leaves its matrix the same BIT BY BIT (checked at
+// tg_init on the values as stored, so no element is changed; a charge-dependent
+// interaction, or one whose elements carry different rounding, simply does not pass)
+// commutes with the block: the elements fall into orbits, and the sums
+// a_chi(O) = sum_p c_chi(p) x_p over an orbit, c = +-1, mix only within a character
+// chi.  A block of s elements becomes 2 (or 4) of about s/2 (s/4): half (a quarter) of
+// the multiply-adds.  Their elements are sums of 2 (4) stored ones, scaled by the power
+// of two |O|, and are kept in FP64; they take the bytes of the FP32 block.  A block with
+// no symmetry keeps its elements as stored (FP32 when the TBMEs are FP32).
+// At 336 states, FP32 TBMEs, 225 angles: ph 1.71e11 -> 5.7e10 flop, pp 8.5e10 ->
+// 5.7e10; the products alone 3.39 -> 1.04 ms and 1.83 -> 0.95 ms, a projection 21.5 ->
+// 18.7 ms.  One set of densities (two products bound by reading W, 0.7 GB) 1.47 -> 0.2 ms.
 #include <algorithm>
+#include <atomic>
 #include <map>
+#include <thread>
 #include <tuple>
 
 #include "tg_internal.h"
@@ -25,86 +44,207 @@ namespace {
 
 constexpr int NT = 256;
 
-// Tiled transposes between the angle-major matrices (angle a at src + a*nn,
-// element (x, y) at linear index x + y*n) and the position-major contraction
-// layouts (X[row0 + a + p*ld], position p of a channel).  A workgroup moves a
-// tile of TL linear indices x TA angles through LDS: the matrix side is read or
-// written as TA runs of TL consecutive elements, the contraction side as TL runs
-// of TA consecutive angles, so both sides are coalesced.  inv maps linear
-// indices to positions (Channel::inv).
-constexpr int TL = 64;   // linear indices per tile
-constexpr int TA = 32;   // angles per tile
+// Orbits of a channel: up to four elements (linear indices in an n x n matrix) and as
+// many sums (positions in the contraction layout X[position * ld + angle]).  Bit
+// 4 j + i of the mask is set where element i enters sum j with a minus.
+// Consecutive orbits are 8 x 8 patches of a block, so the accesses on the matrix side,
+// along columns for one image and along rows for its transposed one, use whole lines
+// within a wave.  Bound by HBM.
 
-// X[row0 + a + inv[lin]*ld] = src_a[lin] for every lin with inv[lin] >= 0
-__global__ void __launch_bounds__(NT)
-gather_tiled_kernel(int na, long long nn, const int* __restrict__ inv,
-                    const cplx* __restrict__ src, int ld, int row0, cplx* __restrict__ X) {
-  __shared__ cplx tile[TL][TA + 1];
-  const long long lin0 = (long long)blockIdx.x * TL;
-  const int a0 = blockIdx.y * TA;
-  const int t = threadIdx.x;
-  {
-    const int l = t % TL;
-    const long long lin = lin0 + l;
-    for (int r = t / TL; r < TA; r += NT / TL) {
-      const int a = a0 + r;
-      if (a < na && lin < nn) tile[l][r] = src[(long long)a * nn + lin];
-    }
+__device__ __forceinline__ double flip(double v, unsigned m, int b) {   // -v where bit b of m
+  return __longlong_as_double(__double_as_longlong(v) ^ ((long long)((m >> b) & 1u) << 63));
+}
+
+// sum j of the orbit from its elements / element i from its sums
+__device__ __forceinline__ cplx orbit_sum(const cplx (&x)[4], unsigned mask, int j) {
+  cplx v = cmk(0.0, 0.0);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    v.x += flip(x[i].x, mask, 4 * j + i);
+    v.y += flip(x[i].y, mask, 4 * j + i);
   }
-  __syncthreads();
-  const int r = t % TA;
-  for (int l = t / TA; l < TL; l += NT / TA) {
-    const long long lin = lin0 + l;
-    const int a = a0 + r;
-    if (lin < nn && a < na) {
-      const int q = inv[lin];
-      if (q >= 0) X[row0 + a + (long long)q * ld] = tile[l][r];
-    }
+  return v;
+}
+__device__ __forceinline__ cplx orbit_element(const cplx (&y)[4], unsigned mask, int i) {
+  cplx v = cmk(0.0, 0.0);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    v.x += flip(y[j].x, mask, 4 * j + i);
+    v.y += flip(y[j].y, mask, 4 * j + i);
+  }
+  return v;
+}
+
+// What a scattered element becomes: the matrix itself; with SKEW minus it at the
+// transposed place as well; with HSP also h = it + H1
+template <bool SKEW, bool HSP>
+__device__ __forceinline__ void put_element(cplx v, int lin, int n, long long d, cplx* __restrict__ dst,
+                                            cplx h, cplx* __restrict__ hsp) {
+  dst[d + lin] = v;
+  if (SKEW) dst[d + lin / n + (long long)(lin % n) * n] = cmk(-v.x, -v.y);
+  if (HSP) hsp[d + lin] = cadd(v, h);
+}
+
+// Few angles (na <= TG_GROUPED_VEC): a thread takes every angle of one orbit
+__global__ void __launch_bounds__(NT)
+gather_few_kernel(int norb, int na, long long nn, const Orbit* __restrict__ orb,
+                  const cplx* __restrict__ src, int ld, int row0, cplx* __restrict__ X) {
+  const int o = blockIdx.x * NT + threadIdx.x;
+  if (o >= norb) return;
+  const Orbit e = orb[o];
+  for (int a = 0; a < na; ++a) {
+    cplx x[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = (i < e.m) ? src[a * nn + e.lin[i]] : cmk(0.0, 0.0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (j < e.m) X[(long long)e.pos[j] * ld + row0 + a] = orbit_sum(x, e.mask, j);
   }
 }
 
-// dst_a[lin] = field at lin from C[row0 + a + q*ld]:  q = inv[lin] >= 0: C;
-// pp (q <= -2): -C at position -2 - q; the diagonal (q == -1): 0.  With hsp:
-// hsp_a[lin] = dst_a[lin] + H1[lin].
+template <bool SKEW, bool HSP>
 __global__ void __launch_bounds__(NT)
-scatter_tiled_kernel(int na, long long nn, const int* __restrict__ inv,
-                     const cplx* __restrict__ C, int ld, int row0, cplx* __restrict__ dst,
-                     const cplx* __restrict__ H1, cplx* __restrict__ hsp) {
-  __shared__ cplx tile[TL][TA + 1];
-  const long long lin0 = (long long)blockIdx.x * TL;
-  const int a0 = blockIdx.y * TA;
-  const int t = threadIdx.x;
+scatter_few_kernel(int norb, int na, int n, const Orbit* __restrict__ orb, const cplx* __restrict__ C,
+                   int ld, int row0, cplx* __restrict__ dst, const cplx* __restrict__ H1,
+                   cplx* __restrict__ hsp) {
+  const int o = blockIdx.x * NT + threadIdx.x;
+  const long long nn = (long long)n * n;
+  if (SKEW && o < n)
+    for (int a = 0; a < na; ++a) dst[a * nn + o + (long long)o * n] = cmk(0.0, 0.0);
+  if (o >= norb) return;
+  const Orbit e = orb[o];
+  for (int a = 0; a < na; ++a) {
+    cplx y[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) y[j] = (j < e.m) ? C[(long long)e.pos[j] * ld + row0 + a] : cmk(0.0, 0.0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (i < e.m)
+        put_element<SKEW, HSP>(orbit_element(y, e.mask, i), e.lin[i], n, a * nn, dst,
+                               HSP ? H1[e.lin[i]] : cmk(0.0, 0.0), hsp);
+  }
+}
+
+// More angles: a workgroup moves TO orbits x TA angles, a lane an orbit on the matrix
+// side (a wave TA / 4 angles) and 16 lanes a row of angles on the other, through LDS.
+// MO: sums of an orbit at most (the LDS it takes).
+constexpr int TO = 64, TA = 16, TAP = TA + 1;
+
+template <int MO>
+__global__ void __launch_bounds__(NT)
+gather_tiled_kernel(int norb, int na, long long nn, const Orbit* __restrict__ orb,
+                    const cplx* __restrict__ src, int ld, int row0, cplx* __restrict__ X) {
+  __shared__ cplx T[MO * TO * TAP];
+  __shared__ int pos[MO * TO];
+  const int t = threadIdx.x, l = t % TO, w = t / TO;
+  const int o = blockIdx.x * TO + l, a0 = blockIdx.y * TA;
+  Orbit e{};
+  if (o < norb) e = orb[o];
+  cplx x[TA / 4][4];
+#pragma unroll
+  for (int u = 0; u < TA / 4; ++u) {
+    const cplx* p = src + (long long)min(a0 + w * (TA / 4) + u, na - 1) * nn;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[u][i] = (i < MO && i < e.m) ? p[e.lin[i]] : cmk(0.0, 0.0);
+  }
+  if (w == 0)
+#pragma unroll
+    for (int j = 0; j < MO; ++j) pos[j * TO + l] = (j < e.m) ? e.pos[j] : -1;
+#pragma unroll
+  for (int u = 0; u < TA / 4; ++u)
+#pragma unroll
+    for (int j = 0; j < MO; ++j) T[(j * TO + l) * TAP + w * (TA / 4) + u] = orbit_sum(x[u], e.mask, j);
+  __syncthreads();
+  const int a = t % TA;
+  if (a0 + a >= na) return;
+#pragma unroll 4
+  for (int r = t / TA; r < MO * TO; r += NT / TA) {
+    const int q = pos[r];
+    if (q >= 0) X[(long long)q * ld + row0 + a0 + a] = T[r * TAP + a];
+  }
+}
+
+template <int MO, bool SKEW, bool HSP>
+__global__ void __launch_bounds__(NT)
+scatter_tiled_kernel(int norb, int na, int n, const Orbit* __restrict__ orb, const cplx* __restrict__ C,
+                     int ld, int row0, cplx* __restrict__ dst, const cplx* __restrict__ H1,
+                     cplx* __restrict__ hsp) {
+  __shared__ cplx T[MO * TO * TAP];
+  __shared__ int pos[MO * TO];
+  const int t = threadIdx.x, l = t % TO, w = t / TO;
+  const int o = blockIdx.x * TO + l, a0 = blockIdx.y * TA;
+  const long long nn = (long long)n * n;
+  Orbit e{};
+  if (o < norb) e = orb[o];
+  if (w == 0)
+#pragma unroll
+    for (int j = 0; j < MO; ++j) pos[j * TO + l] = (j < e.m) ? e.pos[j] : -1;
+  __syncthreads();
   {
-    const int r = t % TA;
-    for (int l = t / TA; l < TL; l += NT / TA) {
-      const long long lin = lin0 + l;
-      const int a = a0 + r;
-      if (lin < nn && a < na) {
-        const int q = inv[lin];
-        cplx v = cmk(0.0, 0.0);
-        if (q >= 0) {
-          v = C[row0 + a + (long long)q * ld];
-        } else if (q <= -2) {
-          v = C[row0 + a + (long long)(-2 - q) * ld];
-          v = cmk(-v.x, -v.y);
-        }
-        tile[l][r] = v;
-      }
+    const int a = t % TA;
+#pragma unroll 4
+    for (int r = t / TA; r < MO * TO; r += NT / TA) {
+      const int q = pos[r];
+      T[r * TAP + a] = (q >= 0 && a0 + a < na) ? C[(long long)q * ld + row0 + a0 + a] : cmk(0.0, 0.0);
     }
   }
   __syncthreads();
-  const int l = t % TL;
-  const long long lin = lin0 + l;
-  if (lin >= nn) return;
-  const cplx h = hsp ? H1[lin] : cmk(0.0, 0.0);
-  for (int r = t / TL; r < TA; r += NT / TL) {
-    const int a = a0 + r;
-    if (a < na) {
-      const cplx v = tile[l][r];
-      dst[(long long)a * nn + lin] = v;
-      if (hsp) hsp[(long long)a * nn + lin] = cadd(v, h);
-    }
+#pragma unroll
+  for (int u = 0; u < TA / 4; ++u) {
+    const int a = a0 + w * (TA / 4) + u;
+    if (a >= na) break;
+    const long long d = (long long)a * nn;
+    if (SKEW && o < n) dst[d + o + (long long)o * n] = cmk(0.0, 0.0);
+    cplx y[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      y[j] = (j < MO) ? T[((j < MO ? j : 0) * TO + l) * TAP + w * (TA / 4) + u] : cmk(0.0, 0.0);
+#pragma unroll
+    for (int i = 0; i < MO; ++i)
+      if (i < e.m)
+        put_element<SKEW, HSP>(orbit_element(y, e.mask, i), e.lin[i], n, d, dst,
+                               HSP ? H1[e.lin[i]] : cmk(0.0, 0.0), hsp);
   }
+}
+
+// The gather of src (na matrices) into rows row0 .. row0 + na - 1 of X, and the scatter
+// of C back
+int gather(hipStream_t s, const Channel& ch, int n, int na, const cplx* src, int ld, int row0, cplx* X) {
+  const long long nn = (long long)n * n;
+  const Orbit* orb = ch.d_orb.as<Orbit>();
+  const dim3 grid((ch.norb + TO - 1) / TO, (na + TA - 1) / TA);
+  if (na <= TG_GROUPED_VEC)
+    hipLaunchKernelGGL(gather_few_kernel, dim3((ch.norb + NT - 1) / NT), dim3(NT), 0, s, ch.norb, na, nn,
+                       orb, src, ld, row0, X);
+#define TG_GATHER(MO)                                                                            \
+  hipLaunchKernelGGL(gather_tiled_kernel<MO>, grid, dim3(NT), 0, s, ch.norb, na, nn, orb, src, ld, \
+                     row0, X)
+  else if (ch.mo > 2) TG_GATHER(4);
+  else if (ch.mo > 1) TG_GATHER(2);
+  else TG_GATHER(1);
+#undef TG_GATHER
+  TG_HIP(hipGetLastError());
+  return TG_OK;
+}
+
+template <bool SKEW, bool HSP>
+int scatter(hipStream_t s, const Channel& ch, int n, int na, const cplx* C, int ld, int row0, cplx* dst,
+            const cplx* H1, cplx* hsp) {
+  const Orbit* orb = ch.d_orb.as<Orbit>();
+  const int cover = SKEW ? std::max(ch.norb, n) : ch.norb;   // the diagonal is set by thread index
+  const dim3 grid((cover + TO - 1) / TO, (na + TA - 1) / TA);
+  if (na <= TG_GROUPED_VEC)
+    hipLaunchKernelGGL((scatter_few_kernel<SKEW, HSP>), dim3((cover + NT - 1) / NT), dim3(NT), 0, s,
+                       ch.norb, na, n, orb, C, ld, row0, dst, H1, hsp);
+#define TG_SCATTER(MO)                                                                           \
+  hipLaunchKernelGGL((scatter_tiled_kernel<MO, SKEW, HSP>), grid, dim3(NT), 0, s, ch.norb, na, n,  \
+                     orb, C, ld, row0, dst, H1, hsp)
+  else if (ch.mo > 2) TG_SCATTER(4);
+  else if (ch.mo > 1) TG_SCATTER(2);
+  else TG_SCATTER(1);
+#undef TG_SCATTER
+  TG_HIP(hipGetLastError());
+  return TG_OK;
 }
 
 // hsp_a = Gamma_a + H1
@@ -136,42 +276,255 @@ struct KeyCmp {
   }
 };
 
-// Assigns each element (x,y) of a channel to its block and position.
-void plan_channel(Channel& ch, int n, const std::vector<int>& m, const std::vector<int>& t,
-                  const std::vector<int>& l, bool pp, std::vector<int>& pos_of) {
-  std::map<std::tuple<int, int, int>, std::vector<int>, KeyCmp> classes;
-  pos_of.assign((size_t)n * n, -1);
+typedef std::tuple<int, int, int> ClassKey;
+
+// Elements of a block channel by class, in patches of 8 x 8 (linear indices x + y n)
+std::map<ClassKey, std::vector<int>> channel_classes(const tg_ctx* c, bool pp) {
+  const int n = c->n;
+  const std::vector<int>&m = c->sp_2mj, &t = c->sp_2mt, &l = c->sp_l;
+  // runs of states with the same m, t and parity, and the place of a state in its run
+  std::vector<int> run(n, 0), in(n, 0);
+  for (int i = 1; i < n; ++i) {
+    const bool same = m[i] == m[i - 1] && t[i] == t[i - 1] && (l[i] & 1) == (l[i - 1] & 1);
+    run[i] = run[i - 1] + (same ? 0 : 1);
+    in[i] = same ? in[i - 1] + 1 : 0;
+  }
+  std::map<ClassKey, std::vector<int>> cls;
   for (int y = 0; y < n; ++y)
     for (int x = 0; x < n; ++x) {
       if (pp && x <= y) continue;
-      std::tuple<int, int, int> key = pp ? std::make_tuple(m[x] + m[y], t[x] + t[y], (l[x] + l[y]) & 1)
-                                         : std::make_tuple(m[x] - m[y], t[x] - t[y], (l[x] + l[y]) & 1);
-      classes[key].push_back(x + y * n);
+      cls[pp ? ClassKey(m[x] + m[y], t[x] + t[y], (l[x] + l[y]) & 1)
+             : ClassKey(m[x] - m[y], t[x] - t[y], (l[x] + l[y]) & 1)]
+          .push_back(x + y * n);
     }
-  ch.groups.clear();
-  ch.perm.clear();
-  long long woff = 0;
-  int off = 0;
-  for (auto& kv : classes) {
-    GroupDesc g;
-    g.off = off;
-    g.size = (int)kv.second.size();
-    g.woff = woff;
-    ch.groups.push_back(g);
-    for (size_t k = 0; k < kv.second.size(); ++k) {
-      pos_of[kv.second[k]] = off + (int)k;
-      ch.perm.push_back(kv.second[k]);
+  for (auto& kv : cls)
+    std::sort(kv.second.begin(), kv.second.end(), [&](int p, int q) {
+      auto key = [&](int e) {
+        const int x = e % n, y = e / n;
+        return std::make_tuple(run[x], run[y], in[y] / 8, in[x] / 8, in[y], in[x]);
+      };
+      return key(p) < key(q);
+    });
+  return cls;
+}
+
+// A signed permutation of a class: element k -> to[k] with sign sg[k]
+struct Sym {
+  std::vector<int> to, sg;
+};
+
+// Whether B(to p, to q) = sg_p sg_q B(p, q) for all p, q, bit by bit (B symmetric in
+// meaning, stored at B[q + p s]).  With `find` the signs are found first: +-1 spread
+// over the elements that B connects, an element and its images (imgs) alike.
+bool sym_holds(const std::vector<double>& B, int s, Sym& g, bool find,
+               const std::vector<const std::vector<int>*>& imgs) {
+  if (find) {
+    g.sg.assign(s, 0);
+    std::vector<int> todo;
+    auto visit = [&](int k, int sg) {
+      std::vector<int> st(1, k);
+      while (!st.empty()) {
+        const int e = st.back();
+        st.pop_back();
+        if (g.sg[e] != 0) continue;
+        g.sg[e] = sg;
+        todo.push_back(e);
+        for (const std::vector<int>* im : imgs) st.push_back((*im)[e]);
+      }
+    };
+    for (int r = 0; r < s; ++r) {
+      if (g.sg[r] != 0) continue;
+      visit(r, 1);
+      while (!todo.empty()) {
+        const int p = todo.back();
+        todo.pop_back();
+        const double* bp = B.data() + (size_t)p * s;
+        const double* bt = B.data() + (size_t)g.to[p] * s;
+        for (int q = 0; q < s; ++q)
+          if (g.sg[q] == 0 && bp[q] != 0.0) visit(q, (bp[q] == bt[g.to[q]]) ? g.sg[p] : -g.sg[p]);
+      }
     }
-    off += g.size;
-    woff += (long long)g.size * g.size;
   }
-  ch.npos = off;
-  ch.ngroups = (int)ch.groups.size();
-  ch.wsize = woff;
-  ch.inv = pos_of;
-  if (pp)
-    for (int y = 0; y < n; ++y)
-      for (int x = 0; x < y; ++x) ch.inv[x + (size_t)y * n] = -2 - pos_of[y + (size_t)x * n];
+  for (int p = 0; p < s; ++p) {
+    const double* bp = B.data() + (size_t)p * s;
+    const double* bt = B.data() + (size_t)g.to[p] * s;
+    const double sp = g.sg[p];
+    for (int q = 0; q < s; ++q)
+      if (!(bt[g.to[q]] == sp * g.sg[q] * bp[q])) return false;
+  }
+  return true;
+}
+
+// One class of a channel reduced by its symmetries: its orbits (positions relative to
+// the class) and the character blocks W (matrix [in * size + out], one after another).
+struct Reduced {
+  std::vector<Orbit> orb;
+  std::vector<int> size;
+  std::vector<double> W;
+  bool split = false;
+};
+
+Reduced reduce_class(const tg_ctx* c, bool pp, const std::vector<int>& el, const std::vector<double>& B) {
+  const int n = c->n, h = n / 2, s = (int)el.size();
+  std::vector<int> at((size_t)n * n, -1);
+  for (int k = 0; k < s; ++k) at[el[k]] = k;
+  // the proton and the neutron half hold the same states, in the same order
+  bool halves = true;
+  for (int i = 0; i < h && halves; ++i)
+    halves = c->sp_2mj[i] == c->sp_2mj[i + h] && c->sp_l[i] == c->sp_l[i + h] &&
+             c->sp_tr[i] < h && c->sp_tr[i + h] == c->sp_tr[i] + h;
+  bool tr_ok = true;
+  for (int i = 0; i < n && tr_ok; ++i) tr_ok = c->sp_tr[c->sp_tr[i]] == i && c->sp_tr[i] != i;
+  // image of element (x, y): time reversal (and transposition in ph), reflection; the
+  // sign where a pp pair changes its order
+  auto image = [&](int e, bool tr, bool ch, int& sg) {
+    int x = e % n, y = e / n;
+    sg = 1;
+    if (tr) {
+      const int tx = c->sp_tr[x], ty = c->sp_tr[y];
+      x = pp ? tx : ty;
+      y = pp ? ty : tx;
+    }
+    if (ch) {
+      x = (x + h) % n;
+      y = (y + h) % n;
+    }
+    if (pp && x < y) {
+      std::swap(x, y);
+      sg = -1;
+    }
+    return x + y * n;
+  };
+  Sym g[3];               // time reversal, reflection, their product
+  bool ok[3];
+  for (int q = 0; q < 3; ++q) {
+    const bool tr = q != 1, ch = q != 0;
+    ok[q] = (!tr || tr_ok) && (!ch || halves) && s > 1;
+    g[q].to.assign(s, 0);
+    g[q].sg.assign(s, 1);
+    for (int k = 0; k < s && ok[q]; ++k) {
+      g[q].to[k] = at[image(el[k], tr, ch, g[q].sg[k])];
+      ok[q] = g[q].to[k] >= 0;
+    }
+    for (int k = 0; k < s && ok[q]; ++k) ok[q] = g[q].to[g[q].to[k]] == k;
+  }
+  std::vector<const std::vector<int>*> imgs;
+  for (int q = 0; q < 3; ++q)
+    if (ok[q]) imgs.push_back(&g[q].to);
+  // the reflection's signs are known; those with time reversal are found
+  if (ok[1]) ok[1] = sym_holds(B, s, g[1], false, imgs);
+  if (ok[0]) ok[0] = sym_holds(B, s, g[0], true, imgs);
+  if (ok[2] && !(ok[0] && ok[1])) ok[2] = sym_holds(B, s, g[2], true, imgs);
+  // signs of an involution agree on an element and its image
+  for (int q = 0; q < 3; ++q)
+    for (int k = 0; k < s && ok[q]; ++k) ok[q] = g[q].sg[k] == g[q].sg[g[q].to[k]];
+  std::vector<const Sym*> gen;
+  if (ok[0] && ok[1]) {
+    bool commute = true;
+    for (int k = 0; k < s && commute; ++k)
+      commute = g[0].to[g[1].to[k]] == g[1].to[g[0].to[k]] &&
+                g[0].sg[g[1].to[k]] * g[1].sg[k] == g[1].sg[g[0].to[k]] * g[0].sg[k];
+    gen.push_back(&g[0]);
+    if (commute) gen.push_back(&g[1]);
+  } else {
+    for (int q = 0; q < 3; ++q)
+      if (ok[q]) {
+        gen.push_back(&g[q]);
+        break;
+      }
+  }
+  Reduced R;
+  R.split = !gen.empty();
+  const int ng = (int)gen.size(), order = 1 << ng;
+  // orbits: element e_b = (product of the generators in b) of the first one, its sign
+  std::vector<char> seen(s, 0);
+  R.size.assign(order, 0);
+  std::vector<std::vector<int>> members;          // elements of each orbit (class index)
+  std::vector<unsigned> masks;                    // bit 4 j + i: minus of element i in sum j
+  std::vector<std::vector<int>> chars;            // character of each of the orbit's sums
+  for (int k = 0; k < s; ++k) {
+    if (seen[k]) continue;
+    int im[4], sg[4];
+    for (int b = 0; b < order; ++b) {
+      int e = k, sgn = 1;
+      for (int q = 0; q < ng; ++q)
+        if (b >> q & 1) {
+          sgn *= gen[q]->sg[e];
+          e = gen[q]->to[e];
+        }
+      im[b] = e;
+      sg[b] = sgn;
+    }
+    std::vector<int> mem, first;
+    for (int b = 0; b < order; ++b)
+      if (std::find(mem.begin(), mem.end(), im[b]) == mem.end()) {
+        mem.push_back(im[b]);
+        first.push_back(b);
+        seen[im[b]] = 1;
+      }
+    std::vector<int> ch;
+    unsigned mask = 0;
+    for (int x = 0; x < order; ++x) {
+      // character x: sign (-1)^(bits of b & x) of the group element b
+      auto cs = [&](int b) { return (__builtin_popcount(b & x) & 1 ? -1 : 1) * sg[b]; };
+      bool fits = true;
+      for (int b = 0; b < order && fits; ++b)
+        for (int b2 = 0; b2 < b && fits; ++b2)
+          if (im[b] == im[b2]) fits = cs(b) == cs(b2);
+      if (!fits) continue;
+      const int j = (int)ch.size();
+      for (size_t i = 0; i < mem.size(); ++i)
+        if (cs(first[i]) < 0) mask |= 1u << (4 * j + (int)i);
+      ch.push_back(x);
+    }
+    members.push_back(mem);
+    masks.push_back(mask);
+    chars.push_back(ch);
+    for (int x : ch) ++R.size[x];
+  }
+  // positions: character blocks one after another, orbits in order inside each
+  std::vector<int> base(order, 0), fill(order, 0);
+  std::vector<size_t> wbase(order, 0);
+  size_t wsz = 0;
+  for (int x = 0, o = 0; x < order; ++x) {
+    base[x] = o;
+    o += R.size[x];
+    wbase[x] = wsz;
+    wsz += (size_t)R.size[x] * R.size[x];
+  }
+  R.W.assign(wsz, 0.0);
+  const size_t no = members.size();
+  std::vector<std::vector<int>> idx(no);          // index of each of its sums in its block
+  for (size_t o = 0; o < no; ++o) {
+    Orbit ob{};
+    ob.m = (int)members[o].size();
+    ob.mask = masks[o];
+    for (int i = 0; i < ob.m; ++i) {
+      ob.lin[i] = el[members[o][i]];
+      const int x = chars[o][i];
+      idx[o].push_back(fill[x]);
+      ob.pos[i] = base[x] + fill[x]++;
+    }
+    R.orb.push_back(ob);
+  }
+  for (size_t out = 0; out < no; ++out) {
+    const double* row = B.data() + (size_t)members[out][0] * s;
+    for (size_t jo = 0; jo < chars[out].size(); ++jo) {
+      const int x = chars[out][jo];
+      double* w = R.W.data() + wbase[x] + idx[out][jo];
+      for (size_t o = 0; o < no; ++o)
+        for (size_t j = 0; j < chars[o].size(); ++j)
+          if (chars[o][j] == x) {
+            double v = 0.0;
+            for (size_t i = 0; i < members[o].size(); ++i) {
+              const double b = row[members[o][i]];
+              v += (masks[o] >> (4 * j + i) & 1u) ? -b : b;
+            }
+            w[(size_t)idx[o][j] * R.size[x]] = v / (double)members[o].size();
+          }
+    }
+  }
+  return R;
 }
 
 }  // namespace
@@ -179,38 +532,39 @@ void plan_channel(Channel& ch, int n, const std::vector<int>& m, const std::vect
 int contraction_build(tg_ctx* c, int64_t ntb, const int16_t* abcd, const void* H2, int h2_bytes,
                       const int8_t* trperm) {
   const int n = c->n;
-  std::vector<int> pos_ph, pos_pp;
-  plan_channel(c->ph, n, c->sp_2mj, c->sp_2mt, c->sp_l, false, pos_ph);
-  plan_channel(c->pp, n, c->sp_2mj, c->sp_2mt, c->sp_l, true, pos_pp);
-  std::vector<double> Wph((size_t)c->ph.wsize, 0.0), Wpp((size_t)c->pp.wsize, 0.0);
-
-  // group index of each position
-  std::vector<int> gph(c->ph.npos), gpp(c->pp.npos);
-  for (int g = 0; g < c->ph.ngroups; ++g)
-    for (int k = 0; k < c->ph.groups[g].size; ++k) gph[c->ph.groups[g].off + k] = g;
-  for (int g = 0; g < c->pp.ngroups; ++g)
-    for (int k = 0; k < c->pp.groups[g].size; ++k) gpp[c->pp.groups[g].off + k] = g;
+  // per channel: the classes, the class and place of every element, the full matrices
+  struct Full {
+    std::vector<std::vector<int>> el;
+    std::vector<int> cls, at;
+    std::vector<std::vector<double>> B;
+  } F[2];
+  for (int q = 0; q < 2; ++q) {
+    F[q].cls.assign((size_t)n * n, -1);
+    F[q].at.assign((size_t)n * n, -1);
+    for (auto& kv : channel_classes(c, q == 1)) {
+      for (size_t k = 0; k < kv.second.size(); ++k) {
+        F[q].cls[kv.second[k]] = (int)F[q].el.size();
+        F[q].at[kv.second[k]] = (int)k;
+      }
+      F[q].B.emplace_back(kv.second.size() * kv.second.size(), 0.0);
+      F[q].el.push_back(std::move(kv.second));
+    }
+  }
 
   bool bad = false;
-  // W(q,p) of the group holding both positions, stored at woff + q + p*s
-  auto add_ph = [&](int a, int cc, int d, int b, double v) {
-    int po = pos_ph[a + cc * n], pi = pos_ph[d + b * n];
-    int g = gph[po];
-    if (gph[pi] != g) { bad = true; return; }
-    const GroupDesc& G = c->ph.groups[g];
-    Wph[(size_t)(G.woff + (long long)(pi - G.off) + (long long)(po - G.off) * G.size)] += v;
+  // B(q, p) of the class holding both elements, stored at q + p * s (p the field's)
+  auto add = [&](Full& f, int out, int in, double v) {
+    const int g = f.cls[out];
+    if (g < 0 || f.cls[in] != g) { bad = true; return; }
+    f.B[g][(size_t)f.at[in] + (size_t)f.at[out] * f.el[g].size()] += v;
   };
+  auto add_ph = [&](int a, int cc, int d, int b, double v) { add(F[0], a + cc * n, d + b * n, v); };
   auto add_pp = [&](int x, int y, int u, int w, double v) {
     // stored pairs have x > y and u > w; Delta and kappa are skew, so a pair
     // in the other order enters with the opposite sign
     if (x < y) { std::swap(x, y); v = -v; }
     if (u < w) { std::swap(u, w); v = -v; }
-    int po = pos_pp[x + y * n], pi = pos_pp[u + w * n];
-    if (po < 0 || pi < 0) { bad = true; return; }
-    int g = gpp[po];
-    if (gpp[pi] != g) { bad = true; return; }
-    const GroupDesc& G = c->pp.groups[g];
-    Wpp[(size_t)(G.woff + (long long)(pi - G.off) + (long long)(po - G.off) * G.size)] += v;
+    add(F[1], x + y * n, u + w * n, v);
   };
 
   const std::vector<int>& tr = c->sp_tr;
@@ -265,36 +619,89 @@ int contraction_build(tg_ctx* c, int64_t ntb, const int16_t* abcd, const void* H
     return TG_E_ARG;
   }
 
-  // upload
-  for (Channel* ch : {&c->ph, &c->pp}) {
-    std::vector<double>& W = (ch == &c->ph) ? Wph : Wpp;
-    TG_TRY(ch->d_inv.ensure(sizeof(int) * ch->inv.size()));
-    TG_HIP(hipMemcpy(ch->d_inv.p, ch->inv.data(), sizeof(int) * ch->inv.size(),
-                     hipMemcpyHostToDevice));
-    TG_TRY(ch->d_groups.ensure(sizeof(GroupDesc) * ch->groups.size()));
-    TG_HIP(hipMemcpy(ch->d_groups.p, ch->groups.data(), sizeof(GroupDesc) * ch->groups.size(),
-                     hipMemcpyHostToDevice));
-    if (c->w_fp32) {
-      std::vector<float> Wf(W.size());
-      for (size_t i = 0; i < W.size(); ++i) Wf[i] = (float)W[i];
-      TG_TRY(ch->d_W.ensure(sizeof(float) * Wf.size()));
-      TG_HIP(hipMemcpy(ch->d_W.p, Wf.data(), sizeof(float) * Wf.size(), hipMemcpyHostToDevice));
-    } else {
-      TG_TRY(ch->d_W.ensure(sizeof(double) * W.size()));
-      TG_HIP(hipMemcpy(ch->d_W.p, W.data(), sizeof(double) * W.size(), hipMemcpyHostToDevice));
-    }
-    // tile table: (group, n0) for every 64-column tile of every group
-    std::vector<int> tg, tn;
-    for (int g = 0; g < ch->ngroups; ++g)
-      for (int n0 = 0; n0 < ch->groups[g].size; n0 += 64) {
-        tg.push_back(g);
-        tn.push_back(n0);
+  // the values as stored, the reduction of every class, the upload
+  for (int q = 0; q < 2; ++q) {
+    Channel& ch = q == 0 ? c->ph : c->pp;
+    Full& f = F[q];
+    const int nc = (int)f.el.size();
+    std::vector<Reduced> red(nc);
+    std::atomic<int> next(0);
+    auto work = [&] {
+      for (int g; (g = next.fetch_add(1)) < nc;) {
+        if (c->w_fp32)
+          for (double& v : f.B[g]) v = (double)(float)v;
+        red[g] = reduce_class(c, q == 1, f.el[g], f.B[g]);
+        std::vector<double>().swap(f.B[g]);
       }
-    ch->ntiles_total = (int)tg.size();
-    TG_TRY(ch->d_tile_group.ensure(sizeof(int) * tg.size()));
-    TG_TRY(ch->d_tile_n0.ensure(sizeof(int) * tn.size()));
-    TG_HIP(hipMemcpy(ch->d_tile_group.p, tg.data(), sizeof(int) * tg.size(), hipMemcpyHostToDevice));
-    TG_HIP(hipMemcpy(ch->d_tile_n0.p, tn.data(), sizeof(int) * tn.size(), hipMemcpyHostToDevice));
+    };
+    const int nt = std::max(1, std::min({8, (int)std::thread::hardware_concurrency(), nc}));
+    std::vector<std::thread> pool;
+    for (int k = 1; k < nt; ++k) pool.emplace_back(work);
+    work();
+    for (std::thread& th : pool) th.join();
+
+    std::vector<GroupDesc> groups;
+    std::vector<Orbit> orb;
+    std::vector<char> W;
+    int off = 0;
+    for (int g = 0; g < nc; ++g) {
+      for (Orbit& o : red[g].orb) {
+        for (int i = 0; i < o.m; ++i) o.pos[i] += off;
+        orb.push_back(o);
+      }
+      const bool f32 = c->w_fp32 && !red[g].split;
+      size_t w0 = 0;
+      for (int sz : red[g].size) {
+        if (sz == 0) continue;
+        const size_t cnt = (size_t)sz * sz;
+        const size_t at = (W.size() + 15) / 16 * 16;
+        W.resize(at + cnt * (f32 ? sizeof(float) : sizeof(double)));
+        for (size_t k = 0; k < cnt; ++k)
+          if (f32) reinterpret_cast<float*>(W.data() + at)[k] = (float)red[g].W[w0 + k];
+          else reinterpret_cast<double*>(W.data() + at)[k] = red[g].W[w0 + k];
+        groups.push_back({off, sz, (long long)at, f32 ? 1 : 0});
+        off += sz;
+        w0 += cnt;
+      }
+      red[g] = Reduced();
+    }
+    ch.npos = off;
+    ch.ngroups = (int)groups.size();
+    ch.norb = (int)orb.size();
+    ch.mo = 1;
+    for (const Orbit& o : orb) ch.mo = std::max(ch.mo, o.m);
+    // (group, first position) of every 64-position tile, entry t for XCD t % 8: each
+    // group, the long ones first, to the XCD with the least work so far
+    std::vector<int> order(groups.size());
+    for (size_t k = 0; k < order.size(); ++k) order[k] = (int)k;
+    std::stable_sort(order.begin(), order.end(),
+                     [&](int x, int y) { return groups[x].size > groups[y].size; });
+    std::vector<std::pair<int, int>> list[8];
+    double load[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    size_t len = 0;
+    for (int g : order) {
+      const int x = (int)(std::min_element(load, load + 8) - load);
+      for (int j0 = 0; j0 < groups[g].size; j0 += 64) list[x].push_back({g, j0});
+      load[x] += (double)groups[g].size * ((groups[g].size + 31) / 32 * 32);
+      len = std::max(len, list[x].size());
+    }
+    std::vector<int> tg(8 * len, -1), tn(8 * len, 0);
+    for (int x = 0; x < 8; ++x)
+      for (size_t k = 0; k < list[x].size(); ++k) {
+        tg[8 * k + x] = list[x][k].first;
+        tn[8 * k + x] = list[x][k].second;
+      }
+    ch.ntiles_total = (int)tg.size();
+    auto up = [](DevBuf& d, const void* src, size_t bytes) -> int {
+      TG_TRY(d.ensure(std::max<size_t>(bytes, 16)));
+      TG_HIP(hipMemcpy(d.p, src, bytes, hipMemcpyHostToDevice));
+      return TG_OK;
+    };
+    TG_TRY(up(ch.d_orb, orb.data(), sizeof(Orbit) * orb.size()));
+    TG_TRY(up(ch.d_groups, groups.data(), sizeof(GroupDesc) * groups.size()));
+    TG_TRY(up(ch.d_W, W.data(), W.size()));
+    TG_TRY(up(ch.d_tile_group, tg.data(), sizeof(int) * tg.size()));
+    TG_TRY(up(ch.d_tile_n0, tn.data(), sizeof(int) * tn.size()));
   }
   return TG_OK;
 }
@@ -305,70 +712,59 @@ int contraction_run(tg_ctx* c, int na, const cplx* rho, const cplx* kLR, const c
   const int n = c->n;
   const long long nn = (long long)n * n;
   hipStream_t s = c->stream;
-  const int nph = c->ph.npos, npp = c->pp.npos;
   const int two = (kRL != nullptr && !hermitian) ? 2 : 1;   // pp right-hand sides per angle
-  // layout: Xph (na x nph), Cph, Xpp (two*na x npp), Cpp
-  size_t need = sizeof(cplx) * ((size_t)2 * na * nph + (size_t)2 * two * na * npp);
-  TG_TRY(c->d_blk.ensure(need));
+  // rows of angles per position: ph the na angles; pp those of kLR, then (from row r2,
+  // at a whole 128-byte line above the vector kernels' sizes) those of kRL
+  const int ldph = grouped_ld(na);
+  const int r2 = (two == 1) ? 0 : (2 * na <= TG_GROUPED_VEC ? na : (na + 7) / 8 * 8);
+  const int Mpp = r2 + na, ldpp = grouped_ld(Mpp);
+  const size_t nph = (size_t)ldph * c->ph.npos, npp = (size_t)ldpp * c->pp.npos;
+  TG_TRY(c->d_blk.ensure(sizeof(cplx) * 2 * (nph + npp)));
   cplx* Xph = c->d_blk.as<cplx>();
-  cplx* Cph = Xph + (size_t)na * nph;
-  cplx* Xpp = Cph + (size_t)na * nph;
-  cplx* Cpp = Xpp + (size_t)two * na * npp;
+  cplx* Cph = Xph + nph;
+  cplx* Xpp = Cph + nph;
+  cplx* Cpp = Xpp + npp;
 
-  const int* iph = c->ph.d_inv.as<int>();
-  const int* ipp = c->pp.d_inv.as<int>();
-  const dim3 tiles((unsigned)((nn + TL - 1) / TL), (unsigned)((na + TA - 1) / TA));
   // the pp channel (gathers, product, scatters) on the third stream beside the ph
   // one: the groups are of very uneven size, so each product's tail leaves CUs the
   // other can use, and the gathers and scatters (HBM-bound) overlap products
   hipStream_t s3 = c->stream3;
   TG_HIP(hipEventRecord(c->ev_fork3, s));
   TG_HIP(hipStreamWaitEvent(s3, c->ev_fork3, 0));
-  hipLaunchKernelGGL(gather_tiled_kernel, tiles, dim3(NT), 0, s, na, nn, iph, rho, na, 0, Xph);
-  hipLaunchKernelGGL(gather_tiled_kernel, tiles, dim3(NT), 0, s3, na, nn, ipp, kLR, two * na, 0,
-                     Xpp);
-  if (two == 2)
-    hipLaunchKernelGGL(gather_tiled_kernel, tiles, dim3(NT), 0, s3, na, nn, ipp, kRL, two * na, na,
-                       Xpp);
-  TG_HIP(hipGetLastError());
-  if (!gemm_grouped_tuned(na, c->ph.ntiles_total, 0) ||
-      !gemm_grouped_tuned(two * na, c->pp.ntiles_total, 1)) {
+  TG_TRY(gather(s, c->ph, n, na, rho, ldph, 0, Xph));
+  TG_TRY(gather(s3, c->pp, n, na, kLR, ldpp, 0, Xpp));
+  if (two == 2) TG_TRY(gather(s3, c->pp, n, na, kRL, ldpp, r2, Xpp));
+  auto product = [&](hipStream_t st, const Channel& ch, int M, const cplx* X, cplx* C, int ld, int tag,
+                     bool tune) -> int {
+    const GroupDesc* g = ch.d_groups.as<GroupDesc>();
+    const int *tg = ch.d_tile_group.as<int>(), *tj = ch.d_tile_n0.as<int>();
+    if (tune) return gemm_tune_grouped(st, M, X, C, ld, ch.d_W.p, g, tg, tj, ch.ntiles_total, tag);
+    return gemm_grouped(st, M, X, C, ld, ch.d_W.p, g, tg, tj, tag, ch.ntiles_total);
+  };
+  if (!gemm_grouped_tuned(na, c->ph.ntiles_total, 0) || !gemm_grouped_tuned(Mpp, c->pp.ntiles_total, 1)) {
     // first call for this batch size: both channels' tile shapes are timed on the
     // context stream alone (outputs recomputed below)
     TG_HIP(hipEventRecord(c->ev_join3, s3));
     TG_HIP(hipStreamWaitEvent(s, c->ev_join3, 0));
-    TG_TRY(gemm_tune_grouped(s, na, Xph, Cph, c->ph.d_W.p, c->w_fp32,
-                             c->ph.d_groups.as<GroupDesc>(), c->ph.d_tile_group.as<int>(),
-                             c->ph.d_tile_n0.as<int>(), c->ph.ntiles_total, 0));
-    TG_TRY(gemm_tune_grouped(s, two * na, Xpp, Cpp, c->pp.d_W.p, c->w_fp32,
-                             c->pp.d_groups.as<GroupDesc>(), c->pp.d_tile_group.as<int>(),
-                             c->pp.d_tile_n0.as<int>(), c->pp.ntiles_total, 1));
+    TG_TRY(product(s, c->ph, na, Xph, Cph, ldph, 0, true));
+    TG_TRY(product(s, c->pp, Mpp, Xpp, Cpp, ldpp, 1, true));
     TG_HIP(hipEventRecord(c->ev_fork3, s));
     TG_HIP(hipStreamWaitEvent(s3, c->ev_fork3, 0));
   }
   {
     ScopedTiming tk(c, "kernel:grouped_pp", s3);
-    TG_TRY(gemm_grouped(s3, two * na, Xpp, Cpp, c->pp.d_W.p, c->w_fp32,
-                        c->pp.d_groups.as<GroupDesc>(), c->pp.d_tile_group.as<int>(),
-                        c->pp.d_tile_n0.as<int>(), 1, c->pp.ntiles_total));
+    TG_TRY(product(s3, c->pp, Mpp, Xpp, Cpp, ldpp, 1, false));
   }
-  hipLaunchKernelGGL(scatter_tiled_kernel, tiles, dim3(NT), 0, s3, na, nn, ipp, Cpp, two * na, 0,
-                     dLR, (const cplx*)nullptr, (cplx*)nullptr);
-  if (two == 2)
-    hipLaunchKernelGGL(scatter_tiled_kernel, tiles, dim3(NT), 0, s3, na, nn, ipp, Cpp, two * na, na,
-                       dRL, (const cplx*)nullptr, (cplx*)nullptr);
-  TG_HIP(hipGetLastError());
+  TG_TRY((scatter<true, false>(s3, c->pp, n, na, Cpp, ldpp, 0, dLR, nullptr, nullptr)));
+  if (two == 2) TG_TRY((scatter<true, false>(s3, c->pp, n, na, Cpp, ldpp, r2, dRL, nullptr, nullptr)));
   {
     ScopedTiming tk(c, "kernel:grouped_ph");
-    TG_TRY(gemm_grouped(s, na, Xph, Cph, c->ph.d_W.p, c->w_fp32, c->ph.d_groups.as<GroupDesc>(),
-                        c->ph.d_tile_group.as<int>(), c->ph.d_tile_n0.as<int>(), 0,
-                        c->ph.ntiles_total));
+    TG_TRY(product(s, c->ph, na, Xph, Cph, ldph, 0, false));
   }
   // Gamma (and h = Gamma + H1 when no hermitian completion follows), DeltaLR, DeltaRL
   const bool fuse_h = hsp != nullptr && !hermitian;
-  hipLaunchKernelGGL(scatter_tiled_kernel, tiles, dim3(NT), 0, s, na, nn, iph, Cph, na, 0, gamma,
-                     fuse_h ? H1 : nullptr, fuse_h ? hsp : nullptr);
-  TG_HIP(hipGetLastError());
+  if (fuse_h) TG_TRY((scatter<false, true>(s, c->ph, n, na, Cph, ldph, 0, gamma, H1, hsp)));
+  else TG_TRY((scatter<false, false>(s, c->ph, n, na, Cph, ldph, 0, gamma, nullptr, nullptr)));
   if (defer_join && two == 2 && fuse_h) return TG_OK;
   TG_TRY(contraction_join(c));
   if (hermitian)

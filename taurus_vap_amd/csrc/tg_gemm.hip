@@ -163,23 +163,6 @@ gemm_batched_kernel(int M, int N, int K, typename Scal<TC>::type alpha,
                                   blockIdx.y * BN, As, Bs);
 }
 
-template <typename TW>
-__global__ void __launch_bounds__(NT)
-gemm_grouped_kernel(int M, const cplx* __restrict__ X, cplx* __restrict__ C,
-                    const TW* __restrict__ W, const GroupDesc* __restrict__ groups,
-                    const int* __restrict__ tile_group, const int* __restrict__ tile_n0) {
-  __shared__ cplx As[BK][BM + 1];
-  __shared__ double Bs[BK][BN + 1];
-  const int tile = blockIdx.x;
-  const GroupDesc g = groups[tile_group[tile]];
-  const int n0 = tile_n0[tile];
-  const cplx* Xg = X + (long long)g.off * M;
-  cplx* Cg = C + (long long)g.off * M;
-  gemm_tile<cplx, TW, cplx, OP_N, OP_N>(M, g.size, g.size, cmk(1.0, 0.0), Xg, M, W + g.woff,
-                                        g.size, cmk(0.0, 0.0), false, Cg, M, blockIdx.y * BM, n0,
-                                        As, Bs);
-}
-
 template <typename TA, typename TB, typename TC, int OPA, int OPB>
 int launch(hipStream_t s, int M, int N, int K, typename Scal<TC>::type alpha, const TA* A,
            int lda, long long sA, const TB* B, int ldb, long long sB,
@@ -337,16 +320,16 @@ int gemm_tune_zd(hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, const c
 }
 
 bool gemm_grouped_tuned(int M, int ntiles_total, int tag) {
-  if (!sel().mfma || sel().grouped >= 0) return true;
+  if (M <= TG_GROUPED_VEC || !sel().mfma || sel().grouped >= 0) return true;
   return choices().count(GemmKey{K_GROUPED, tag, 0, M, ntiles_total, 0, 1}) != 0;
 }
 
-int gemm_tune_grouped(hipStream_t s, int M, const cplx* X, cplx* C, const void* W, int w_is_fp32,
+int gemm_tune_grouped(hipStream_t s, int M, const cplx* X, cplx* C, int ld, const void* W,
                       const GroupDesc* groups_dev, const int* tile_group_dev,
-                      const int* tile_n0_dev, int ntiles_total, int tag) {
+                      const int* tile_j0_dev, int ntiles_total, int tag) {
   const GemmKey key{K_GROUPED, tag, 0, M, ntiles_total, 0, 1};
   return tune(s, key, TG_MFMA_GROUPED_VARIANTS, [&](int v) {
-    return mfma_gemm_grouped(v, s, M, X, C, W, w_is_fp32, groups_dev, tile_group_dev, tile_n0_dev,
+    return mfma_gemm_grouped(v, s, M, X, C, ld, W, groups_dev, tile_group_dev, tile_j0_dev,
                              ntiles_total);
   });
 }
@@ -404,21 +387,9 @@ int gemm_dd(hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, double alpha
                                           beta, beta != 0.0, C, ldc, sC, batch, divA, divB);
 }
 
-int gemm_grouped(hipStream_t s, int M, const cplx* X, cplx* C, const void* W, int w_is_fp32,
-                 const GroupDesc* groups_dev, const int* tile_group_dev, const int* tile_n0_dev,
+int gemm_grouped(hipStream_t s, int M, const cplx* X, cplx* C, int ld, const void* W,
+                 const GroupDesc* groups_dev, const int* tile_group_dev, const int* tile_j0_dev,
                  int tag, int ntiles_total) {
-  if (M <= 0 || ntiles_total <= 0) return TG_OK;
-  if (sel().mfma)
-    return mfma_gemm_grouped(variant_for(GemmKey{K_GROUPED, tag, 0, M, ntiles_total, 0, 1}), s, M,
-                             X, C, W, w_is_fp32, groups_dev, tile_group_dev, tile_n0_dev,
-                             ntiles_total);
-  dim3 grid(ntiles_total, (M + BM - 1) / BM, 1);
-  if (w_is_fp32)
-    hipLaunchKernelGGL(gemm_grouped_kernel<float>, grid, dim3(NT), 0, s, M, X, C,
-                       (const float*)W, groups_dev, tile_group_dev, tile_n0_dev);
-  else
-    hipLaunchKernelGGL(gemm_grouped_kernel<double>, grid, dim3(NT), 0, s, M, X, C,
-                       (const double*)W, groups_dev, tile_group_dev, tile_n0_dev);
-  TG_HIP(hipGetLastError());
-  return TG_OK;
+  return mfma_gemm_grouped(variant_for(GemmKey{K_GROUPED, tag, 0, M, ntiles_total, 0, 1}), s, M, X, C,
+                           ld, W, groups_dev, tile_group_dev, tile_j0_dev, ntiles_total);
 }

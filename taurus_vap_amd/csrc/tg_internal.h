@@ -111,17 +111,22 @@ int gemm_dd(hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, double alpha
             double beta, double* C, int ldc, long long sC, int batch, int divA = 1,
             int divB = 1);
 
-// Grouped GEMM for the contraction blocks:
-//   C_g (M x s_g, ld M) = X_g (M x s_g, ld M) * W_g (s_g x s_g, ld s_g)
-// X_g / C_g start at column offset off_g of X / C; W_g at woff_g (float or double).
+// Grouped GEMM for the contraction blocks: for every group g and angle a,
+//   C(off + j, a) = sum_k W_g(k, j) X(off + k, a), j, k < size,
+// X and C with rows of `ld` angles per position (angle contiguous), W_g(k, j) at
+// k size + j.  grouped_ld(M): the row stride for M angles (whole 128-byte lines above
+// the vector kernels' TG_GROUPED_VEC angles).
+constexpr int TG_GROUPED_VEC = 4;
+inline int grouped_ld(int M) { return M <= TG_GROUPED_VEC ? M : (M + 7) / 8 * 8; }
 struct GroupDesc {
-  int off;        // first column of the group in X/C
+  int off;        // first position of the group in X / C
   int size;       // s_g
-  long long woff; // offset of W_g
+  long long woff; // byte offset of W_g
+  int fp32;       // W_g in float (else double)
 };
 // `tag` names the channel (0 = ph, 1 = pp) for the autotuner.
-int gemm_grouped(hipStream_t s, int M, const cplx* X, cplx* C, const void* W, int w_is_fp32,
-                 const GroupDesc* groups_dev, const int* tile_group_dev, const int* tile_n0_dev,
+int gemm_grouped(hipStream_t s, int M, const cplx* X, cplx* C, int ld, const void* W,
+                 const GroupDesc* groups_dev, const int* tile_group_dev, const int* tile_j0_dev,
                  int tag, int ntiles_total);
 
 // Autotuner: time every matrix-core tile variant of one GEMM signature on the
@@ -136,9 +141,9 @@ int gemm_tune_dz(hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, const d
 int gemm_tune_zd(hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, const cplx* A, int lda,
                  long long sA, const double* B, int ldb, long long sB, cplx* C, int ldc,
                  long long sC, int batch);
-int gemm_tune_grouped(hipStream_t s, int M, const cplx* X, cplx* C, const void* W, int w_is_fp32,
+int gemm_tune_grouped(hipStream_t s, int M, const cplx* X, cplx* C, int ld, const void* W,
                       const GroupDesc* groups_dev, const int* tile_group_dev,
-                      const int* tile_n0_dev, int ntiles_total, int tag);
+                      const int* tile_j0_dev, int ntiles_total, int tag);
 // true when gemm_tune_grouped has nothing left to time for this signature
 bool gemm_grouped_tuned(int M, int ntiles_total, int tag);
 // tile variant the dispatcher uses for a signature (kind: 0 zz, 1 dz, 2 zd, 3 grouped)
@@ -163,18 +168,21 @@ int batched_pfaffian(hipStream_t s, int n, cplx* A, int lda, long long sA, int b
 // ---------------------------------------------------------------------------
 // Contraction plan (tg_fields.hip)
 // ---------------------------------------------------------------------------
+// An orbit of matrix elements under the symmetries of its block and the sums the
+// contraction takes over it (kernels of tg_fields.hip); m elements and m sums.
+struct Orbit {
+  int lin[4];                   // linear indices x + y*n of the elements
+  int pos[4];                   // positions of the sums
+  unsigned mask;                // bit 4 j + i: element i enters sum j with a minus
+  int m;
+};
+
 struct Channel {
   int npos = 0;                 // number of positions (n*n for ph, n(n-1)/2 for pp)
-  int ngroups = 0;
-  std::vector<GroupDesc> groups;
-  std::vector<int> perm;        // position -> linear index (x + y*n) of the element
-  // linear index -> position: >= 0 for a stored element; pp: -2 - position of
-  // the transposed element for x < y (the field there is minus it), -1 on the
-  // diagonal
-  std::vector<int> inv;
-  long long wsize = 0;          // sum of s_g^2
-  DevBuf d_inv, d_groups, d_W, d_tile_group, d_tile_n0;
-  int ntiles_n = 0, ntiles_total = 0;
+  int ngroups = 0, norb = 0;
+  int mo = 1;                   // sums of an orbit at most
+  DevBuf d_orb, d_groups, d_W, d_tile_group, d_tile_n0;
+  int ntiles_total = 0;
 };
 
 // Configuration a captured projection graph is valid for.

@@ -34,11 +34,9 @@ template <> struct IsC<cplx> { static constexpr bool v = true; };
 
 __device__ inline void split(cplx v, double& r, double& i) { r = v.x; i = v.y; }
 __device__ inline void split(double v, double& r, double& i) { r = v; i = 0.0; }
-__device__ inline void split(float v, double& r, double& i) { r = (double)v; i = 0.0; }
 
 template <typename T> __device__ inline T zero_v();
 template <> __device__ inline double zero_v<double>() { return 0.0; }
-template <> __device__ inline float zero_v<float>() { return 0.0f; }
 template <> __device__ inline cplx zero_v<cplx>() { return cmk(0.0, 0.0); }
 
 constexpr int XCDS = 8;
@@ -327,19 +325,177 @@ mfma_dd_kernel(int M, int N, int K, double alpha, const double* __restrict__ A, 
   }
 }
 
-// Grouped contraction: C_g (M x s_g) = X_g (M x s_g) W_g (s_g x s_g), W real (float/double).
-template <typename TW, int BM, int BN, int WM, int WN, int OCC = 1>
-__global__ void __launch_bounds__(64 * WM * WN * OCC)
-mfma_grouped_kernel(int M, const cplx* __restrict__ X, cplx* __restrict__ C,
-                    const TW* __restrict__ W, const GroupDesc* __restrict__ groups,
-                    const int* __restrict__ tile_group, const int* __restrict__ tile_n0) {
-  typedef Tile<cplx, TW, OP_N, OP_N, BM, BN, WM, WN> T;
-  __shared__ typename T::Smem sm;
-  const int tile = blockIdx.x;
-  const GroupDesc g = groups[tile_group[tile]];
-  const int n0 = tile_n0[tile];
-  T::run(M, g.size, g.size, cmk(1.0, 0.0), X + (long long)g.off * M, M, W + g.woff, g.size,
-         cmk(0.0, 0.0), false, C + (long long)g.off * M, M, blockIdx.y * BM, n0, sm);
+// Grouped contraction: C(j, a) = sum_k W_g(k, j) X(k, a) for every group g; X and C hold
+// a row of `ld` angles per position (angle contiguous), W_g is real, j contiguous.  The
+// scheme of mfma_batched_kernel with both operands contiguous across the lanes: a wave
+// takes TJ x 16 positions and TA x 16 angles of one group.  tile_group / tile_j0 list
+// tiles of 64 positions, entry t for XCD t % 8 (group < 0: none); a group stays on one
+// XCD, whose L2 then holds its X and W_g, and the groups are dealt to the XCDs by work.
+// A unit of work is (tile, angle tile, part of the tile), four neighbouring units of an
+// XCD's list per workgroup.
+// Bound by the matrix cores: 225 angles x 400 groups of up to 820 positions 1.04 ms, 55
+// TF/s (72 % of the FP64 matrix rate with the padding of the tiles counted), 450 angles x
+// 200 groups 0.95 ms, 60 TF/s.  Through LDS with 80 x 64 tiles 1.17 and 1.07 ms; with the
+// groups not kept on one XCD 1.10 and 1.06 ms; with X and W contiguous in k (each lane
+// its own row) 1.46 and 1.39 ms.
+struct GroupedArgs {
+  int M;                       // angles
+  int ld;                      // stride of a position's row (>= M)
+  const cplx* X;
+  cplx* C;
+  const void* W;
+  const GroupDesc* groups;
+  const int* tile_group;
+  const int* tile_j0;
+  int mtiles, units;
+};
+
+template <typename TW, int TA, int TJ, int KS>
+__device__ __forceinline__ void grouped_tile(const GroupedArgs& g, const GroupDesc& gd, int a0, int j0) {
+  const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+  const int s = gd.size;
+  const cplx* Xb = g.X + (long long)gd.off * g.ld;
+  const TW* Wb = reinterpret_cast<const TW*>(static_cast<const char*>(g.W) + gd.woff);
+  unsigned xo[TA], wo[TJ];
+#pragma unroll
+  for (int x = 0; x < TA; ++x) xo[x] = min(a0 + 16 * x + lr, g.M - 1) + lk * g.ld;
+#pragma unroll
+  for (int y = 0; y < TJ; ++y) wo[y] = min(j0 + 16 * y + lr, s - 1) + lk * s;
+  d4 cr[TA][TJ], ci[TA][TJ];
+#pragma unroll
+  for (int x = 0; x < TA; ++x)
+#pragma unroll
+    for (int y = 0; y < TJ; ++y) {
+      cr[x][y] = d4{0.0, 0.0, 0.0, 0.0};
+      ci[x][y] = d4{0.0, 0.0, 0.0, 0.0};
+    }
+  cplx xv[KS][TA];
+  TW wv[KS][TJ];
+  auto load = [&](int q, int k0, bool mask) {
+    const cplx* px = Xb + (long long)(k0 + 4 * q) * g.ld;
+    const TW* pw = Wb + (long long)(k0 + 4 * q) * s;
+    const bool in = !mask || k0 + 4 * q + lk < s;
+#pragma unroll
+    for (int x = 0; x < TA; ++x) {
+      if (mask) xv[q][x] = cmk(0.0, 0.0);
+      if (in) xv[q][x] = px[xo[x]];
+    }
+#pragma unroll
+    for (int y = 0; y < TJ; ++y) {
+      if (mask) wv[q][y] = (TW)0;
+      if (in) wv[q][y] = pw[wo[y]];
+    }
+  };
+  auto multiply = [&](int q) {
+#pragma unroll
+    for (int x = 0; x < TA; ++x)
+#pragma unroll
+      for (int y = 0; y < TJ; ++y) {
+        cr[x][y] = mfma((double)wv[q][y], xv[q][x].x, cr[x][y]);
+        ci[x][y] = mfma((double)wv[q][y], xv[q][x].y, ci[x][y]);
+      }
+  };
+  const int kf = s / (4 * KS) * (4 * KS);
+  if (kf > 0) {
+#pragma unroll
+    for (int q = 0; q < KS; ++q) load(q, 0, false);
+#pragma unroll 1
+    for (int k0 = 4 * KS; k0 < kf; k0 += 4 * KS) {
+#pragma unroll
+      for (int q = 0; q < KS; ++q) {
+        multiply(q);
+        __builtin_amdgcn_sched_barrier(0);
+        load(q, k0, false);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < KS; ++q) multiply(q);
+  }
+  if (kf < s) {
+#pragma unroll
+    for (int q = 0; q < KS; ++q) load(q, kf, true);
+#pragma unroll
+    for (int q = 0; q < KS; ++q) multiply(q);
+  }
+  // lane: rows lk + 4 r (positions), column lr (angle) of each 16 x 16 block
+#pragma unroll
+  for (int x = 0; x < TA; ++x) {
+    const int a = a0 + 16 * x + lr;
+    if (a >= g.M) continue;
+#pragma unroll
+    for (int y = 0; y < TJ; ++y)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int j = j0 + 16 * y + lk + 4 * r;
+        if (j < s) g.C[(long long)(gd.off + j) * g.ld + a] = cmk(cr[x][y][r], ci[x][y][r]);
+      }
+  }
+}
+
+template <int TA, int TJ, int KS, int OCC>
+__global__ void __launch_bounds__(256, OCC)
+mfma_grouped_kernel(GroupedArgs g) {
+  constexpr int PARTS = 4 / TJ;
+  const int u = blockIdx.x / XCDS * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (u >= g.units) return;
+  const int part = u % PARTS, at = u / PARTS % g.mtiles;
+  const int tile = u / (PARTS * g.mtiles) * XCDS + blockIdx.x % XCDS;
+  const int grp = g.tile_group[tile];
+  if (grp < 0) return;
+  const GroupDesc gd = g.groups[grp];
+  const int j0 = g.tile_j0[tile] + 16 * TJ * part;
+  if (j0 >= gd.size) return;
+  if (gd.fp32) grouped_tile<float, TA, TJ, KS>(g, gd, at * 16 * TA, j0);
+  else grouped_tile<double, TA, TJ, KS>(g, gd, at * 16 * TA, j0);
+}
+
+// The same for M <= 4 angles: matrix-vector products, bound by reading W once.  A
+// workgroup takes one tile of 64 positions, a lane a position; its eight waves take
+// eighths of k (X elements are uniform loads) and meet in LDS.
+constexpr int GV_W = 8;
+template <typename TW, int M>
+__device__ __forceinline__ void grouped_vec(const GroupedArgs& g, const GroupDesc& gd, int j0,
+                                            cplx (&acc)[M]) {
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int s = gd.size, k0 = (int)((long long)s * w / GV_W), k1 = (int)((long long)s * (w + 1) / GV_W);
+  const TW* W = reinterpret_cast<const TW*>(static_cast<const char*>(g.W) + gd.woff) + min(j0 + lane, s - 1);
+  const cplx* X = g.X + (long long)gd.off * g.ld;
+#pragma unroll 16
+  for (int k = k0; k < k1; ++k) {
+    const double v = (double)W[(long long)k * s];
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      const cplx x = X[(long long)k * g.ld + m];
+      acc[m].x = fma(x.x, v, acc[m].x);
+      acc[m].y = fma(x.y, v, acc[m].y);
+    }
+  }
+}
+
+template <int M>
+__global__ void __launch_bounds__(64 * GV_W)
+grouped_vec_kernel(GroupedArgs g) {
+  __shared__ cplx part[GV_W][M][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int grp = g.tile_group[blockIdx.x];
+  if (grp < 0) return;
+  const GroupDesc gd = g.groups[grp];
+  const int j0 = g.tile_j0[blockIdx.x];
+  cplx acc[M];
+#pragma unroll
+  for (int m = 0; m < M; ++m) acc[m] = cmk(0.0, 0.0);
+  if (gd.fp32) grouped_vec<float, M>(g, gd, j0, acc);
+  else grouped_vec<double, M>(g, gd, j0, acc);
+#pragma unroll
+  for (int m = 0; m < M; ++m) part[w][m][lane] = acc[m];
+  __syncthreads();
+  if (w < M && j0 + lane < gd.size) {
+    cplx v = part[0][w][lane];
+#pragma unroll
+    for (int q = 1; q < GV_W; ++q) v = cadd(v, part[q][w][lane]);
+    g.C[(long long)(gd.off + j0 + lane) * g.ld + w] = v;
+  }
 }
 
 template <typename TA, typename TB, int OPA, int OPB, int BM, int BN, int WM, int WN,
@@ -454,55 +610,43 @@ int mfma_gemm_zd(int variant, hipStream_t s, TgOp opa, TgOp opb, int M, int N, i
                                 use_beta, C, ldc, sC, batch, divA, divB);
 }
 
-int mfma_gemm_grouped(int variant, hipStream_t s, int M, const cplx* X, cplx* C, const void* W,
-                      int w_is_fp32, const GroupDesc* groups_dev, const int* tile_group_dev,
-                      const int* tile_n0_dev, int ntiles_total) {
+int mfma_gemm_grouped(int variant, hipStream_t s, int M, const cplx* X, cplx* C, int ld,
+                      const void* W, const GroupDesc* groups_dev, const int* tile_group_dev,
+                      const int* tile_j0_dev, int ntiles_total) {
   if (M <= 0 || ntiles_total <= 0) return TG_OK;
-  // the tile lists are built for 64-column tiles of each group
-  if (variant == 0) {
-    dim3 grid(ntiles_total, (M + 63) / 64, 1);
-    if (w_is_fp32)
-      hipLaunchKernelGGL((mfma_grouped_kernel<float, 64, 64, 2, 2>), grid, dim3(256), 0, s, M, X,
-                         C, (const float*)W, groups_dev, tile_group_dev, tile_n0_dev);
-    else
-      hipLaunchKernelGGL((mfma_grouped_kernel<double, 64, 64, 2, 2>), grid, dim3(256), 0, s, M, X,
-                         C, (const double*)W, groups_dev, tile_group_dev, tile_n0_dev);
-  } else if (variant == 1) {
-    dim3 grid(ntiles_total, (M + 127) / 128, 1);
-    if (w_is_fp32)
-      hipLaunchKernelGGL((mfma_grouped_kernel<float, 128, 64, 4, 1>), grid, dim3(256), 0, s, M, X,
-                         C, (const float*)W, groups_dev, tile_group_dev, tile_n0_dev);
-    else
-      hipLaunchKernelGGL((mfma_grouped_kernel<double, 128, 64, 4, 1>), grid, dim3(256), 0, s, M,
-                         X, C, (const double*)W, groups_dev, tile_group_dev, tile_n0_dev);
-  } else if (variant == 2) {
-    dim3 grid(ntiles_total, (M + 255) / 256, 1);
-    if (w_is_fp32)
-      hipLaunchKernelGGL((mfma_grouped_kernel<float, 256, 64, 4, 2>), grid, dim3(512), 0, s, M, X,
-                         C, (const float*)W, groups_dev, tile_group_dev, tile_n0_dev);
-    else
-      hipLaunchKernelGGL((mfma_grouped_kernel<double, 256, 64, 4, 2>), grid, dim3(512), 0, s, M,
-                         X, C, (const double*)W, groups_dev, tile_group_dev, tile_n0_dev);
-  } else if (variant == 3) {
-    dim3 grid(ntiles_total, (M + 127) / 128, 1);
-    if (w_is_fp32)
-      hipLaunchKernelGGL((mfma_grouped_kernel<float, 128, 64, 4, 1, 2>), grid, dim3(256), 0, s, M,
-                         X, C, (const float*)W, groups_dev, tile_group_dev, tile_n0_dev);
-    else
-      hipLaunchKernelGGL((mfma_grouped_kernel<double, 128, 64, 4, 1, 2>), grid, dim3(256), 0, s, M,
-                         X, C, (const double*)W, groups_dev, tile_group_dev, tile_n0_dev);
-  } else if (variant == 4) {
-    dim3 grid(ntiles_total, (M + 63) / 64, 1);
-    if (w_is_fp32)
-      hipLaunchKernelGGL((mfma_grouped_kernel<float, 64, 64, 2, 2, 3>), grid, dim3(256), 0, s, M, X,
-                         C, (const float*)W, groups_dev, tile_group_dev, tile_n0_dev);
-    else
-      hipLaunchKernelGGL((mfma_grouped_kernel<double, 64, 64, 2, 2, 3>), grid, dim3(256), 0, s, M,
-                         X, C, (const double*)W, groups_dev, tile_group_dev, tile_n0_dev);
-  } else {
-    tg_set_error("mfma grouped gemm: bad tile variant");
-    return TG_E_ARG;
+  GroupedArgs g{M, ld, X, C, W, groups_dev, tile_group_dev, tile_j0_dev, 1, 0};
+  if (M <= TG_GROUPED_VEC) {
+    const dim3 grid(ntiles_total), th(64 * GV_W);
+    if (M == 1) hipLaunchKernelGGL(grouped_vec_kernel<1>, grid, th, 0, s, g);
+    else if (M == 2) hipLaunchKernelGGL(grouped_vec_kernel<2>, grid, th, 0, s, g);
+    else if (M == 3) hipLaunchKernelGGL(grouped_vec_kernel<3>, grid, th, 0, s, g);
+    else hipLaunchKernelGGL(grouped_vec_kernel<4>, grid, th, 0, s, g);
+    TG_HIP(hipGetLastError());
+    return TG_OK;
   }
+#define TG_GROUPED(TA, TJ, KS, OCC)                                                            \
+  do {                                                                                         \
+    g.mtiles = (M + 16 * TA - 1) / (16 * TA);                                                  \
+    const long long units = (long long)(4 / TJ) * (ntiles_total / XCDS) * g.mtiles;            \
+    if (units > 0x3fffffffLL) {                                                                \
+      tg_set_error("mfma grouped gemm: grid too large");                                       \
+      return TG_E_ARG;                                                                         \
+    }                                                                                          \
+    g.units = (int)units;                                                                      \
+    hipLaunchKernelGGL((mfma_grouped_kernel<TA, TJ, KS, OCC>),                                 \
+                       dim3((unsigned)((units + 3) / 4 * XCDS)), dim3(256), 0, s, g);          \
+  } while (0)
+  switch (variant) {
+    case 0: TG_GROUPED(3, 2, 2, 3); break;
+    case 1: TG_GROUPED(3, 2, 3, 2); break;
+    case 2: TG_GROUPED(2, 2, 4, 3); break;
+    case 3: TG_GROUPED(2, 2, 2, 4); break;
+    case 4: TG_GROUPED(1, 2, 4, 4); break;
+    default:
+      tg_set_error("mfma grouped gemm: bad tile variant");
+      return TG_E_ARG;
+  }
+#undef TG_GROUPED
   TG_HIP(hipGetLastError());
   return TG_OK;
 }

@@ -966,7 +966,8 @@ int project_upload(tg_ctx* c) {
       const size_t nn = (size_t)F.nn;
       const size_t per_item = sizeof(cplx) * (W_COUNT * nn) + (F.chunk ? F.pfw_bytes / F.chunk : 0) +
                               sizeof(cplx) * 4 * nn;   // contraction layouts (upper bound)
-      const size_t fixed = sizeof(cplx) * 2 * (size_t)F.B * nn;
+      // (and the contraction's rows of angles filled up to whole lines)
+      const size_t fixed = sizeof(cplx) * (2 * (size_t)F.B + 32) * nn;
       const size_t budget = (size_t)(0.85 * (double)have);
       if (fixed + per_item * (size_t)F.chunk > budget && budget > fixed + per_item)
         c->mem_chunk = (int)std::max<size_t>(1, (budget - fixed) / per_item);
@@ -1763,7 +1764,7 @@ int tg_finalize(tg_ctx* c) {
                     &c->d_Z, &c->d_psign, &c->d_cHO, &c->d_it, &c->d_obs, &c->d_canon, &c->d_cq})
     b->release();
   for (Channel* ch : {&c->ph, &c->pp})
-    for (DevBuf* b : {&ch->d_inv, &ch->d_groups, &ch->d_W, &ch->d_tile_group, &ch->d_tile_n0})
+    for (DevBuf* b : {&ch->d_orb, &ch->d_groups, &ch->d_W, &ch->d_tile_group, &ch->d_tile_n0})
       b->release();
   if (c->stream2) (void)hipStreamSynchronize(c->stream2);
   if (c->stream3) (void)hipStreamSynchronize(c->stream3);
