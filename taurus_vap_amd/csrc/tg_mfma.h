@@ -1,12 +1,12 @@
-// FP64 matrix-core GEMM entry points (tg_mfma.hip).  `variant` selects the tile
-// shape: 0 = 64x64 (2x2 waves), 1 = 48x48 (3 waves), 2 = 112x112 (7 waves),
-// 3 = 96x64 (2x2 waves), 4 / 5 = 112x112 / 48x48 with every XCD given the same
-// number of tiles, 6 / 7 = 48x48 bounded to four workgroups per CU, 8 = 64x32
-// (2 waves, 256 VGPRs), 9 / 10 = 7 / 5 with both operands staged k-major in LDS;
-// grouped (angles x positions per wave, k steps of 4 in flight): 0 = 48x32, 2; 1 = 48x32,
-// 3; 2 = 32x32, 4; 3 = 32x32, 2 (four waves per SIMD); 4 = 16x32, 4; up to TG_GROUPED_VEC
-// angles take matrix-vector kernels whatever the variant.  Batch element b reads A + (b / divA) * sA and
-// B + (b / divB) * sB (an operand shared by runs of divA consecutive elements).
+// FP64 matrix-core GEMM entry points (tg_mfma.hip).  `variant` selects the tile of a wave
+// (rows x columns, k steps of 4 in flight): 0 = 32x32, 2; 1 = 32x32, 4; 2 = 48x32, 2;
+// 3 = 32x48, 2; 4 = 48x32, 3; 5 = 48x16, 3; 6 = 32x16, 3; 7 = 32x16, 4; 8 = 16x16, 2;
+// 9 = 16x16, 4; 10 = 48x16, 4.
+// Grouped (angles x positions): 0 = 48x32, 2; 1 = 48x32, 3; 2 = 32x32, 4; 3 = 32x32, 2
+// (four waves per SIMD); 4 = 16x32, 4; up to TG_GROUPED_VEC angles take matrix-vector
+// kernels whatever the variant.
+// Batch element b reads A + (b / divA) * sA and B + (b / divB) * sB (an operand shared by
+// runs of divA consecutive elements).
 #pragma once
 #include "tg_internal.h"
 

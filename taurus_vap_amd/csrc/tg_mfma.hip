@@ -1,23 +1,13 @@
 // FP64 matrix-core GEMMs (v_mfma_f64_16x16x4f64) for gfx950.
 //
-// C[b] = alpha * op(A[b]) op(B[b]) + beta * C[b], column-major, with complex
-// operands split into real and imaginary planes in LDS:
-//   complex x complex : Cr += Ar Br - Ai Bi, Ci += Ar Bi + Ai Br  (4 MFMA)
-//   real x complex    : Cr += A Br,          Ci += A Bi          (2 MFMA)
-//   complex x real    : Cr += Ar B,          Ci += Ai B          (2 MFMA)
-// A workgroup of WM x WN waves owns a BM x BN tile of C; each wave owns a
-// (BM/WM) x (BN/WN) sub-tile of 16 x 16 MFMA blocks.  K advances in chunks of 16
-// staged through LDS; the next chunk is loaded into registers while the
-// current one is multiplied.  Each operand is kept in LDS with its contiguous
-// global dimension fastest, so the staging stores are unit-stride.
+// C[b] = alpha * op(A[b]) op(B[b]) + beta * C[b], column-major:
+//   complex x complex : three real products (Gauss)
+//   real x complex    : Cr += A Br, Ci += A Bi  (2 MFMA)
+//   complex x real    : Cr += Ar B, Ci += Ai B  (2 MFMA)
 //
 // MFMA 16x16x4 f64 operand layout (lane l = 0..63):
 //   A(16x4): lane l holds A[l % 16][l / 16];  B(4x16): lane l holds B[l / 16][l % 16];
 //   D(16x16): lane l, register r holds D[l / 16 + 4 * r][l % 16].
-//
-// Batched launches are mapped XCD-aware: workgroup ids are dealt round-robin
-// to the 8 XCDs, so all tiles of one batch element are given ids congruent
-// modulo 8 and share that XCD's L2.
 #include "tg_internal.h"
 #include "tg_mfma.h"
 
@@ -32,8 +22,8 @@ __device__ inline d4 mfma(double a, double b, d4 c) {
 template <typename T> struct IsC { static constexpr bool v = false; };
 template <> struct IsC<cplx> { static constexpr bool v = true; };
 
-__device__ inline void split(cplx v, double& r, double& i) { r = v.x; i = v.y; }
-__device__ inline void split(double v, double& r, double& i) { r = v; i = 0.0; }
+template <int OP> __device__ inline cplx conj_op(cplx v) { return OP == OP_C ? cconj(v) : v; }
+template <int OP> __device__ inline double conj_op(double v) { return v; }
 
 template <typename T> __device__ inline T zero_v();
 template <> __device__ inline double zero_v<double>() { return 0.0; }
@@ -41,222 +31,156 @@ template <> __device__ inline cplx zero_v<cplx>() { return cmk(0.0, 0.0); }
 
 constexpr int XCDS = 8;
 
-// KM = true stages both operands k-major in LDS ([k][i], [k][j], rows of BM / BN
-// plus a pad) whatever their layout in memory; false keeps each operand's
-// memory order (the row of a k-contiguous operand then holds BK + 1).
-template <typename TA, typename TB, int OPA, int OPB, int BM, int BN, int WM, int WN,
-          bool KM = false>
-struct Tile {
-  static constexpr int BK = 16;
-  static constexpr int NW = WM * WN, NTH = 64 * NW;
-  static constexpr int TM = BM / WM / 16, TN = BN / WN / 16;
-  static constexpr bool CA = IsC<TA>::v, CB = IsC<TB>::v;
-  // A(i,k) in memory: OP_N -> contiguous in i (AG), else contiguous in k
-  static constexpr bool AG = (OPA == OP_N);
-  // B(k,j) in memory: OP_N -> contiguous in k (BG), else contiguous in j
-  static constexpr bool BG = (OPB == OP_N);
-  // LDS: A as [k][i] (AK) or [i][k]; B as [j][k] (BJ) or [k][j]
-  static constexpr bool AK = AG || KM;
-  static constexpr bool BJ = BG && !KM;
-  static constexpr int PADR = 4;                   // pad of rows of length BM / BN
-  static constexpr int LDA_ = AK ? BM + PADR : BK + 1;
-  static constexpr int LDB_ = BJ ? BK + 1 : BN + PADR;
-  static constexpr int SA = AK ? BK * LDA_ : BM * LDA_;
-  static constexpr int SB = BJ ? BN * LDB_ : BK * LDB_;
-  static constexpr int NA = BM * BK / NTH, NB = BN * BK / NTH;
-  static_assert(BM % (16 * WM) == 0 && BN % (16 * WN) == 0, "tile");
-  static_assert((BM * BK) % NTH == 0 && (BN * BK) % NTH == 0, "staging");
-
-  __device__ static inline int ia(int i, int k) { return AK ? k * LDA_ + i : i * LDA_ + k; }
-  __device__ static inline int ib(int k, int j) { return BJ ? j * LDB_ + k : k * LDB_ + j; }
-
-  struct Smem {
-    double ar[SA];
-    double ai[CA ? SA : 1];
-    double br[SB];
-    double bi[CB ? SB : 1];
+// One (TM x 16) x (TN x 16) tile of C per wave, operands straight from global memory
+// (L1 / L2) into the matrix-core registers: a lane loads the element of op(A) and op(B)
+// that it feeds, so there is no LDS, no barrier and no wave waits for another.  KS steps
+// of 4 k each are in flight: a step's operands are loaded as soon as its registers are
+// free, KS - 1 steps of products before they are needed.  Lane quarter lk
+// takes k = k0 + KS lk + s in step s (any assignment serves, the same for both operands):
+// an operand contiguous in k is then read as whole runs of 4 KS elements.
+// The products are formed transposed (MFMA rows = columns of C), so that lanes 0..15
+// hold 16 consecutive rows of a column and loads and stores of C are unit-stride.
+// Rows and columns past the edge repeat the last one and are not stored; k past the
+// end is masked in the last chunk only.
+// Complex x complex is three real products (Gauss): cr = sum Ar Br, ci = sum Ai Bi,
+// c3 = sum (Ar + Ai)(Br + Bi); C = (cr - ci, c3 - cr - ci).
+// Bound by the matrix cores, the load latency covered by the steps in flight and 2-4
+// waves per SIMD.  The launch bound keeps the accumulators in VGPRs: without it the
+// compiler parks them in AGPRs and moves every one out and back in each trip (1.4-1.9 ms
+// for the first figure below).  Best tile of each, against workgroup tiles staged through
+// LDS with two barriers per 16 k (48 x 48, three waves; they spent a third of their time
+// waiting at barriers and for LDS):
+//   225 x 336^3 complex 0.81 ms (84 TF/s, 80 % of the matrix rate at three products), 0.99
+//     before; with A transposed 0.83 (0.99); real x complex 0.54 (0.64)
+//   78 x 224^3 0.090 (0.136), 0.100 (0.137), 0.067 (0.092)
+//   121 x 140^3 0.043 (0.065), 0.047 (0.063), 0.034 (0.039)
+//   1296 x 64^3 0.046 (0.064), 0.055 (0.063), 0.038 (0.043); 49 x 24^3 0.004 (0.007)
+template <typename TA, typename TB, int OPA, int OPB, int TM, int TN, int KS, int OCC>
+__global__ void __launch_bounds__(256, OCC)
+mfma_batched_kernel(int M, int N, int K, cplx alpha, const TA* __restrict__ A, int lda,
+                    long long sA, const TB* __restrict__ B, int ldb, long long sB, cplx beta,
+                    int use_beta, cplx* __restrict__ C, int ldc, long long sC, int batch,
+                    int tiles_m, int tiles, int per, int divA, int divB) {
+  constexpr bool CA = IsC<TA>::v, CB = IsC<TB>::v, CC = CA && CB;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // the batch * tiles (element, tile) pairs are cut into 8 contiguous runs, one per XCD
+  // (workgroup ids are dealt round-robin to the XCDs), so the tiles of one element share
+  // an L2 and every XCD gets the same number
+  const unsigned g = (blockIdx.x % XCDS * (unsigned)per + blockIdx.x / XCDS) * 4 + w;
+  if (g >= (unsigned)batch * (unsigned)tiles) return;
+  const int b = (int)(g / (unsigned)tiles), tile = (int)(g - (unsigned)b * (unsigned)tiles);
+  const int m0 = (tile % tiles_m) * 16 * TM, n0 = (tile / tiles_m) * 16 * TN;
+  const int lr = lane & 15, lk = lane >> 4;
+  const TA* Ab = A + (long long)(b / divA) * sA;
+  const TB* Bb = B + (long long)(b / divB) * sB;
+  constexpr bool AN = OPA == OP_N, BN = OPB == OP_N;
+  // element offsets of the lane's rows / columns at k = KS lk (32 bits: one matrix)
+  unsigned ao[TM], bo[TN];
+#pragma unroll
+  for (int x = 0; x < TM; ++x) {
+    const unsigned i = min(m0 + 16 * x + lr, M - 1);
+    ao[x] = AN ? i + KS * lk * (unsigned)lda : KS * lk + i * (unsigned)lda;
+  }
+#pragma unroll
+  for (int y = 0; y < TN; ++y) {
+    const unsigned j = min(n0 + 16 * y + lr, N - 1);
+    bo[y] = BN ? KS * lk + j * (unsigned)ldb : j + KS * lk * (unsigned)ldb;
+  }
+  const long long ka = AN ? lda : 1, kb = BN ? 1 : ldb;   // elements per k
+  d4 cr[TM][TN], ci[TM][TN], c3[CC ? TM : 1][CC ? TN : 1];
+#pragma unroll
+  for (int x = 0; x < TM; ++x)
+#pragma unroll
+    for (int y = 0; y < TN; ++y) {
+      cr[x][y] = d4{0.0, 0.0, 0.0, 0.0};
+      ci[x][y] = d4{0.0, 0.0, 0.0, 0.0};
+      if constexpr (CC) c3[x][y] = d4{0.0, 0.0, 0.0, 0.0};
+    }
+  TA va[KS][TM];
+  TB vb[KS][TN];
+  auto load = [&](int s, int k0, bool mask) {
+    const TA* pa = Ab + (k0 + s) * ka;
+    const TB* pb = Bb + (k0 + s) * kb;
+    const bool in = !mask || k0 + KS * lk + s < K;
+#pragma unroll
+    for (int x = 0; x < TM; ++x) {
+      if (mask) va[s][x] = zero_v<TA>();
+      if (in) va[s][x] = pa[ao[x]];
+    }
+#pragma unroll
+    for (int y = 0; y < TN; ++y) {
+      if (mask) vb[s][y] = zero_v<TB>();
+      if (in) vb[s][y] = pb[bo[y]];
+    }
   };
-
-  // element (i, k) of op(A) and (k, j) of op(B) handled by staging slot e
-  // (consecutive slots follow the memory order: coalesced loads)
-  __device__ static inline void slot_a(int e, int& i, int& k) {
-    if (AG) { i = e % BM; k = e / BM; } else { k = e % BK; i = e / BK; }
-  }
-  __device__ static inline void slot_b(int e, int& k, int& j) {
-    if (BG) { k = e % BK; j = e / BK; } else { j = e % BN; k = e / BN; }
-  }
-
-  // always inlined: several kernels share one tile body
-  __device__ __forceinline__ static void run(int M, int N, int K, cplx alpha, const TA* __restrict__ A, int lda,
-                             const TB* __restrict__ B, int ldb, cplx beta, bool use_beta,
-                             cplx* __restrict__ C, int ldc, int m0, int n0, Smem& sm) {
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int wm0 = (w % WM) * (BM / WM), wn0 = (w / WM) * (BN / WN);
-    const int lr = lane & 15, lk = lane >> 4;
-
-    // complex x complex in three real products (Gauss): cr = sum Ar Br, ci = sum
-    // Ai Bi, c3 = sum (Ar + Ai)(Br + Bi); C = (cr - ci, c3 - cr - ci) at the end.
-    // A real operand takes two products: cr, ci are the real and imaginary parts.
-    constexpr bool CC = CA && CB;
-    d4 cr[TM][TN], ci[TM][TN], c3[CC ? TM : 1][CC ? TN : 1];
+  auto multiply = [&](int s) {
 #pragma unroll
     for (int x = 0; x < TM; ++x)
 #pragma unroll
       for (int y = 0; y < TN; ++y) {
-        cr[x][y] = d4{0.0, 0.0, 0.0, 0.0};
-        ci[x][y] = d4{0.0, 0.0, 0.0, 0.0};
-        if constexpr (CC) c3[x][y] = d4{0.0, 0.0, 0.0, 0.0};
-      }
-
-    TA ra[NA];
-    TB rb[NB];
-    auto load = [&](int k0) {
-#pragma unroll
-      for (int r = 0; r < NA; ++r) {
-        int i, k;
-        slot_a(t + r * NTH, i, k);
-        const int gi = m0 + i, gk = k0 + k;
-        TA v = zero_v<TA>();
-        if (gi < M && gk < K) v = AG ? A[gi + (long long)gk * lda] : A[gk + (long long)gi * lda];
-        ra[r] = v;
-      }
-#pragma unroll
-      for (int r = 0; r < NB; ++r) {
-        int k, j;
-        slot_b(t + r * NTH, k, j);
-        const int gk = k0 + k, gj = n0 + j;
-        TB v = zero_v<TB>();
-        if (gk < K && gj < N) v = BG ? B[gk + (long long)gj * ldb] : B[gj + (long long)gk * ldb];
-        rb[r] = v;
-      }
-    };
-    auto store = [&]() {
-#pragma unroll
-      for (int r = 0; r < NA; ++r) {
-        int i, k;
-        slot_a(t + r * NTH, i, k);
-        double vr, vi;
-        split(ra[r], vr, vi);
-        sm.ar[ia(i, k)] = vr;
-        if (CA) sm.ai[ia(i, k)] = (OPA == OP_C) ? -vi : vi;
-      }
-#pragma unroll
-      for (int r = 0; r < NB; ++r) {
-        int k, j;
-        slot_b(t + r * NTH, k, j);
-        double vr, vi;
-        split(rb[r], vr, vi);
-        sm.br[ib(k, j)] = vr;
-        if (CB) sm.bi[ib(k, j)] = (OPB == OP_C) ? -vi : vi;
-      }
-    };
-
-    load(0);
-    for (int k0 = 0; k0 < K; k0 += BK) {
-      store();
-      __syncthreads();
-      if (k0 + BK < K) load(k0 + BK);
-#pragma unroll
-      for (int kk = 0; kk < BK; kk += 4) {
-        double ar[TM], ai[TM], br[TN], bi[TN];
-#pragma unroll
-        for (int x = 0; x < TM; ++x) {
-          const int idx = ia(wm0 + 16 * x + lr, kk + lk);
-          ar[x] = sm.ar[idx];
-          if (CA) ai[x] = sm.ai[idx];
-        }
-#pragma unroll
-        for (int y = 0; y < TN; ++y) {
-          const int idx = ib(kk + lk, wn0 + 16 * y + lr);
-          br[y] = sm.br[idx];
-          if (CB) bi[y] = sm.bi[idx];
-        }
-        double sa[CC ? TM : 1], sb[CC ? TN : 1];
+        const auto av = conj_op<OPA>(va[s][x]);
+        const auto bv = conj_op<OPB>(vb[s][y]);
         if constexpr (CC) {
-#pragma unroll
-          for (int x = 0; x < TM; ++x) sa[x] = ar[x] + ai[x];
-#pragma unroll
-          for (int y = 0; y < TN; ++y) sb[y] = br[y] + bi[y];
-        }
-#pragma unroll
-        for (int x = 0; x < TM; ++x)
-#pragma unroll
-          for (int y = 0; y < TN; ++y) {
-            if constexpr (CC) {
-              cr[x][y] = mfma(ar[x], br[y], cr[x][y]);
-              ci[x][y] = mfma(ai[x], bi[y], ci[x][y]);
-              c3[x][y] = mfma(sa[x], sb[y], c3[x][y]);
-            } else if constexpr (CA) {
-              cr[x][y] = mfma(ar[x], br[y], cr[x][y]);
-              ci[x][y] = mfma(ai[x], br[y], ci[x][y]);
-            } else {
-              cr[x][y] = mfma(ar[x], br[y], cr[x][y]);
-              ci[x][y] = mfma(ar[x], bi[y], ci[x][y]);
-            }
-          }
-      }
-      __syncthreads();
-    }
-
-    // epilogue: lane holds rows lk + 4*r of column lr of each 16x16 block
-#pragma unroll
-    for (int y = 0; y < TN; ++y) {
-      const int gj = n0 + wn0 + 16 * y + lr;
-      if (gj >= N) continue;
-#pragma unroll
-      for (int x = 0; x < TM; ++x) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int gi = m0 + wm0 + 16 * x + lk + 4 * r;
-          if (gi >= M) continue;
-          cplx* cp = C + gi + (long long)gj * ldc;
-          cplx p;
-          if constexpr (CC)
-            p = cmk(cr[x][y][r] - ci[x][y][r], c3[x][y][r] - cr[x][y][r] - ci[x][y][r]);
-          else
-            p = cmk(cr[x][y][r], ci[x][y][r]);
-          cplx v = cmul(alpha, p);
-          if (use_beta) v = cadd(v, cmul(beta, *cp));
-          *cp = v;
+          cr[x][y] = mfma(bv.x, av.x, cr[x][y]);
+          ci[x][y] = mfma(bv.y, av.y, ci[x][y]);
+          c3[x][y] = mfma(bv.x + bv.y, av.x + av.y, c3[x][y]);
+        } else if constexpr (CA) {
+          cr[x][y] = mfma(bv, av.x, cr[x][y]);
+          ci[x][y] = mfma(bv, av.y, ci[x][y]);
+        } else {
+          cr[x][y] = mfma(bv.x, av, cr[x][y]);
+          ci[x][y] = mfma(bv.y, av, ci[x][y]);
         }
       }
+  };
+  // step s of the next chunk is loaded as soon as step s of this one is multiplied
+  const int kf = K / (4 * KS) * (4 * KS);    // whole chunks
+  if (kf > 0) {
+#pragma unroll
+    for (int s = 0; s < KS; ++s) load(s, 0, false);
+    int k0 = 4 * KS;
+#pragma unroll 1
+    for (; k0 < kf; k0 += 4 * KS) {
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        multiply(s);
+        __builtin_amdgcn_sched_barrier(0);
+        load(s, k0, false);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
+#pragma unroll
+    for (int s = 0; s < KS; ++s) multiply(s);
   }
-};
-
-// Batched: grid = XCDS * per workgroups.  BAL = false: batch element b goes to
-// XCD b % 8 (per = ceil(batch / 8) * tiles); BAL = true: the batch * tiles
-// (element, tile) pairs are cut into 8 contiguous runs of `per`, one per XCD, so
-// every XCD gets the same number of tiles.  Either way the tiles of one element
-// are consecutive on their XCD.  OCC > 1 bounds the registers for OCC times the
-// workgroup's waves per CU.
-template <typename TA, typename TB, int OPA, int OPB, int BM, int BN, int WM, int WN, bool BAL,
-          int OCC, bool KM>
-__global__ void __launch_bounds__(64 * WM * WN * OCC)
-mfma_batched_kernel(int M, int N, int K, cplx alpha, const TA* __restrict__ A, int lda,
-                    long long sA, const TB* __restrict__ B, int ldb, long long sB, cplx beta,
-                    int use_beta, cplx* __restrict__ C, int ldc, long long sC, int batch,
-                    int tiles_m, int tiles, long long per, int divA, int divB) {
-  typedef Tile<TA, TB, OPA, OPB, BM, BN, WM, WN, KM> T;
-  __shared__ typename T::Smem sm;
-  const int L = blockIdx.x;
-  const int xcd = L % XCDS, q = L / XCDS;
-  long long b;
-  int tile;
-  if (BAL) {
-    const long long g = (long long)xcd * per + q;
-    if (g >= (long long)batch * tiles) return;
-    b = g / tiles;
-    tile = (int)(g - b * tiles);
-  } else {
-    const int slot = q / tiles;
-    tile = q % tiles;
-    b = xcd + (long long)XCDS * slot;
-    if (b >= batch) return;
+  if (kf < K) {
+#pragma unroll
+    for (int s = 0; s < KS; ++s) load(s, kf, true);
+#pragma unroll
+    for (int s = 0; s < KS; ++s) multiply(s);
   }
-  const int tm = tile % tiles_m, tn = tile / tiles_m;
-  T::run(M, N, K, alpha, A + (b / divA) * sA, lda, B + (b / divB) * sB, ldb, beta, use_beta != 0,
-         C + b * sC, ldc, tm * BM, tn * BN, sm);
+  // lane: row lr, columns lk + 4 r of each 16 x 16 block
+  cplx* Cb = C + (long long)b * sC;
+#pragma unroll
+  for (int x = 0; x < TM; ++x) {
+    const int gi = m0 + 16 * x + lr;
+    if (gi >= M) continue;
+#pragma unroll
+    for (int y = 0; y < TN; ++y)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int gj = n0 + 16 * y + lk + 4 * r;
+        if (gj >= N) continue;
+        cplx* cp = Cb + gi + (long long)gj * ldc;
+        cplx p;
+        if constexpr (CC)
+          p = cmk(cr[x][y][r] - ci[x][y][r], c3[x][y][r] - cr[x][y][r] - ci[x][y][r]);
+        else
+          p = cmk(cr[x][y][r], ci[x][y][r]);
+        cplx v = cmul(alpha, p);
+        if (use_beta) v = cadd(v, cmul(beta, *cp));
+        *cp = v;
+      }
+  }
 }
 
 // Real FP64 GEMM on the matrix cores for the real products of the constraint
@@ -498,24 +422,22 @@ grouped_vec_kernel(GroupedArgs g) {
   }
 }
 
-template <typename TA, typename TB, int OPA, int OPB, int BM, int BN, int WM, int WN,
-          bool BAL = false, int OCC = 1, bool KM = false>
+template <typename TA, typename TB, int OPA, int OPB, int TM, int TN, int KS, int OCC>
 int launch_batched(hipStream_t s, int M, int N, int K, cplx alpha, const TA* A, int lda,
                    long long sA, const TB* B, int ldb, long long sB, cplx beta, int use_beta,
                    cplx* C, int ldc, long long sC, int batch, int divA, int divB) {
-  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+  const int tiles_m = (M + 16 * TM - 1) / (16 * TM), tiles_n = (N + 16 * TN - 1) / (16 * TN);
   const int tiles = tiles_m * tiles_n;
-  const long long per = BAL ? ((long long)batch * tiles + XCDS - 1) / XCDS
-                            : (long long)((batch + XCDS - 1) / XCDS) * tiles;
-  const long long grid = (long long)XCDS * per;
-  if (grid > 0x7fffffffLL) {
+  const long long wgs = ((long long)batch * tiles + 3) / 4;      // four waves, a tile each
+  const long long per = (wgs + XCDS - 1) / XCDS, grid = (long long)XCDS * per;
+  if (grid > 0x1fffffffLL) {          // tile numbers in 32 bits
     tg_set_error("mfma gemm: grid too large");
     return TG_E_ARG;
   }
   if (grid == 0) return TG_OK;
-  hipLaunchKernelGGL((mfma_batched_kernel<TA, TB, OPA, OPB, BM, BN, WM, WN, BAL, OCC, KM>),
-                     dim3((unsigned)grid), dim3(64 * WM * WN), 0, s, M, N, K, alpha, A, lda, sA, B,
-                     ldb, sB, beta, use_beta, C, ldc, sC, batch, tiles_m, tiles, per, divA, divB);
+  hipLaunchKernelGGL((mfma_batched_kernel<TA, TB, OPA, OPB, TM, TN, KS, OCC>), dim3((unsigned)grid),
+                     dim3(256), 0, s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, use_beta, C, ldc,
+                     sC, batch, tiles_m, tiles, (int)per, divA, divB);
   TG_HIP(hipGetLastError());
   return TG_OK;
 }
@@ -524,43 +446,25 @@ template <typename TA, typename TB, int OPA, int OPB>
 int launch_variant(int variant, hipStream_t s, int M, int N, int K, cplx alpha, const TA* A,
                    int lda, long long sA, const TB* B, int ldb, long long sB, cplx beta,
                    int use_beta, cplx* C, int ldc, long long sC, int batch, int divA, int divB) {
+#define TG_V(K_, TM, TN, KS, OCC)                                                               \
+  case K_:                                                                                      \
+    return launch_batched<TA, TB, OPA, OPB, TM, TN, KS, OCC>(s, M, N, K, alpha, A, lda, sA, B,  \
+                                                             ldb, sB, beta, use_beta, C, ldc,   \
+                                                             sC, batch, divA, divB);
   switch (variant) {
-    case 0:
-      return launch_batched<TA, TB, OPA, OPB, 64, 64, 2, 2>(s, M, N, K, alpha, A, lda, sA, B, ldb,
-                                                            sB, beta, use_beta, C, ldc, sC, batch, divA, divB);
-    case 1:
-      return launch_batched<TA, TB, OPA, OPB, 48, 48, 1, 3>(s, M, N, K, alpha, A, lda, sA, B, ldb,
-                                                            sB, beta, use_beta, C, ldc, sC, batch, divA, divB);
-    case 2:
-      return launch_batched<TA, TB, OPA, OPB, 112, 112, 1, 7>(s, M, N, K, alpha, A, lda, sA, B,
-                                                              ldb, sB, beta, use_beta, C, ldc, sC,
-                                                              batch, divA, divB);
-    case 3:
-      return launch_batched<TA, TB, OPA, OPB, 96, 64, 2, 2>(s, M, N, K, alpha, A, lda, sA, B, ldb,
-                                                            sB, beta, use_beta, C, ldc, sC, batch,
-                                                            divA, divB);
-    case 4:
-      return launch_batched<TA, TB, OPA, OPB, 112, 112, 1, 7, true>(
-          s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, use_beta, C, ldc, sC, batch, divA, divB);
-    case 5:
-      return launch_batched<TA, TB, OPA, OPB, 48, 48, 1, 3, true>(
-          s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, use_beta, C, ldc, sC, batch, divA, divB);
-    case 6:
-      return launch_batched<TA, TB, OPA, OPB, 48, 48, 1, 3, false, 4>(
-          s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, use_beta, C, ldc, sC, batch, divA, divB);
-    case 7:
-      return launch_batched<TA, TB, OPA, OPB, 48, 48, 1, 3, true, 4>(
-          s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, use_beta, C, ldc, sC, batch, divA, divB);
-    case 8:
-      return launch_batched<TA, TB, OPA, OPB, 64, 32, 1, 2, true, 4>(
-          s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, use_beta, C, ldc, sC, batch, divA, divB);
-    case 9:
-      return launch_batched<TA, TB, OPA, OPB, 48, 48, 1, 3, true, 4, true>(
-          s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, use_beta, C, ldc, sC, batch, divA, divB);
-    case 10:
-      return launch_batched<TA, TB, OPA, OPB, 48, 48, 1, 3, true, 1, true>(
-          s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, use_beta, C, ldc, sC, batch, divA, divB);
+    TG_V(0, 2, 2, 2, 3)
+    TG_V(1, 2, 2, 4, 2)
+    TG_V(2, 3, 2, 2, 2)
+    TG_V(3, 2, 3, 2, 2)
+    TG_V(4, 3, 2, 3, 2)
+    TG_V(5, 3, 1, 3, 3)
+    TG_V(6, 2, 1, 3, 4)
+    TG_V(7, 2, 1, 4, 3)
+    TG_V(8, 1, 1, 2, 4)
+    TG_V(9, 1, 1, 4, 4)
+    TG_V(10, 3, 1, 4, 2)
   }
+#undef TG_V
   tg_set_error("mfma gemm: bad tile variant");
   return TG_E_ARG;
 }
