@@ -469,16 +469,7 @@ __device__ __forceinline__ int gj_source(const int* perm, int k0, int w, int t) 
   return src;
 }
 
-typedef double gj_d4 __attribute__((ext_vector_type(4)));
-constexpr int GJ_MFQ = 3;   // row blocks per wave in the matrix-core update (TH = 512)
-
-// MF (TH = 512, n <= 384): the rank-32 update of the other columns as 16 x 16
-// tiles of v_mfma_f64_16x16x4f64 (U = 16 then: one column tile of slack).  The
-// tile computes C^T = Pw^T W^T, so a lane holds 16 consecutive rows of four
-// columns (coalesced loads and stores) and each LDS operand serves 48 rows
-// instead of one; with the next tile's loads in flight during the products,
-// eight waves keep about four times the bytes of the scalar update in flight.
-template <int TH, int WIN, int U, bool MF>
+template <int TH, int WIN, int U>
 __global__ void __launch_bounds__(TH)
 gj_wide_kernel(int n, cplx* __restrict__ Aall, int lda, long long sA, cplx* __restrict__ det,
                int* __restrict__ info, int* __restrict__ perm_all) {
@@ -573,39 +564,6 @@ gj_wide_kernel(int n, cplx* __restrict__ Aall, int lda, long long sA, cplx* __re
     const int blk = t - k0;
     const bool inblk = own && blk >= 0 && blk < w;
     if (inblk) srcs[blk] = src;
-    // MF: matrix-core operands of W.  Wave v updates row blocks v + 8 q (q < 3,
-    // rows 16 (v + 8 q) + li), so every SIMD holds six of the 24 blocks of
-    // n <= 384; fr/fi[q][kk] = W(16 (v + 8 q) + li, 4 kk + lq), moved between
-    // waves through a TH x 16 slab of the (idle) Pw area per half
-    const int lane = t & 63, li = lane & 15, lq = lane >> 4;
-    const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
-    double fr[GJ_MFQ][8], fi[GJ_MFQ][8];
-    if constexpr (MF) {
-      cplx* slab = &Pw[0][0];
-#pragma unroll
-      for (int m = 0; m < H; ++m) slab[m * TH + t] = pA[m];
-      __syncthreads();
-#pragma unroll
-      for (int q = 0; q < GJ_MFQ; ++q)
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-          const cplx v = slab[(4 * kk + lq) * TH + 16 * (wv + 8 * q) + li];
-          fr[q][kk] = v.x;
-          fi[q][kk] = v.y;
-        }
-      __syncthreads();
-#pragma unroll
-      for (int m = 0; m < H; ++m) slab[m * TH + t] = pB[m];
-      __syncthreads();
-#pragma unroll
-      for (int q = 0; q < GJ_MFQ; ++q)
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-          const cplx v = slab[(4 * kk + lq) * TH + 16 * (wv + 8 * q) + li];
-          fr[q][4 + kk] = v.x;
-          fi[q][4 + kk] = v.y;
-        }
-    }
     __syncthreads();
     // interchanges and rank-w update of the other columns, WIN at a time; Pw row
     // m < wA is panel position k0 + m, row H + q position kB + q
@@ -630,90 +588,7 @@ gj_wide_kernel(int n, cplx* __restrict__ Aall, int lda, long long sA, cplx* __re
           a[t + j * lda] = a[src + j * lda];
         }
       __syncthreads();
-      if constexpr (MF) {
-        // this lane's elements of tile jt: rows 16 (wv + 8 q) + li, columns
-        // jt + lq + 4 r (loads clamped into the matrix and the window; stored
-        // only inside both); block rows start from zero.  The next tile's
-        // values are loaded while the current tile's products run.
-        int rowc[GJ_MFQ];
-        bool ld[GJ_MFQ], st[GJ_MFQ];
-#pragma unroll
-        for (int q = 0; q < GJ_MFQ; ++q) {
-          const int row = 16 * (wv + 8 * q) + li;
-          rowc[q] = min(row, n - 1);
-          st[q] = row < n;
-          ld[q] = row < n && !(row >= k0 && row < k0 + w);
-        }
-        auto colo = [&](int c) -> long long {
-          const int jj = c0 + min(c, cw - 1);
-          return (long long)((jj < k0) ? jj : jj + w) * lda;
-        };
-        cplx nx[GJ_MFQ][4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const long long o = colo(lq + 4 * r);
-#pragma unroll
-          for (int q = 0; q < GJ_MFQ; ++q) nx[q][r] = a[rowc[q] + o];
-        }
-#pragma unroll 1
-        for (int jt = 0; jt < cw; jt += 16) {
-          // three real products per complex one (Gauss): t1 = C_re + sum Pr Wr,
-          // t2 = sum Pi Wi, t3 = C_re + C_im + sum (Pr + Pi)(Wr + Wi); then
-          // C = (t1 - t2, t3 - t1 - t2)
-          gj_d4 t1[GJ_MFQ], t2[GJ_MFQ], t3[GJ_MFQ];
-#pragma unroll
-          for (int q = 0; q < GJ_MFQ; ++q)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const double cr = ld[q] ? nx[q][r].x : 0.0, ci = ld[q] ? nx[q][r].y : 0.0;
-              t1[q][r] = cr;
-              t2[q][r] = 0.0;
-              t3[q][r] = cr + ci;
-            }
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const long long o = colo(jt + 16 + lq + 4 * r);
-#pragma unroll
-            for (int q = 0; q < GJ_MFQ; ++q) nx[q][r] = a[rowc[q] + o];
-          }
-#pragma unroll
-          for (int kk = 0; kk < 8; ++kk) {
-            const cplx pv = Pw[4 * kk + lq][jt + li];
-            const double ps = pv.x + pv.y;
-#pragma unroll
-            for (int q = 0; q < GJ_MFQ; ++q) {
-              const double ws = fr[q][kk] + fi[q][kk];
-              t1[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(pv.x, fr[q][kk], t1[q], 0, 0, 0);
-              t2[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(pv.y, fi[q][kk], t2[q], 0, 0, 0);
-              t3[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(ps, ws, t3[q], 0, 0, 0);
-            }
-          }
-          gj_d4 dr[GJ_MFQ], di[GJ_MFQ];
-#pragma unroll
-          for (int q = 0; q < GJ_MFQ; ++q) {
-            dr[q] = t1[q] - t2[q];
-            di[q] = t3[q] - t1[q] - t2[q];
-          }
-          // the empty asm statements keep the products ahead of the guarded stores
-#pragma unroll
-          for (int q = 0; q < GJ_MFQ; ++q)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              double x = dr[q][r], y = di[q][r];
-              asm volatile("" : "+v"(x), "+v"(y));
-              dr[q][r] = x;
-              di[q][r] = y;
-            }
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const long long o = colo(jt + lq + 4 * r);
-            const bool cok = jt + lq + 4 * r < cw;
-#pragma unroll
-            for (int q = 0; q < GJ_MFQ; ++q)
-              if (st[q] && cok) a[rowc[q] + o] = cmk(dr[q][r], di[q][r]);
-          }
-        }
-      } else if (own) {
+      if (own) {
         // column c of the window, clamped into it: a group that runs past the
         // window loads, computes and stores its last column again (same value),
         // so loads and stores are unconditional; block rows start from zero
@@ -765,6 +640,567 @@ gj_wide_kernel(int n, cplx* __restrict__ Aall, int lda, long long sA, cplx* __re
   if (t == 0) {
     det[blockIdx.x] = d;
     info[blockIdx.x] = inf;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Gauss-Jordan inverse without interchanges, one thread per row.  A row stays where it
+// is and carries the label (position) the interchanges of ZGETRF would have given it;
+// pivot k is the first maximum of |Re| + |Im| in label order over the rows not yet used.
+// With p_k the row of pivot k, the reduced matrix B holds inverse(k, p_j) = B(p_k, j):
+// one permutation of rows and columns at the end replaces every interchange.
+//
+// A panel of 16 columns is reduced in registers, the pivot column always in pr[0]: a
+// step forms row - (f / pivot) r one place further down and appends the pivot column's
+// new value, so that 16 steps bring every column back to its place with no selection by
+// a run-time index.
+// ---------------------------------------------------------------------------
+
+typedef double gj_d4 __attribute__((ext_vector_type(4)));
+
+// 1/a: a scaled by a power of two, then conj(a) / |a|^2 with one division
+__device__ __forceinline__ cplx gj_cinv(cplx a) {
+  const int e = -ilogb(fmax(fabs(a.x), fabs(a.y)));
+  const double x = ldexp(a.x, e), y = ldexp(a.y, e);
+  const double r = ldexp(1.0 / fma(x, x, y * y), e);
+  return cmk(x * r, -y * r);
+}
+
+template <int CTRL, int RM>
+__device__ __forceinline__ unsigned gj_dpp_umax_step(unsigned v) {
+  return max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, RM, 0xf, false));
+}
+
+// maximum of v over lanes 0 .. W-1, every lane receiving it (row moves of
+// gj_wave_argmax_dpp; one instruction a step)
+template <int W>
+__device__ __forceinline__ unsigned gj_wave_umax(unsigned v) {
+  v = gj_dpp_umax_step<0x111, 0xf>(v);
+  v = gj_dpp_umax_step<0x112, 0xf>(v);
+  v = gj_dpp_umax_step<0x114, 0xf>(v);
+  if constexpr (W > 8) {
+    v = gj_dpp_umax_step<0x118, 0xf>(v);
+    v = gj_dpp_umax_step<0x142, 0xa>(v);
+    v = gj_dpp_umax_step<0x143, 0xc>(v);
+  }
+  return __builtin_amdgcn_readlane(v, W - 1);
+}
+
+__device__ __forceinline__ double gj_readlane(double v, int lane) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)(unsigned long long)b, lane);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+
+// The lane (of lanes 0 .. W-1) with the largest v, the smallest label on ties; -1 if no
+// v is positive.  Compared by its bits: the upper words decide nearly
+// always, the lower words and the labels are looked at only when they tie.  NaN is no
+// candidate.
+template <int W>
+__device__ __forceinline__ int gj_pick(double v, int lab) {
+  v = v > 0.0 ? v : 0.0;
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned hi = (unsigned)(b >> 32), lo = (unsigned)b;
+  const unsigned long long lanes = W == 64 ? ~0ull : (1ull << W) - 1;
+  const unsigned mh = gj_wave_umax<W>(hi);
+  unsigned long long m = __ballot(hi == mh) & lanes;
+  if ((m & (m - 1)) == 0 && mh != 0) return __ffsll((unsigned long long)m) - 1;
+  const unsigned ml = gj_wave_umax<W>(hi == mh ? lo : 0u);
+  if (mh == 0 && ml == 0) return -1;
+  m = __ballot(hi == mh && lo == ml) & lanes;
+  int best = __ffsll((unsigned long long)m) - 1;
+  int bl = __builtin_amdgcn_readlane(lab, best);
+  for (m &= m - 1; m; m &= m - 1) {
+    const int q = __ffsll((unsigned long long)m) - 1, l = __builtin_amdgcn_readlane(lab, q);
+    if (l < bl) { bl = l; best = q; }
+  }
+  return best;
+}
+
+__device__ __forceinline__ void gj_rotate(cplx (&pr)[16]) {
+  const cplx f = pr[0];
+#pragma unroll
+  for (int j = 0; j < 15; ++j) pr[j] = pr[j + 1];
+  pr[15] = f;
+}
+
+// One step with pivot row r (r[0] the pivot): pivrow marks the thread whose row it is
+template <typename R>
+__device__ __forceinline__ void gj_eliminate(cplx (&pr)[16], cplx pinv, bool pivrow, const R& r) {
+  cplx g = cmul(pr[0], pinv);
+  if (pivrow) {
+    g = cmk(-pinv.x, -pinv.y);
+#pragma unroll
+    for (int j = 1; j < 16; ++j) pr[j] = cmk(0.0, 0.0);
+  }
+#pragma unroll
+  for (int j = 1; j < 16; ++j) {
+    cplx v = pr[j];
+    cfms(v, g, r(j));
+    pr[j - 1] = v;
+  }
+  pr[15] = cmk(-g.x, -g.y);
+}
+
+// n <= 64: one wave, the matrix in LDS, the pivot row by readlane, so a matrix needs no
+// other wave.  Bound by the chain of n pivots (about 1.7 us each) and, with more matrices
+// than the LDS holds, by the waves per CU.  81 matrices of order 16, 40, 64: 20, 71, 130 us
+// (the 16-column kernel above: 40, 119, 223); 1944 of order 24, 40: 66, 214 us (150, 288).
+constexpr int GJ_SMALL = 64;
+__global__ void __launch_bounds__(64)
+gj_small_kernel(int n, cplx* __restrict__ Aall, int lda, long long sA, cplx* __restrict__ det,
+                int* __restrict__ info) {
+  extern __shared__ cplx gjm[];               // column c of the matrix at c * n
+  __shared__ int prow[GJ_SMALL + 16], pcol[GJ_SMALL];
+  const int t = threadIdx.x;
+  const bool own = t < n;
+  const int tr = min(t, n - 1);
+  cplx* a = Aall + (long long)blockIdx.x * sA;
+#pragma unroll 8
+  for (int c = 0; c < n; ++c) {
+    const cplx v = a[tr + (long long)c * lda];
+    if (own) gjm[c * n + t] = v;
+  }
+  prow[t] = 0;
+  if (t < 16) prow[GJ_SMALL + t] = 0;
+  __syncthreads();
+  cplx d = cmk(1.0, 0.0);
+  int inf = 0, lab = t;
+  bool used = !own;
+  for (int k0 = 0; k0 < n; k0 += 16) {
+    const int w = min(16, n - k0);
+    cplx pr[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) pr[j] = (j < w) ? gjm[(k0 + j) * n + tr] : cmk(0.0, 0.0);
+    bool inpan = false;
+    for (int mm = 0; mm < 16; ++mm) {
+      const int k = k0 + mm;
+      if (mm >= w) {
+        gj_rotate(pr);
+        continue;
+      }
+      const double v = used ? 0.0 : cabs1(pr[0]);
+      const cplx mine = gj_cinv(pr[0]);       // in the shadow of the search
+      int p = gj_pick<64>(v, lab);
+      const bool singular = p < 0;            // a vanishing (or NaN) column
+      if (singular) p = __ffsll((unsigned long long)__ballot(!used && lab == k)) - 1;
+      const int L = __builtin_amdgcn_readlane(lab, p);
+      if (lab == k) lab = L;
+      if (t == p) {
+        lab = k;
+        used = inpan = true;
+        prow[k] = p;
+        pcol[p] = k;
+      }
+      if (singular) {
+        if (inf == 0) inf = k + 1;
+        d = cmk(0.0, 0.0);
+        gj_rotate(pr);
+        continue;
+      }
+      const cplx piv = cmk(gj_readlane(pr[0].x, p), gj_readlane(pr[0].y, p));
+      if (L != k) d = cmk(-d.x, -d.y);
+      d = cmul(d, piv);
+      cplx r[16];
+#pragma unroll
+      for (int j = 1; j < 16; ++j) r[j] = cmk(gj_readlane(pr[j].x, p), gj_readlane(pr[j].y, p));
+      gj_eliminate(pr, cmk(gj_readlane(mine.x, p), gj_readlane(mine.y, p)), t == p,
+                   [&](int j) { return r[j]; });
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+      if (own && j < w) gjm[(k0 + j) * n + t] = pr[j];
+    // the other columns: c <- (0 in the panel's rows, c elsewhere) + W c[pivot rows];
+    // the wave reads a column before any lane writes it (columns past w have zero W)
+    for (int cc = 0; cc < n - w; ++cc) {
+      const int c = (cc < k0) ? cc : cc + w;
+      cplx acc = inpan ? cmk(0.0, 0.0) : gjm[c * n + tr];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) cfma(acc, pr[j], gjm[c * n + prow[k0 + j]]);
+      __builtin_amdgcn_wave_barrier();
+      if (own) gjm[c * n + t] = acc;
+      __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+  }
+  const int src = prow[tr];
+#pragma unroll 4
+  for (int c = 0; c < n; ++c) {
+    const cplx v = gjm[pcol[c] * n + src];
+    if (own) a[t + (long long)c * lda] = v;
+  }
+  if (t == 0) {
+    det[blockIdx.x] = d;
+    info[blockIdx.x] = inf;
+  }
+}
+
+// 64 < n <= 384: NW waves, panels of 32 columns as two halves A and B of 16.  A half
+// is reduced with one thread per row (its 16 columns in registers); everything else runs
+// on the matrix cores in 16 x 16 tiles of v_mfma_f64_16x16x4f64 computing C^T = P^T W^T,
+// wave v on the row blocks v + NW q, q < Q.  A
+// tile's C elements and the operand W of the next product have the same place in a wave
+// (row li, columns lq + 4 r), so the half A stays in registers as W while B's columns
+// receive its rank-16 update, B is reduced, and A receives B's; the panel is stored from
+// there, and the other columns take one rank-32 update, the next tile's values loaded
+// during the products.
+// One barrier per pivot: every wave leaves its best candidate's row and key in LDS, in
+// turn in two areas, and after the barrier each reads the winner's.
+// The update takes four real products per complex one, above order 256 (where the
+// products are the larger part) three (gj_tile_step3).
+// Bound by one CU per matrix: the pivot chain (1.5 to 2 us a pivot, of which the barrier,
+// the search, the reciprocal and 15 complex multiply-adds on the pivot row are about
+// equal parts) and the products (n = 336: 0.74 ms on one CU's matrix cores).
+// 121 matrices of order 80, 128, 140, 256: 156, 291, 467, 1170 us with random matrices
+// (16-column kernel: 380, 809, 1029, 3225); 225 of order 336 with a large diagonal, so
+// without interchanges: 2.93 ms (row interchanges, two barriers a pivot: 3.17).
+// Below order 129 four waves leave room for two matrices on a CU: 512 of order 128 take
+// 513 us (eight waves: 648), but a single round takes 10 % longer (128: 323 against 291).
+constexpr int GJM_NMAX = 384;
+
+struct __align__(16) GjKey { double v; int lab, row; };
+
+template <int NW, int WIN>
+struct GjShared {
+  cplx row[2][NW][16];        // candidate rows, the pivot first
+  cplx pinv[2][NW];           // 1 / pivot of each
+  GjKey key[2][NW];
+  cplx Pw[32][WIN + 16];      // panel source rows of a window (16 columns of slack)
+  cplx tab[16][17];
+  int prow[GJM_NMAX + 32], pcol[GJM_NMAX];
+};
+
+// reduces the 16 columns k0 .. k0 + w - 1 held in pr; a wave without rows only keeps the
+// barriers (it would take issue slots of its SIMD from one that has them)
+template <int NW, typename SH>
+__device__ __forceinline__ void gj_reduce(SH& S, cplx (&pr)[16], int n, int k0, int w, int t, bool& used,
+                                          int& lab, cplx& d, int& inf) {
+  const int lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
+  if (64 * wv >= n) {
+    for (int mm = 0; mm < w; ++mm) __syncthreads();
+    return;
+  }
+#pragma unroll 1
+  for (int mm = 0; mm < 16; ++mm) {
+    const int k = k0 + mm, buf = mm & 1;
+    if (mm >= w) {
+      gj_rotate(pr);
+      continue;
+    }
+    const double v = used ? 0.0 : cabs1(pr[0]);
+    const cplx mine = gj_cinv(pr[0]);         // in the shadow of the search
+    const int pl = gj_pick<64>(v, lab);
+    if (lane == max(pl, 0)) {
+      S.key[buf][wv] = GjKey{pl < 0 ? 0.0 : v, lab, t};
+      S.pinv[buf][wv] = mine;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) S.row[buf][wv][j] = pr[j];
+    }
+    __syncthreads();
+    // lane q of every wave takes wave q's candidate
+    const GjKey kq = S.key[buf][lane & (NW - 1)];
+    const int wq = gj_pick<NW>(kq.v, kq.lab);
+    if (wq < 0) {                             // a vanishing (or NaN) column
+      if (inf == 0) inf = k + 1;
+      d = cmk(0.0, 0.0);
+      if (!used && lab == k) {
+        used = true;
+        S.prow[k] = t;
+        S.pcol[t] = k;
+      }
+      gj_rotate(pr);
+      continue;
+    }
+    const int p = __builtin_amdgcn_readlane(kq.row, wq), L = __builtin_amdgcn_readlane(kq.lab, wq);
+    const cplx* r = S.row[buf][wq];
+    const cplx pinv = S.pinv[buf][wq];
+    d = cmul(d, (L != k) ? cmk(-r[0].x, -r[0].y) : r[0]);
+    if (lab == k) lab = L;
+    if (t == p) {
+      lab = k;
+      used = true;
+      S.prow[k] = p;
+      S.pcol[p] = k;
+    }
+    gj_eliminate(pr, pinv, t == p, [&](int j) { return r[j]; });
+  }
+}
+
+// C += P W, four k: the four real products of a complex one
+__device__ __forceinline__ void gj_tile_step(cplx pv, double fr, double fi, gj_d4& cr, gj_d4& ci) {
+  cr = __builtin_amdgcn_mfma_f64_16x16x4f64(pv.x, fr, cr, 0, 0, 0);
+  ci = __builtin_amdgcn_mfma_f64_16x16x4f64(pv.y, fr, ci, 0, 0, 0);
+  cr = __builtin_amdgcn_mfma_f64_16x16x4f64(-pv.y, fi, cr, 0, 0, 0);
+  ci = __builtin_amdgcn_mfma_f64_16x16x4f64(pv.x, fi, ci, 0, 0, 0);
+}
+
+// the same with three: t1 = C_re + sum Pr Wr, t2 = sum Pi Wi, t3 = C_re + C_im +
+// sum (Pr + Pi)(Wr + Wi); C = (t1 - t2, t3 - t1 - t2)
+__device__ __forceinline__ void gj_tile_step3(cplx pv, double fr, double fi, gj_d4& t1, gj_d4& t2, gj_d4& t3) {
+  t1 = __builtin_amdgcn_mfma_f64_16x16x4f64(pv.x, fr, t1, 0, 0, 0);
+  t2 = __builtin_amdgcn_mfma_f64_16x16x4f64(pv.y, fi, t2, 0, 0, 0);
+  t3 = __builtin_amdgcn_mfma_f64_16x16x4f64(pv.x + pv.y, fr + fi, t3, 0, 0, 0);
+}
+
+template <int NW, int Q, int WIN>
+__global__ void __launch_bounds__(64 * NW, 2)
+gj_mfma_kernel(int n, cplx* __restrict__ Aall, int lda, long long sA, cplx* __restrict__ det,
+               int* __restrict__ info) {
+  constexpr bool G3 = Q > 2;   // n > 256: three products
+  constexpr int H = 16, NR = 16 * NW * Q;   // rows the tiles cover
+  constexpr int TH = 64 * NW;
+  __shared__ GjShared<NW, WIN> S;
+  const int t = threadIdx.x, lane = t & 63, li = lane & 15, lq = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int tr = min(t, n - 1);
+  cplx* a = Aall + (long long)blockIdx.x * sA;
+  cplx* slab = &S.Pw[0][0];                     // [column][row], NR rows: a half on its way
+  cplx d = cmk(1.0, 0.0);
+  int inf = 0, lab = t;
+  bool used = t >= n;
+  for (int i = t; i < GJM_NMAX; i += TH) S.pcol[i] = -1;
+  for (int i = t; i < GJM_NMAX + 32; i += TH) S.prow[i] = 0;
+  if (t < 2 * NW) S.key[t / NW][t % NW] = GjKey{0.0, 64 * NW, 0};
+  int rowc[Q];
+  bool st[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const int row = 16 * (wv + NW * q) + li;
+    rowc[q] = min(row, n - 1);
+    st[q] = row < n;
+  }
+  for (int k0 = 0; k0 < n; k0 += 2 * H) {
+    const int w = min(2 * H, n - k0), wA = min(H, w), wB = w - wA, kB = k0 + H;
+    cplx pr[H];
+    double fr[Q][8], fi[Q][8];                  // W(row, 4 kk + lq) of the wave's row blocks
+#pragma unroll
+    for (int m = 0; m < H; ++m) {
+      const cplx v = a[tr + (long long)min(k0 + m, n - 1) * lda];
+      pr[m] = (t < n && m < wA) ? v : cmk(0.0, 0.0);
+    }
+    gj_reduce<NW>(S, pr, n, k0, wA, t, used, lab, d, inf);
+    __syncthreads();                            // window area free, prow of the half
+    auto to_operand = [&](int o) {
+      if (t < NR)
+#pragma unroll
+        for (int m = 0; m < H; ++m) slab[m * NR + t] = pr[m];
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+          const cplx v = slab[(4 * kk + lq) * NR + 16 * (wv + NW * q) + li];
+          fr[q][o + kk] = v.x;
+          fi[q][o + kk] = v.y;
+        }
+    };
+    if (wB > 0) {
+      // B's columns: (0 in A's rows, c elsewhere) + W_A c[A's rows]
+      cplx nx[Q][4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const long long o = (long long)min(kB + lq + 4 * r, n - 1) * lda;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) nx[q][r] = a[rowc[q] + o];
+      }
+      if (t < H * H)   // TH >= 256
+        S.tab[t % H][t / H] = (t / H < wB) ? a[S.prow[k0 + t % H] + (long long)(kB + t / H) * lda]
+                                           : cmk(0.0, 0.0);
+      to_operand(0);
+      __syncthreads();                          // slab read, tab written
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const bool keep = st[q] && !(S.pcol[rowc[q]] >= k0);
+        gj_d4 cr, ci;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const bool in = keep && lq + 4 * r < wB;
+          cr[r] = in ? nx[q][r].x : 0.0;
+          ci[r] = in ? nx[q][r].y : 0.0;
+        }
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) gj_tile_step(S.tab[4 * kk + lq][li], fr[q][kk], fi[q][kk], cr, ci);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          slab[(lq + 4 * r) * NR + 16 * (wv + NW * q) + li] = cmk(cr[r], ci[r]);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int m = 0; m < H; ++m) pr[m] = slab[m * NR + min(t, NR - 1)];
+      if (t >= n)
+#pragma unroll
+        for (int m = 0; m < H; ++m) pr[m] = cmk(0.0, 0.0);
+      gj_reduce<NW>(S, pr, n, kB, wB, t, used, lab, d, inf);
+      __syncthreads();
+      to_operand(4);
+      // the A half: (0 in B's rows, itself elsewhere) + W_B A[B's rows]
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const int j = st[q] ? S.pcol[rowc[q]] - kB : -1;
+        if (j >= 0)
+#pragma unroll
+          for (int kk = 0; kk < 4; ++kk) {
+            S.tab[j][4 * kk + lq] = cmk(fr[q][kk], fi[q][kk]);
+            fr[q][kk] = 0.0;
+            fi[q][kk] = 0.0;
+          }
+      }
+      if (t < H)
+        for (int j = wB; j < H; ++j) S.tab[j][t] = cmk(0.0, 0.0);
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        gj_d4 cr, ci;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          cr[r] = fr[q][r];
+          ci[r] = fi[q][r];
+        }
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk)
+          gj_tile_step(S.tab[4 * kk + lq][li], fr[q][4 + kk], fi[q][4 + kk], cr, ci);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          fr[q][r] = cr[r];
+          fi[q][r] = ci[r];
+        }
+      }
+    } else {
+      to_operand(0);
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int kk = 4; kk < 8; ++kk) fr[q][kk] = fi[q][kk] = 0.0;
+    }
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk)
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+        if (st[q] && 4 * kk + lq < w)
+          a[rowc[q] + (long long)(k0 + 4 * kk + lq) * lda] = cmk(fr[q][kk], fi[q][kk]);
+    const int nrest = n - w;
+    bool keep[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) keep[q] = st[q] && !(S.pcol[rowc[q]] >= k0);
+    // the other columns in equal windows of whole tiles
+    const int nwin = (nrest + WIN - 1) / WIN;
+    const int win = nwin ? ((nrest + nwin - 1) / nwin + 15) / 16 * 16 : 16;
+    for (int c0 = 0; c0 < nrest; c0 += win) {
+      const int cw = min(win, nrest - c0);
+      __syncthreads();
+      // source rows of the window (zero past the panel width); the 16 slack columns
+      // repeat the last one
+      for (int e = t; e < 2 * H * (cw + 16); e += TH) {
+        const int m2 = e % (2 * H), c = e / (2 * H);
+        const int jj = c0 + min(c, cw - 1);
+        const cplx v = a[S.prow[k0 + m2] + (long long)((jj < k0) ? jj : jj + w) * lda];
+        S.Pw[m2][c] = (m2 < w) ? v : cmk(0.0, 0.0);
+      }
+      __syncthreads();
+      if (16 * wv >= n) continue;
+      // this lane's elements of tile jt: rows rowc, columns jt + lq + 4 r (clamped into
+      // the window; stored only inside it)
+      auto colo = [&](int c) -> long long {
+        const int jj = c0 + min(c, cw - 1);
+        return (long long)((jj < k0) ? jj : jj + w) * lda;
+      };
+      cplx nx[Q][4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const long long o = colo(lq + 4 * r);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) nx[q][r] = a[rowc[q] + o];
+      }
+#pragma unroll 1
+      for (int jt = 0; jt < cw; jt += 16) {
+        gj_d4 dr[Q], di[Q], t3[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const double cr = keep[q] ? nx[q][r].x : 0.0, ci = keep[q] ? nx[q][r].y : 0.0;
+            dr[q][r] = cr;
+            di[q][r] = G3 ? 0.0 : ci;
+            if constexpr (G3) t3[q][r] = cr + ci;
+          }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const long long o = colo(jt + 16 + lq + 4 * r);
+#pragma unroll
+          for (int q = 0; q < Q; ++q) nx[q][r] = a[rowc[q] + o];
+        }
+#pragma unroll
+        for (int kk = 0; kk < 8; ++kk) {
+          const cplx pv = S.Pw[4 * kk + lq][jt + li];
+#pragma unroll
+          for (int q = 0; q < Q; ++q) {
+            if constexpr (G3)
+              gj_tile_step3(pv, fr[q][kk], fi[q][kk], dr[q], di[q], t3[q]);
+            else
+              gj_tile_step(pv, fr[q][kk], fi[q][kk], dr[q], di[q]);
+          }
+        }
+        if constexpr (G3)
+#pragma unroll
+          for (int q = 0; q < Q; ++q) {
+            t3[q] = t3[q] - dr[q] - di[q];
+            dr[q] = dr[q] - di[q];
+            di[q] = t3[q];
+          }
+        // the empty asm statements keep the products ahead of the guarded stores
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            double x = dr[q][r], y = di[q][r];
+            asm volatile("" : "+v"(x), "+v"(y));
+            dr[q][r] = x;
+            di[q][r] = y;
+          }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const long long o = colo(jt + lq + 4 * r);
+          const bool cok = jt + lq + 4 * r < cw;
+#pragma unroll
+          for (int q = 0; q < Q; ++q)
+            if (st[q] && cok) a[rowc[q] + o] = cmk(dr[q][r], di[q][r]);
+        }
+      }
+    }
+    __syncthreads();   // the next panel's loads follow every store
+  }
+  if (t == 0) {
+    det[blockIdx.x] = d;
+    info[blockIdx.x] = inf;
+  }
+  // inverse(i, j) = B(prow[i], pcol[j]): columns within blocks of rows, then rows within
+  // blocks of columns, through the window area
+  cplx* buf = &S.Pw[0][0];
+  constexpr int CAP = 32 * (WIN + 16);
+  const int rb = min(64, CAP / n / 8 * 8);
+  for (int r0 = 0; r0 < n; r0 += rb) {
+    const int rows = min(rb, n - r0);
+    for (int e = t; e < rb * n; e += TH) {
+      const int r = e % rb, c = e / rb;
+      if (r < rows) buf[e] = a[r0 + r + (long long)c * lda];
+    }
+    __syncthreads();
+    for (int e = t; e < rb * n; e += TH) {
+      const int r = e % rb, c = e / rb;
+      if (r < rows) a[r0 + r + (long long)c * lda] = buf[r + S.pcol[c] * rb];
+    }
+    __syncthreads();
+  }
+  const int cb = CAP / n;
+  for (int c0 = 0; c0 < n; c0 += cb) {
+    const int cols_ = min(cb, n - c0);
+    for (int e = t; e < cols_ * n; e += TH) buf[e] = a[e % n + (long long)(c0 + e / n) * lda];
+    __syncthreads();
+    for (int e = t; e < cols_ * n; e += TH)
+      a[e % n + (long long)(c0 + e / n) * lda] = buf[S.prow[e % n] + e / n * n];
+    __syncthreads();
   }
 }
 
@@ -1268,12 +1704,10 @@ int batched_inverse(hipStream_t s, int n, cplx* A, int lda, long long sA, int ba
                     int* info, int* perm) {
   if (n <= 0 || batch <= 0) return TG_OK;
   if (n <= GJ_THREADS) {
-    // one thread per row in the smallest workgroup that holds the rows (the
-    // LDS window shrinks with it, so small matrices share a CU); above 256 rows
-    // the 32-column panels of gj_wide_kernel.  TG_GJ=1: 16-column panels at
-    // every order; TG_GJ=2: 16-column panels with two threads per row (the
-    // second mirrors the panel reduction and takes half of the column updates),
-    // n <= 384
+    // TG_GJ=1: 16-column panels at every order; TG_GJ=2: 16-column panels with two
+    // threads per row (the second mirrors the panel reduction and takes half of the
+    // column updates), n <= 384
+    constexpr int CUS = 256;
     static const int rp = [] {
       const char* e = std::getenv("TG_GJ");
       return e ? std::atoi(e) : 0;
@@ -1283,15 +1717,23 @@ int batched_inverse(hipStream_t s, int n, cplx* A, int lda, long long sA, int ba
                      lda, sA, det, info, perm)
     if (rp == 2 && n <= 384)
       TG_GJ_LAUNCH(2, 384, GJ_WIN);
-    else if (rp == 4 && n > 256 && n <= 384)
-      hipLaunchKernelGGL((gj_wide_kernel<384, 256, 4, false>), dim3(batch), dim3(384), 0, s, n, A,
-                         lda, sA, det, info, perm);
-    else if (rp != 1 && n > 256 && n <= 384)
-      hipLaunchKernelGGL((gj_wide_kernel<512, 256, 16, true>), dim3(batch), dim3(512), 0, s, n, A,
-                         lda, sA, det, info, perm);
-    else if (rp != 1 && n > 384)
-      hipLaunchKernelGGL((gj_wide_kernel<512, 256, 4, false>), dim3(batch), dim3(512), 0, s, n, A,
-                         lda, sA, det, info, perm);
+    // the LDS of a CU holds three matrices of order 48 or two of order 64: past two
+    // rounds of the latter the 16-column kernel, which shares a CU among more waves, is
+    // ahead (order 64, 400 matrices: 142 against 242 us; 1296: 418 against 322)
+    else if (rp != 1 && (n <= 48 || (n <= GJ_SMALL && batch <= 2 * CUS)))
+      hipLaunchKernelGGL(gj_small_kernel, dim3(batch), dim3(64), sizeof(cplx) * n * n, s, n, A, lda, sA,
+                         det, info);
+    else if (rp != 1 && n > 64 && n <= 128 && batch > CUS)
+      hipLaunchKernelGGL((gj_mfma_kernel<4, 2, 96>), dim3(batch), dim3(256), 0, s, n, A, lda, sA, det, info);
+    else if (rp != 1 && n > 64 && n <= 128)
+      hipLaunchKernelGGL((gj_mfma_kernel<8, 1, 96>), dim3(batch), dim3(512), 0, s, n, A, lda, sA, det, info);
+    else if (rp != 1 && n > 64 && n <= 256)
+      hipLaunchKernelGGL((gj_mfma_kernel<8, 2, 256>), dim3(batch), dim3(512), 0, s, n, A, lda, sA, det, info);
+    else if (rp != 1 && n > 64 && n <= GJM_NMAX)
+      hipLaunchKernelGGL((gj_mfma_kernel<8, 3, 256>), dim3(batch), dim3(512), 0, s, n, A, lda, sA, det, info);
+    else if (rp != 1 && n > GJM_NMAX)
+      hipLaunchKernelGGL((gj_wide_kernel<512, 256, 4>), dim3(batch), dim3(512), 0, s, n, A, lda, sA, det,
+                         info, perm);
     else if (n <= 64)
       TG_GJ_LAUNCH(1, 64, 64);
     else if (n <= 128)
