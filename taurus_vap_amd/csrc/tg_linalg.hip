@@ -963,6 +963,7 @@ gj_mfma_kernel(int n, cplx* __restrict__ Aall, int lda, long long sA, cplx* __re
   for (int i = t; i < GJM_NMAX; i += TH) S.pcol[i] = -1;
   for (int i = t; i < GJM_NMAX + 32; i += TH) S.prow[i] = 0;
   if (t < 2 * NW) S.key[t / NW][t % NW] = GjKey{0.0, 64 * NW, 0};
+  __syncthreads();   // the keys of waves without rows stay as set here, the others follow
   int rowc[Q];
   bool st[Q];
 #pragma unroll
