@@ -35,6 +35,8 @@
 #include <algorithm>
 #include <atomic>
 #include <map>
+#include <new>
+#include <system_error>
 #include <thread>
 #include <tuple>
 
@@ -527,10 +529,8 @@ Reduced reduce_class(const tg_ctx* c, bool pp, const std::vector<int>& el, const
   return R;
 }
 
-}  // namespace
-
-int contraction_build(tg_ctx* c, int64_t ntb, const int16_t* abcd, const void* H2, int h2_bytes,
-                      const int8_t* trperm) {
+int build_blocks(tg_ctx* c, int64_t ntb, const int16_t* abcd, const void* H2, int h2_bytes,
+                 const int8_t* trperm) {
   const int n = c->n;
   // per channel: the classes, the class and place of every element, the full matrices
   struct Full {
@@ -626,19 +626,29 @@ int contraction_build(tg_ctx* c, int64_t ntb, const int16_t* abcd, const void* H
     const int nc = (int)f.el.size();
     std::vector<Reduced> red(nc);
     std::atomic<int> next(0);
+    std::atomic<bool> nomem(false);
     auto work = [&] {
-      for (int g; (g = next.fetch_add(1)) < nc;) {
-        if (c->w_fp32)
-          for (double& v : f.B[g]) v = (double)(float)v;
-        red[g] = reduce_class(c, q == 1, f.el[g], f.B[g]);
-        std::vector<double>().swap(f.B[g]);
+      try {
+        for (int g; (g = next.fetch_add(1)) < nc;) {
+          if (c->w_fp32)
+            for (double& v : f.B[g]) v = (double)(float)v;
+          red[g] = reduce_class(c, q == 1, f.el[g], f.B[g]);
+          std::vector<double>().swap(f.B[g]);
+        }
+      } catch (const std::bad_alloc&) {      // nothing may leave a thread
+        nomem = true;
       }
     };
     const int nt = std::max(1, std::min({8, (int)std::thread::hardware_concurrency(), nc}));
     std::vector<std::thread> pool;
-    for (int k = 1; k < nt; ++k) pool.emplace_back(work);
+    pool.reserve(nt);
+    try {
+      for (int k = 1; k < nt; ++k) pool.emplace_back(work);
+    } catch (const std::system_error&) {     // the threads there are take the work
+    }
     work();
     for (std::thread& th : pool) th.join();
+    if (nomem) throw std::bad_alloc();
 
     std::vector<GroupDesc> groups;
     std::vector<Orbit> orb;
@@ -704,6 +714,18 @@ int contraction_build(tg_ctx* c, int64_t ntb, const int16_t* abcd, const void* H
     TG_TRY(up(ch.d_tile_n0, tn.data(), sizeof(int) * tn.size()));
   }
   return TG_OK;
+}
+
+}  // namespace
+
+int contraction_build(tg_ctx* c, int64_t ntb, const int16_t* abcd, const void* H2, int h2_bytes,
+                      const int8_t* trperm) {
+  try {
+    return build_blocks(c, ntb, abcd, H2, h2_bytes, trperm);
+  } catch (const std::bad_alloc&) {
+    tg_set_error("tg_init: out of host memory for the interaction blocks");
+    return TG_E_NOMEM;
+  }
 }
 
 int contraction_run(tg_ctx* c, int na, const cplx* rho, const cplx* kLR, const cplx* kRL,
