@@ -52,6 +52,12 @@ __device__ inline double epi(double alpha, double acc, double beta, const double
   if (use_beta) r = fma(beta, *cptr, r);
   return r;
 }
+__device__ inline cplx extra(const GemmEpi& e, cplx v, const double* add) {
+  if (e.conj) v = cconj(v);
+  if (add) v.x += *add;
+  return v;
+}
+__device__ inline double extra(const GemmEpi&, double v, const double*) { return v; }
 
 // One 64x64 tile: C(m0:m0+64, n0:n0+64) of a column-major M x N result.
 template <typename TA, typename TB, typename TC, int OPA, int OPB>
@@ -60,6 +66,7 @@ __device__ inline void gemm_tile(int M, int N, int K, typename Scal<TC>::type al
                                  const TB* __restrict__ B, int ldb,
                                  typename Scal<TC>::type beta, bool use_beta,
                                  TC* __restrict__ C, int ldc, int m0, int n0,
+                                 const GemmEpi& ep, const double* __restrict__ add,
                                  typename Stage<TA>::type (*As)[BM + 1],
                                  typename Stage<TB>::type (*Bs)[BN + 1]) {
   typedef typename Stage<TA>::type SA;
@@ -142,7 +149,8 @@ __device__ inline void gemm_tile(int M, int N, int K, typename Scal<TC>::type al
       const int gi = m0 + tx + 16 * i;
       if (gi >= M) continue;
       TC* cp = C + gi + (long long)gj * ldc;
-      *cp = epi(alpha, acc[i][j], beta, cp, use_beta);
+      *cp = extra(ep, epi(alpha, acc[i][j], beta, cp, use_beta),
+                  add ? add + gi + (long long)gj * ldc : nullptr);
     }
   }
 }
@@ -153,21 +161,22 @@ gemm_batched_kernel(int M, int N, int K, typename Scal<TC>::type alpha,
                     const TA* __restrict__ A, int lda, long long sA,
                     const TB* __restrict__ B, int ldb, long long sB,
                     typename Scal<TC>::type beta, int use_beta,
-                    TC* __restrict__ C, int ldc, long long sC, int divA, int divB) {
+                    TC* __restrict__ C, int ldc, long long sC, int divA, int divB, GemmEpi ep) {
   __shared__ typename Stage<TA>::type As[BK][BM + 1];
   __shared__ typename Stage<TB>::type Bs[BK][BN + 1];
   const long long b = blockIdx.z;
   gemm_tile<TA, TB, TC, OPA, OPB>(M, N, K, alpha, A + (b / divA) * sA, lda, B + (b / divB) * sB,
                                   ldb, beta,
                                   use_beta != 0, C + b * sC, ldc, blockIdx.x * BM,
-                                  blockIdx.y * BN, As, Bs);
+                                  blockIdx.y * BN, ep,
+                                  ep.add ? ep.add + (b / ep.divAdd) * ep.sAdd : nullptr, As, Bs);
 }
 
 template <typename TA, typename TB, typename TC, int OPA, int OPB>
 int launch(hipStream_t s, int M, int N, int K, typename Scal<TC>::type alpha, const TA* A,
            int lda, long long sA, const TB* B, int ldb, long long sB,
            typename Scal<TC>::type beta, int use_beta, TC* C, int ldc, long long sC, int batch,
-           int divA, int divB) {
+           int divA, int divB, const GemmEpi& ep) {
   if (M <= 0 || N <= 0 || batch <= 0) return TG_OK;
   if (batch > 65535) {
     tg_set_error("gemm: batch too large");
@@ -175,7 +184,8 @@ int launch(hipStream_t s, int M, int N, int K, typename Scal<TC>::type alpha, co
   }
   dim3 grid((M + BM - 1) / BM, (N + BN - 1) / BN, batch);
   hipLaunchKernelGGL((gemm_batched_kernel<TA, TB, TC, OPA, OPB>), grid, dim3(NT), 0, s, M, N,
-                     K, alpha, A, lda, sA, B, ldb, sB, beta, use_beta, C, ldc, sC, divA, divB);
+                     K, alpha, A, lda, sA, B, ldb, sB, beta, use_beta, C, ldc, sC, divA, divB,
+                     ep);
   TG_HIP(hipGetLastError());
   return TG_OK;
 }
@@ -184,11 +194,11 @@ template <typename TA, typename TB, typename TC>
 int dispatch(hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K,
              typename Scal<TC>::type alpha, const TA* A, int lda, long long sA, const TB* B,
              int ldb, long long sB, typename Scal<TC>::type beta, int use_beta, TC* C, int ldc,
-             long long sC, int batch, int divA, int divB) {
+             long long sC, int batch, int divA, int divB, const GemmEpi& ep = GemmEpi()) {
 #define TG_CASE(OA, OB)                                                                   \
   if (opa == OA && opb == OB)                                                             \
     return launch<TA, TB, TC, OA, OB>(s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta,    \
-                                      use_beta, C, ldc, sC, batch, divA, divB);
+                                      use_beta, C, ldc, sC, batch, divA, divB, ep);
   TG_CASE(OP_N, OP_N) TG_CASE(OP_N, OP_T) TG_CASE(OP_N, OP_C)
   TG_CASE(OP_T, OP_N) TG_CASE(OP_T, OP_T) TG_CASE(OP_T, OP_C)
   TG_CASE(OP_C, OP_N) TG_CASE(OP_C, OP_T) TG_CASE(OP_C, OP_C)
@@ -230,7 +240,9 @@ struct GemmKey {
     return false;
   }
 };
-enum { K_ZZ = 0, K_DZ = 1, K_ZD = 2, K_GROUPED = 3 };
+enum { K_ZZ = 0, K_DZ = 1, K_ZD = 2, K_GROUPED = 3, K_SKEW = 4 };
+// (K_SKEW added for a skew product, which takes the full product's tile unless it was
+// timed itself)
 std::map<GemmKey, int>& choices() {
   static std::map<GemmKey, int> m;
   return m;
@@ -239,6 +251,8 @@ int variant_for(const GemmKey& k) {
   const int forced = (k.kind == K_GROUPED) ? sel().grouped : sel().variant;
   if (forced >= 0) return forced;
   auto it = choices().find(k);
+  if (it == choices().end() && k.kind >= K_SKEW)
+    it = choices().find(GemmKey{k.kind - K_SKEW, k.opa, k.opb, k.M, k.N, k.K, k.batch});
   return it == choices().end() ? 0 : it->second;
 }
 
@@ -289,33 +303,39 @@ int gemm_tuned_variant(int kind, TgOp opa, TgOp opb, int M, int N, int K, int ba
 
 int gemm_tune_zz(hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, const cplx* A, int lda,
                  long long sA, const cplx* B, int ldb, long long sB, cplx* C, int ldc,
-                 long long sC, int batch) {
-  const GemmKey key{K_ZZ, (int)opa, (int)opb, M, N, K, batch};
+                 long long sC, int batch, int skew) {
+  const GemmKey key{K_ZZ + K_SKEW * skew, (int)opa, (int)opb, M, N, K, batch};
   return tune(s, key, TG_MFMA_VARIANTS, [&](int v) {
+    GemmEpi epi;
+    epi.skew = skew;
     return mfma_gemm_zz(v, s, opa, opb, M, N, K, cmk(1, 0), A, lda, sA, B, ldb, sB, cmk(0, 0), 0,
-                        C, ldc, sC, batch);
+                        C, ldc, sC, batch, 1, 1, epi);
   });
 }
 
 int gemm_tune_dz(hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, const double* A,
                  int lda, long long sA, const cplx* B, int ldb, long long sB, cplx* C, int ldc,
-                 long long sC, int batch) {
+                 long long sC, int batch, int skew) {
   if (opa == OP_C) opa = OP_T;
-  const GemmKey key{K_DZ, (int)opa, (int)opb, M, N, K, batch};
+  const GemmKey key{K_DZ + K_SKEW * skew, (int)opa, (int)opb, M, N, K, batch};
   return tune(s, key, TG_MFMA_VARIANTS, [&](int v) {
+    GemmEpi epi;
+    epi.skew = skew;
     return mfma_gemm_dz(v, s, opa, opb, M, N, K, cmk(1, 0), A, lda, sA, B, ldb, sB, cmk(0, 0), 0,
-                        C, ldc, sC, batch);
+                        C, ldc, sC, batch, 1, 1, epi);
   });
 }
 
 int gemm_tune_zd(hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, const cplx* A, int lda,
                  long long sA, const double* B, int ldb, long long sB, cplx* C, int ldc,
-                 long long sC, int batch) {
+                 long long sC, int batch, int skew) {
   if (opb == OP_C) opb = OP_T;
-  const GemmKey key{K_ZD, (int)opa, (int)opb, M, N, K, batch};
+  const GemmKey key{K_ZD + K_SKEW * skew, (int)opa, (int)opb, M, N, K, batch};
   return tune(s, key, TG_MFMA_VARIANTS, [&](int v) {
+    GemmEpi epi;
+    epi.skew = skew;
     return mfma_gemm_zd(v, s, opa, opb, M, N, K, cmk(1, 0), A, lda, sA, B, ldb, sB, cmk(0, 0), 0,
-                        C, ldc, sC, batch);
+                        C, ldc, sC, batch, 1, 1, epi);
   });
 }
 
@@ -337,42 +357,44 @@ int gemm_tune_grouped(hipStream_t s, int M, const cplx* X, cplx* C, int ld, cons
 int gemm_zz(hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, cplx alpha,
             const cplx* A, int lda, long long sA, const cplx* B, int ldb, long long sB,
             cplx beta, cplx* C, int ldc, long long sC, int batch, int divA, int divB,
-            int variant) {
+            int variant, GemmEpi epi) {
   if (M <= 0 || N <= 0 || batch <= 0) return TG_OK;
   if (sel().mfma)
     return mfma_gemm_zz(variant >= 0 ? variant
-                                     : variant_for(GemmKey{K_ZZ, (int)opa, (int)opb, M, N, K, batch}),
+                                     : variant_for(GemmKey{K_ZZ + K_SKEW * epi.skew, (int)opa, (int)opb, M, N, K, batch}),
                         s, opa,
                         opb, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta,
-                        !is_zero(beta), C, ldc, sC, batch, divA, divB);
+                        !is_zero(beta), C, ldc, sC, batch, divA, divB, epi);
   return dispatch<cplx, cplx, cplx>(s, opa, opb, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta,
-                                    !is_zero(beta), C, ldc, sC, batch, divA, divB);
+                                    !is_zero(beta), C, ldc, sC, batch, divA, divB, epi);
 }
 
 int gemm_dz(hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, cplx alpha,
             const double* A, int lda, long long sA, const cplx* B, int ldb, long long sB,
-            cplx beta, cplx* C, int ldc, long long sC, int batch, int divA, int divB) {
+            cplx beta, cplx* C, int ldc, long long sC, int batch, int divA, int divB,
+            GemmEpi epi) {
   if (M <= 0 || N <= 0 || batch <= 0) return TG_OK;
   if (opa == OP_C) opa = OP_T;
   if (sel().mfma)
-    return mfma_gemm_dz(variant_for(GemmKey{K_DZ, (int)opa, (int)opb, M, N, K, batch}), s, opa,
+    return mfma_gemm_dz(variant_for(GemmKey{K_DZ + K_SKEW * epi.skew, (int)opa, (int)opb, M, N, K, batch}), s, opa,
                         opb, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta,
-                        !is_zero(beta), C, ldc, sC, batch, divA, divB);
+                        !is_zero(beta), C, ldc, sC, batch, divA, divB, epi);
   return dispatch<double, cplx, cplx>(s, opa, opb, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta,
-                                      !is_zero(beta), C, ldc, sC, batch, divA, divB);
+                                      !is_zero(beta), C, ldc, sC, batch, divA, divB, epi);
 }
 
 int gemm_zd(hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, cplx alpha,
             const cplx* A, int lda, long long sA, const double* B, int ldb, long long sB,
-            cplx beta, cplx* C, int ldc, long long sC, int batch, int divA, int divB) {
+            cplx beta, cplx* C, int ldc, long long sC, int batch, int divA, int divB,
+            GemmEpi epi) {
   if (M <= 0 || N <= 0 || batch <= 0) return TG_OK;
   if (opb == OP_C) opb = OP_T;
   if (sel().mfma)
-    return mfma_gemm_zd(variant_for(GemmKey{K_ZD, (int)opa, (int)opb, M, N, K, batch}), s, opa,
+    return mfma_gemm_zd(variant_for(GemmKey{K_ZD + K_SKEW * epi.skew, (int)opa, (int)opb, M, N, K, batch}), s, opa,
                         opb, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta,
-                        !is_zero(beta), C, ldc, sC, batch, divA, divB);
+                        !is_zero(beta), C, ldc, sC, batch, divA, divB, epi);
   return dispatch<cplx, double, cplx>(s, opa, opb, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta,
-                                      !is_zero(beta), C, ldc, sC, batch, divA, divB);
+                                      !is_zero(beta), C, ldc, sC, batch, divA, divB, epi);
 }
 
 int gemm_dd(hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, double alpha,

@@ -89,22 +89,32 @@ struct DevBuf {
 // ---------------------------------------------------------------------------
 enum TgOp { OP_N = 0, OP_T = 1, OP_C = 2 };
 
+// What the complex products do as they store C, in place of passes of their own.
+struct GemmEpi {
+  int skew = 0;                  // C is skew: tiles on and below the diagonal, -C^T above
+                                 // it, zero on it (M == N, beta = 0)
+  int conj = 0;                  // conj(C)
+  const double* add = nullptr;   // + a real matrix, element b's at add + (b / divAdd) * sAdd
+  long long sAdd = 0;            // (leading dimension ldc)
+  int divAdd = 1;
+};
+
 // complex = complex x complex
 // variant >= 0 forces a matrix-core tile variant (tg_mfma.h) instead of the tuned one
 int gemm_zz(hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, cplx alpha,
             const cplx* A, int lda, long long sA, const cplx* B, int ldb, long long sB,
             cplx beta, cplx* C, int ldc, long long sC, int batch, int divA = 1,
-            int divB = 1, int variant = -1);
+            int divB = 1, int variant = -1, GemmEpi epi = GemmEpi());
 // complex = real x complex
 int gemm_dz(hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, cplx alpha,
             const double* A, int lda, long long sA, const cplx* B, int ldb, long long sB,
             cplx beta, cplx* C, int ldc, long long sC, int batch, int divA = 1,
-            int divB = 1);
+            int divB = 1, GemmEpi epi = GemmEpi());
 // complex = complex x real
 int gemm_zd(hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, cplx alpha,
             const cplx* A, int lda, long long sA, const double* B, int ldb, long long sB,
             cplx beta, cplx* C, int ldc, long long sC, int batch, int divA = 1,
-            int divB = 1);
+            int divB = 1, GemmEpi epi = GemmEpi());
 // real = real x real
 int gemm_dd(hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, double alpha,
             const double* A, int lda, long long sA, const double* B, int ldb, long long sB,
@@ -134,13 +144,13 @@ int gemm_grouped(hipStream_t s, int M, const cplx* X, cplx* C, int ld, const voi
 // that signature.  No effect with TG_GEMM=vector or a forced variant.
 int gemm_tune_zz(hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, const cplx* A, int lda,
                  long long sA, const cplx* B, int ldb, long long sB, cplx* C, int ldc,
-                 long long sC, int batch);
+                 long long sC, int batch, int skew = 0);
 int gemm_tune_dz(hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, const double* A,
                  int lda, long long sA, const cplx* B, int ldb, long long sB, cplx* C, int ldc,
-                 long long sC, int batch);
+                 long long sC, int batch, int skew = 0);
 int gemm_tune_zd(hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, const cplx* A, int lda,
                  long long sA, const double* B, int ldb, long long sB, cplx* C, int ldc,
-                 long long sC, int batch);
+                 long long sC, int batch, int skew = 0);
 int gemm_tune_grouped(hipStream_t s, int M, const cplx* X, cplx* C, int ld, const void* W,
                       const GroupDesc* groups_dev, const int* tile_group_dev,
                       const int* tile_j0_dev, int ntiles_total, int tag);

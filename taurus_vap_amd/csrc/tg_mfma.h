@@ -16,15 +16,15 @@ constexpr int TG_MFMA_GROUPED_VARIANTS = 5;
 int mfma_gemm_zz(int variant, hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, cplx alpha,
                  const cplx* A, int lda, long long sA, const cplx* B, int ldb, long long sB,
                  cplx beta, int use_beta, cplx* C, int ldc, long long sC, int batch,
-                 int divA = 1, int divB = 1);
+                 int divA = 1, int divB = 1, const GemmEpi& epi = GemmEpi());
 int mfma_gemm_dz(int variant, hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, cplx alpha,
                  const double* A, int lda, long long sA, const cplx* B, int ldb, long long sB,
                  cplx beta, int use_beta, cplx* C, int ldc, long long sC, int batch,
-                 int divA = 1, int divB = 1);
+                 int divA = 1, int divB = 1, const GemmEpi& epi = GemmEpi());
 int mfma_gemm_zd(int variant, hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, cplx alpha,
                  const cplx* A, int lda, long long sA, const double* B, int ldb, long long sB,
                  cplx beta, int use_beta, cplx* C, int ldc, long long sC, int batch,
-                 int divA = 1, int divB = 1);
+                 int divA = 1, int divB = 1, const GemmEpi& epi = GemmEpi());
 int mfma_gemm_grouped(int variant, hipStream_t s, int M, const cplx* X, cplx* C, int ld,
                       const void* W, const GroupDesc* groups_dev, const int* tile_group_dev,
                       const int* tile_j0_dev, int ntiles_total);

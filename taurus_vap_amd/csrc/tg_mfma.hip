@@ -42,6 +42,8 @@ constexpr int XCDS = 8;
 // hold 16 consecutive rows of a column and loads and stores of C are unit-stride.
 // Rows and columns past the edge repeat the last one and are not stored; k past the
 // end is masked in the last chunk only.
+// A skew product (GemmEpi) forms the tiles that reach the diagonal or lie below it, 44 of
+// 77 of 48 x 32 at order 336, and stores each element at its transposed place as well.
 // Complex x complex is three real products (Gauss): cr = sum Ar Br, ci = sum Ai Bi,
 // c3 = sum (Ar + Ai)(Br + Bi); C = (cr - ci, c3 - cr - ci).
 // Bound by the matrix cores, the load latency covered by the steps in flight and 2-4
@@ -60,7 +62,7 @@ __global__ void __launch_bounds__(256, OCC)
 mfma_batched_kernel(int M, int N, int K, cplx alpha, const TA* __restrict__ A, int lda,
                     long long sA, const TB* __restrict__ B, int ldb, long long sB, cplx beta,
                     int use_beta, cplx* __restrict__ C, int ldc, long long sC, int batch,
-                    int tiles_m, int tiles, int per, int divA, int divB) {
+                    int tiles_m, int tiles, int per, int divA, int divB, GemmEpi ep) {
   constexpr bool CA = IsC<TA>::v, CB = IsC<TB>::v, CC = CA && CB;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // the batch * tiles (element, tile) pairs are cut into 8 contiguous runs, one per XCD
@@ -69,7 +71,13 @@ mfma_batched_kernel(int M, int N, int K, cplx alpha, const TA* __restrict__ A, i
   const unsigned g = (blockIdx.x % XCDS * (unsigned)per + blockIdx.x / XCDS) * 4 + w;
   if (g >= (unsigned)batch * (unsigned)tiles) return;
   const int b = (int)(g / (unsigned)tiles), tile = (int)(g - (unsigned)b * (unsigned)tiles);
-  const int m0 = (tile % tiles_m) * 16 * TM, n0 = (tile / tiles_m) * 16 * TN;
+  int ti = tile % tiles_m, tj = tile / tiles_m;
+  if (ep.skew) {        // the tiles that reach the diagonal or lie below it, by columns
+    ti = tile;
+    for (tj = 0; ti >= tiles_m - tj * TN / TM; ++tj) ti -= tiles_m - tj * TN / TM;
+    ti += tj * TN / TM;
+  }
+  const int m0 = ti * 16 * TM, n0 = tj * 16 * TN;
   const int lr = lane & 15, lk = lane >> 4;
   const TA* Ab = A + (long long)(b / divA) * sA;
   const TB* Bb = B + (long long)(b / divB) * sB;
@@ -160,6 +168,7 @@ mfma_batched_kernel(int M, int N, int K, cplx alpha, const TA* __restrict__ A, i
   }
   // lane: row lr, columns lk + 4 r of each 16 x 16 block
   cplx* Cb = C + (long long)b * sC;
+  const double* add = ep.add ? ep.add + (long long)(b / ep.divAdd) * ep.sAdd : nullptr;
 #pragma unroll
   for (int x = 0; x < TM; ++x) {
     const int gi = m0 + 16 * x + lr;
@@ -169,7 +178,7 @@ mfma_batched_kernel(int M, int N, int K, cplx alpha, const TA* __restrict__ A, i
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int gj = n0 + 16 * y + lk + 4 * r;
-        if (gj >= N) continue;
+        if (gj >= N || (ep.skew && gi < gj)) continue;
         cplx* cp = Cb + gi + (long long)gj * ldc;
         cplx p;
         if constexpr (CC)
@@ -178,6 +187,12 @@ mfma_batched_kernel(int M, int N, int K, cplx alpha, const TA* __restrict__ A, i
           p = cmk(cr[x][y][r], ci[x][y][r]);
         cplx v = cmul(alpha, p);
         if (use_beta) v = cadd(v, cmul(beta, *cp));
+        if (ep.conj) v.y = -v.y;
+        if (add) v.x += add[gi + (long long)gj * ldc];
+        if (ep.skew) {
+          if (gi == gj) v = cmk(0.0, 0.0);
+          else Cb[gj + (long long)gi * ldc] = cmk(-v.x, -v.y);
+        }
         *cp = v;
       }
   }
@@ -425,9 +440,18 @@ grouped_vec_kernel(GroupedArgs g) {
 template <typename TA, typename TB, int OPA, int OPB, int TM, int TN, int KS, int OCC>
 int launch_batched(hipStream_t s, int M, int N, int K, cplx alpha, const TA* A, int lda,
                    long long sA, const TB* B, int ldb, long long sB, cplx beta, int use_beta,
-                   cplx* C, int ldc, long long sC, int batch, int divA, int divB) {
+                   cplx* C, int ldc, long long sC, int batch, int divA, int divB,
+                   const GemmEpi& ep) {
   const int tiles_m = (M + 16 * TM - 1) / (16 * TM), tiles_n = (N + 16 * TN - 1) / (16 * TN);
-  const int tiles = tiles_m * tiles_n;
+  int tiles = tiles_m * tiles_n;
+  if (ep.skew) {
+    if (M != N || use_beta) {
+      tg_set_error("mfma gemm: a skew product is square and written, not added");
+      return TG_E_ARG;
+    }
+    tiles = 0;
+    for (int j = 0; j < tiles_n; ++j) tiles += tiles_m - j * TN / TM;
+  }
   const long long wgs = ((long long)batch * tiles + 3) / 4;      // four waves, a tile each
   const long long per = (wgs + XCDS - 1) / XCDS, grid = (long long)XCDS * per;
   if (grid > 0x1fffffffLL) {          // tile numbers in 32 bits
@@ -437,7 +461,7 @@ int launch_batched(hipStream_t s, int M, int N, int K, cplx alpha, const TA* A, 
   if (grid == 0) return TG_OK;
   hipLaunchKernelGGL((mfma_batched_kernel<TA, TB, OPA, OPB, TM, TN, KS, OCC>), dim3((unsigned)grid),
                      dim3(256), 0, s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, use_beta, C, ldc,
-                     sC, batch, tiles_m, tiles, (int)per, divA, divB);
+                     sC, batch, tiles_m, tiles, (int)per, divA, divB, ep);
   TG_HIP(hipGetLastError());
   return TG_OK;
 }
@@ -445,12 +469,13 @@ int launch_batched(hipStream_t s, int M, int N, int K, cplx alpha, const TA* A, 
 template <typename TA, typename TB, int OPA, int OPB>
 int launch_variant(int variant, hipStream_t s, int M, int N, int K, cplx alpha, const TA* A,
                    int lda, long long sA, const TB* B, int ldb, long long sB, cplx beta,
-                   int use_beta, cplx* C, int ldc, long long sC, int batch, int divA, int divB) {
+                   int use_beta, cplx* C, int ldc, long long sC, int batch, int divA, int divB,
+                   const GemmEpi& ep) {
 #define TG_V(K_, TM, TN, KS, OCC)                                                               \
   case K_:                                                                                      \
     return launch_batched<TA, TB, OPA, OPB, TM, TN, KS, OCC>(s, M, N, K, alpha, A, lda, sA, B,  \
                                                              ldb, sB, beta, use_beta, C, ldc,   \
-                                                             sC, batch, divA, divB);
+                                                             sC, batch, divA, divB, ep);
   switch (variant) {
     TG_V(0, 2, 2, 2, 3)
     TG_V(1, 2, 2, 4, 2)
@@ -472,11 +497,12 @@ int launch_variant(int variant, hipStream_t s, int M, int N, int K, cplx alpha, 
 template <typename TA, typename TB>
 int dispatch(int variant, hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, cplx alpha,
              const TA* A, int lda, long long sA, const TB* B, int ldb, long long sB, cplx beta,
-             int use_beta, cplx* C, int ldc, long long sC, int batch, int divA, int divB) {
+             int use_beta, cplx* C, int ldc, long long sC, int batch, int divA, int divB,
+             const GemmEpi& ep) {
 #define TG_CASE(OA, OB)                                                                        \
   if (opa == OA && opb == OB)                                                                  \
     return launch_variant<TA, TB, OA, OB>(variant, s, M, N, K, alpha, A, lda, sA, B, ldb, sB,  \
-                                          beta, use_beta, C, ldc, sC, batch, divA, divB);
+                                          beta, use_beta, C, ldc, sC, batch, divA, divB, ep);
   TG_CASE(OP_N, OP_N) TG_CASE(OP_N, OP_T) TG_CASE(OP_T, OP_N) TG_CASE(OP_T, OP_T)
   if (IsC<TA>::v) { TG_CASE(OP_C, OP_N) TG_CASE(OP_C, OP_T) }
   if (IsC<TB>::v) { TG_CASE(OP_N, OP_C) TG_CASE(OP_T, OP_C) }
@@ -490,28 +516,28 @@ int dispatch(int variant, hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K
 
 int mfma_gemm_zz(int variant, hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, cplx alpha,
                  const cplx* A, int lda, long long sA, const cplx* B, int ldb, long long sB,
-                 cplx beta, int use_beta, cplx* C, int ldc, long long sC, int batch, int divA,
-                 int divB) {
+                 cplx beta, int use_beta, cplx* C, int ldc, long long sC, int batch, int divA, int divB,
+                 const GemmEpi& ep) {
   return dispatch<cplx, cplx>(variant, s, opa, opb, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta,
-                              use_beta, C, ldc, sC, batch, divA, divB);
+                              use_beta, C, ldc, sC, batch, divA, divB, ep);
 }
 
 int mfma_gemm_dz(int variant, hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, cplx alpha,
                  const double* A, int lda, long long sA, const cplx* B, int ldb, long long sB,
-                 cplx beta, int use_beta, cplx* C, int ldc, long long sC, int batch, int divA,
-                 int divB) {
+                 cplx beta, int use_beta, cplx* C, int ldc, long long sC, int batch, int divA, int divB,
+                 const GemmEpi& ep) {
   if (opa == OP_C) opa = OP_T;
   return dispatch<double, cplx>(variant, s, opa, opb, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta,
-                                use_beta, C, ldc, sC, batch, divA, divB);
+                                use_beta, C, ldc, sC, batch, divA, divB, ep);
 }
 
 int mfma_gemm_zd(int variant, hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, cplx alpha,
                  const cplx* A, int lda, long long sA, const double* B, int ldb, long long sB,
-                 cplx beta, int use_beta, cplx* C, int ldc, long long sC, int batch, int divA,
-                 int divB) {
+                 cplx beta, int use_beta, cplx* C, int ldc, long long sC, int batch, int divA, int divB,
+                 const GemmEpi& ep) {
   if (opb == OP_C) opb = OP_T;
   return dispatch<cplx, double>(variant, s, opa, opb, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta,
-                                use_beta, C, ldc, sC, batch, divA, divB);
+                                use_beta, C, ldc, sC, batch, divA, divB, ep);
 }
 
 int mfma_gemm_grouped(int variant, hipStream_t s, int M, const cplx* X, cplx* C, int ld,

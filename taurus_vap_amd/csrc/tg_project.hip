@@ -130,21 +130,6 @@ __global__ void row_sign_kernel(long long tot, int n, const double* __restrict__
   Ds[idx] = sgn[idx % n] * D[idx];
 }
 
-// One pass after the A_phi product: A_phi = conj(A_phi), and U~, V~ preset to the
-// real U, V of the item's state (state (b0 + a) / A at U + s * nn) for the
-// GEMMs that add V A_phi and U A_phi
-__global__ void thouless_prep_kernel(long long nn, int na, long long b0, int A,
-                                     const double* __restrict__ U, const double* __restrict__ V,
-                                     cplx* __restrict__ Aphi, cplx* __restrict__ Ut,
-                                     cplx* __restrict__ Vt) {
-  long long idx = (long long)blockIdx.x * NT + threadIdx.x;
-  if (idx >= nn * na) return;
-  const long long st = (b0 + idx / nn) / A, e = st * nn + idx % nn;
-  Aphi[idx].y = -Aphi[idx].y;
-  Ut[idx] = cmk(U[e], 0.0);
-  Vt[idx] = cmk(V[e], 0.0);
-}
-
 // h_a = Gamma_a + H1
 __global__ void add_h1_kernel(long long nn, int na, const cplx* __restrict__ H1,
                               const cplx* __restrict__ G, cplx* __restrict__ h) {
@@ -1015,7 +1000,7 @@ int project_upload(tg_ctx* c) {
     TG_TRY(gemm_tune_zz(s, OP_N, OP_N, n, n, n, Xa, n, nn, Ta, n, nn, Ya, n, nn, chunk));
     TG_TRY(gemm_tune_zz(s, OP_T, OP_N, n, n, n, Xa, n, nn, Ta, n, nn, Ya, n, nn, chunk));
     TG_TRY(gemm_tune_dz(s, OP_N, OP_N, n, n, n, U, n, 0, Xa, n, nn, Ya, n, nn, chunk));
-    TG_TRY(gemm_tune_dz(s, OP_N, OP_T, n, n, n, U, n, 0, Xa, n, nn, Ya, n, nn, chunk));
+    TG_TRY(gemm_tune_dz(s, OP_N, OP_T, n, n, n, U, n, 0, Xa, n, nn, Ya, n, nn, chunk, 1));
     TG_TRY(gemm_tune_zd(s, OP_N, OP_T, n, n, n, Xa, n, nn, U, n, 0, Ya, n, nn, chunk));
     c->tuned_n = n;
     c->tuned_chunk = chunk;
@@ -1260,19 +1245,29 @@ int project_run(tg_ctx* c) {
       ScopedTiming tm(c, "gemm");
       const double* Uc = U + (size_t)(a0 / A) * nn;
       const double* Vc = V + (size_t)(a0 / A) * nn;
+      // A_phi = conj(V_phi U_phi^-1) and the pairing tensors are skew, so half of each
+      // product gives it; U and V are added, and A_phi conjugated, as the products are
+      // stored (225 angles, 336 states: 17.6 -> 16.8 ms a projection)
+      GemmEpi skew, aphi;
+      skew.skew = aphi.skew = aphi.conj = 1;
+      auto plus = [&](const double* W) {
+        GemmEpi e;
+        e.add = W;
+        e.sAdd = nn;
+        e.divAdd = A;
+        return e;
+      };
       {
         ScopedTiming tz(c, "kernel:zgemm");
-        TG_TRY(gemm_zz(s, OP_N, OP_N, n, n, n, one, Vphi, n, nn, Uphi, n, nn, zero, Aphi, n, nn, na));
+        TG_TRY(gemm_zz(s, OP_N, OP_N, n, n, n, one, Vphi, n, nn, Uphi, n, nn, zero, Aphi, n, nn, na, 1, 1,
+                       -1, aphi));
       }
-      hipLaunchKernelGGL(thouless_prep_kernel, dim3(nblk(tot)), dim3(NT), 0, s, nn, na,
-                         (long long)a0, A, U, V, Aphi, Ut, Vt);
-      TG_HIP(hipGetLastError());
-      TG_TRY(gemm_dz(s, OP_N, OP_N, n, n, n, one, Vc, n, nn, Aphi, n, nn, one, Ut, n, nn, na, A, 1));
-      TG_TRY(gemm_dz(s, OP_N, OP_N, n, n, n, one, Uc, n, nn, Aphi, n, nn, one, Vt, n, nn, na, A, 1));
+      TG_TRY(gemm_dz(s, OP_N, OP_N, n, n, n, one, Vc, n, nn, Aphi, n, nn, zero, Ut, n, nn, na, A, 1, plus(Uc)));
+      TG_TRY(gemm_dz(s, OP_N, OP_N, n, n, n, one, Uc, n, nn, Aphi, n, nn, zero, Vt, n, nn, na, A, 1, plus(Vc)));
       // densities (calculate_densities with conj(U~), conj(V~))
       TG_TRY(gemm_zd(s, OP_N, OP_T, n, n, n, one, Vt, n, nn, Vc, n, nn, zero, rho, n, nn, na, 1, A));
-      TG_TRY(gemm_zd(s, OP_N, OP_T, n, n, n, one, Vt, n, nn, Uc, n, nn, zero, kLR, n, nn, na, 1, A));
-      TG_TRY(gemm_dz(s, OP_N, OP_T, n, n, n, one, Vc, n, nn, Ut, n, nn, zero, kRL, n, nn, na, A, 1));
+      TG_TRY(gemm_zd(s, OP_N, OP_T, n, n, n, one, Vt, n, nn, Uc, n, nn, zero, kLR, n, nn, na, 1, A, skew));
+      TG_TRY(gemm_dz(s, OP_N, OP_T, n, n, n, one, Vc, n, nn, Ut, n, nn, zero, kRL, n, nn, na, A, 1, skew));
     }
     // fields; in the projection the pp channel's scatters (third stream) are joined
     // after the first H20 product, which needs only h
