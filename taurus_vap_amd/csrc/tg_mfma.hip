@@ -200,67 +200,67 @@ mfma_batched_kernel(int M, int N, int K, cplx alpha, const TA* __restrict__ A, i
 
 // Real FP64 GEMM on the matrix cores for the real products of the constraint
 // machinery and the canonical basis (n x n, batched over states):
-// C[b] = alpha op(A[b]) op(B[b]) + beta C[b].  A 32 x 32 tile per workgroup of
-// four waves, one 16 x 16 MFMA block per wave, K staged 16 deep in LDS.  Each
-// wave computes the transposed block (D = op(B)^T op(A)^T), so that lane l
-// holds rows l % 16 of four columns: the stores are unit-stride.
+// C[b] = alpha op(A[b]) op(B[b]) + beta C[b].  One 16 x 16 tile of C per workgroup, a
+// quarter of k per wave: few tiles (one state's matrices) and short products, so the time
+// is the latency of a wave's chain, and a quarter of it with every wave's operands, 32 k
+// at a time, straight in registers (mfma_batched_kernel's scheme) is the shortest one.  The
+// four partial sums meet in LDS.  The transposed block is computed (D = op(B)^T op(A)^T),
+// so that lane l holds rows l % 16 of four columns: the stores are unit-stride.
+// One product of order 224 6.1 us, 336 14.7, medians inside a descent (32 x 32 tiles
+// staged 16 k at a time through LDS: 19-23, 27).
 template <int OPA, int OPB>
 __global__ void __launch_bounds__(256)
 mfma_dd_kernel(int M, int N, int K, double alpha, const double* __restrict__ A, int lda,
                long long sA, const double* __restrict__ B, int ldb, long long sB, double beta,
                int use_beta, double* __restrict__ C, int ldc, long long sC, int tiles_m, int divA,
                int divB) {
-  constexpr int BT = 32, BK = 16, LD = BT + 1;
-  __shared__ double As[BK][LD], Bs[BK][LD];     // As[k][i] = op(A)(i,k), Bs[k][j] = op(B)(k,j)
+  constexpr int KS = 8;                          // k steps of 4 in flight
+  constexpr bool AN = OPA == OP_N, BN = OPB == OP_N;
+  __shared__ double part[4][4][64];
   const int b = blockIdx.y;
   const double* Ab = A + (long long)(b / divA) * sA;
   const double* Bb = B + (long long)(b / divB) * sB;
   double* Cb = C + (long long)b * sC;
-  const int m0 = (blockIdx.x % tiles_m) * BT, n0 = (blockIdx.x / tiles_m) * BT;
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const int wi = (w & 1) * 16, wj = (w >> 1) * 16;
+  const int m0 = (blockIdx.x % tiles_m) * 16, n0 = (blockIdx.x / tiles_m) * 16;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lr = lane & 15, lk = lane >> 4;
+  const int kq = (K + 15) / 16 * 4;              // k of a wave
+  const int kb = w * kq, ke = min(K, kb + kq);
+  const long long ka = AN ? lda : 1, kc = BN ? 1 : ldb;      // elements per k
+  const double* pa = Ab + (AN ? (long long)min(m0 + lr, M - 1) : (long long)min(m0 + lr, M - 1) * lda);
+  const double* pb = Bb + (BN ? (long long)min(n0 + lr, N - 1) * ldb : (long long)min(n0 + lr, N - 1));
   d4 acc = {0.0, 0.0, 0.0, 0.0};
-  for (int k0 = 0; k0 < K; k0 += BK) {
-    // 512 elements of each operand tile, two per thread, contiguous index fastest
+  double va[KS], vb[KS];
+  // lane quarter lk takes k = k0 + KS lk + s in step s
+  auto load = [&](int s, int k0) {
+    const int k = k0 + KS * lk + s;
+    const bool in = k < ke;
+    va[s] = in ? pa[k * ka] : 0.0;
+    vb[s] = in ? pb[k * kc] : 0.0;
+  };
+  if (kb < ke) {
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      const int e = t + 256 * r;
-      int i, k;
-      if (OPA == OP_N) { i = e % BT; k = e / BT; } else { k = e % BK; i = e / BK; }
-      const int gi = m0 + i, gk = k0 + k;
-      double v = 0.0;
-      if (gi < M && gk < K) v = (OPA == OP_N) ? Ab[gi + (long long)gk * lda] : Ab[gk + (long long)gi * lda];
-      As[k][i] = v;
-      int j, k2;
-      if (OPB == OP_N) { k2 = e % BK; j = e / BK; } else { j = e % BT; k2 = e / BT; }
-      const int gj = n0 + j, gk2 = k0 + k2;
-      double u = 0.0;
-      if (gj < N && gk2 < K) u = (OPB == OP_N) ? Bb[gk2 + (long long)gj * ldb] : Bb[gj + (long long)gk2 * ldb];
-      Bs[k2][j] = u;
-    }
-    __syncthreads();
+    for (int s = 0; s < KS; ++s) load(s, kb);
+    for (int k0 = kb + 4 * KS; k0 < ke; k0 += 4 * KS) {
 #pragma unroll
-    for (int kk = 0; kk < BK; kk += 4) {
-      const double av = Bs[kk + lk][wj + lr];    // D rows: columns of C
-      const double bv = As[kk + lk][wi + lr];    // D columns: rows of C
-      acc = mfma(av, bv, acc);
-    }
-    __syncthreads();
-  }
-  // lane l, register r: C(m0 + wi + lr, n0 + wj + lk + 4 r)
-  const int gi = m0 + wi + lr;
-  if (gi < M) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int gj = n0 + wj + lk + 4 * r;
-      if (gj < N) {
-        double* cp = Cb + gi + (long long)gj * ldc;
-        double v = alpha * acc[r];
-        if (use_beta) v = fma(beta, *cp, v);
-        *cp = v;
+      for (int s = 0; s < KS; ++s) {
+        acc = mfma(vb[s], va[s], acc);
+        load(s, k0);
       }
     }
+#pragma unroll
+    for (int s = 0; s < KS; ++s) acc = mfma(vb[s], va[s], acc);
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) part[w][r][lane] = acc[r];
+  __syncthreads();
+  // wave w adds register w: C(m0 + lr, n0 + lk + 4 w)
+  const int gi = m0 + lr, gj = n0 + lk + 4 * w;
+  if (gi < M && gj < N) {
+    double* cp = Cb + gi + (long long)gj * ldc;
+    double v = alpha * ((part[0][w][lane] + part[1][w][lane]) + (part[2][w][lane] + part[3][w][lane]));
+    if (use_beta) v = fma(beta, *cp, v);
+    *cp = v;
   }
 }
 
@@ -586,7 +586,7 @@ int mfma_gemm_dd(hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, double 
                  double beta, int use_beta, double* C, int ldc, long long sC, int batch, int divA,
                  int divB) {
   if (M <= 0 || N <= 0 || batch <= 0) return TG_OK;
-  const int tiles_m = (M + 31) / 32, tiles_n = (N + 31) / 32;
+  const int tiles_m = (M + 15) / 16, tiles_n = (N + 15) / 16;
   const dim3 grid(tiles_m * tiles_n, batch);
 #define TG_DD(OA, OB)                                                                              \
   hipLaunchKernelGGL((mfma_dd_kernel<OA, OB>), grid, dim3(256), 0, s, M, N, K, alpha, A, lda, sA, \
