@@ -138,41 +138,15 @@ __global__ void add_h1_kernel(long long nn, int na, const cplx* __restrict__ H1,
   h[idx] = cadd(G[idx], H1[idx % nn]);
 }
 
-// H20 = G - G^T per angle, through 32 x 32 LDS tiles (both reads coalesced).
-// With G = U~^T (h V~ + fd/2 DeltaLR U~) - fd/2 V~^T DeltaRL V~ this is
-// calculate_H20 (module_fields.f90:366-391): U~^T h V~ - (.)^T + fd (U~^T DeltaLR U~
-// - V~^T DeltaRL V~), the two Delta terms being skew.
-__global__ void __launch_bounds__(256)
-skew_part_kernel(int n, const cplx* __restrict__ G, cplx* __restrict__ H) {
-  __shared__ cplx ta[32][33], tb[32][33];
-  const long long nn = (long long)n * n;
-  const long long a = blockIdx.z;
-  const int i0 = blockIdx.x * 32, j0 = blockIdx.y * 32;
-  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;   // 32 x 8
-  const cplx* g = G + a * nn;
-  for (int r = ty; r < 32; r += 8) {
-    const int i = i0 + tx, j = j0 + r;           // G(i, j): column j, row i (coalesced in i)
-    ta[r][tx] = (i < n && j < n) ? g[i + (long long)j * n] : cmk(0.0, 0.0);
-    const int i2 = j0 + tx, j2 = i0 + r;         // G(j0 + tx, i0 + r)
-    tb[r][tx] = (i2 < n && j2 < n) ? g[i2 + (long long)j2 * n] : cmk(0.0, 0.0);
-  }
-  __syncthreads();
-  for (int r = ty; r < 32; r += 8) {
-    const int i = i0 + tx, j = j0 + r;
-    if (i < n && j < n) {
-      const cplx x = ta[r][tx], xt = tb[tx][r];   // G(i, j), G(j, i)
-      H[a * nn + i + (long long)j * n] = cmk(x.x - xt.x, x.y - xt.y);
-    }
-  }
-}
-
 // Per-angle traces (calculate_particle_number :78-143, calculate_expectval_energy
 // module_hamiltonian.f90:1098-1126).  out[a*9 + k]:
 // 0 prot, 1 neut, 2 Tr(rho_p^2), 3 Tr(kRL_p^T kLR_p), 4 Tr(rho_n^2),
 // 5 Tr(kRL_n^T kLR_n), 6 Tr(H1 rho), 7 Tr(Gamma rho), 8 Tr(DeltaLR kRL^T)
 // A workgroup sums the elements (i, j) of one band of 32 rows i of one angle,
 // 32 columns j at a time; rho(j, i) comes from a 32 x 32 tile of rho staged in
-// LDS, so every global read is coalesced.  part[(a * bands + band) * 9 + k];
+// LDS, so every global read is coalesced; kLR, kRL and DeltaLR are skew, so the
+// elements below the diagonal count twice.  225 angles of
+// order 336 0.33 ms (whole matrices 0.42).  part[(a * bands + band) * 9 + k];
 // traces_sum_kernel adds the bands.
 constexpr int TRT = 32;
 __global__ void __launch_bounds__(NT)
@@ -208,16 +182,20 @@ traces_kernel(int n, const cplx* __restrict__ H1, const cplx* __restrict__ rho,
         const cplx rji = T[jj][tx];
         const bool pj = j < h;
         if (i == j) acc[pi ? 0 : 1] = cadd(acc[pi ? 0 : 1], r_[idx]);
-        if (pi == pj) {
-          cfma(acc[pi ? 2 : 4], r_[idx], rji);
-          cfma(acc[pi ? 3 : 5], kr[idx], kl[idx]);
-        }
+        if (pi == pj) cfma(acc[pi ? 2 : 4], r_[idx], rji);
         cfma(acc[6], H1[idx], rji);
         cfma(acc[7], g_[idx], rji);
-        cfma(acc[8], dl[idx], kr[idx]);
+        if (i > j) {
+          const cplx k = kr[idx];
+          if (pi == pj) cfma(acc[pi ? 3 : 5], k, kl[idx]);
+          cfma(acc[8], dl[idx], k);
+        }
       }
     __syncthreads();
   }
+  acc[3] = cscale(acc[3], 2.0);
+  acc[5] = cscale(acc[5], 2.0);
+  acc[8] = cscale(acc[8], 2.0);
   __shared__ cplx red[NT];
   for (int k = 0; k < 9; ++k) {
     red[threadIdx.x] = acc[k];
@@ -417,40 +395,90 @@ gauge_scalars_kernel(int na, int n, cplx H0, const cplx* __restrict__ w, const c
   if (threadIdx.x < 7) pnp[threadIdx.x] = red[threadIdx.x][0];
 }
 
-// pnp_A = sum f1 A, pnp_H20 = sum f1 H20, pnp_AH20 = sum f2 A   (angles in order)
-// state blockIdx.y: items s*na .., sums at pA/pH/pAH + s * os
-__global__ void gauge_matrices_kernel(long long nn, int na, const cplx* __restrict__ f120,
-                                      const double* __restrict__ mult,
-                                      const cplx* __restrict__ Aphi0, const cplx* __restrict__ H200,
-                                      long long stride, cplx* __restrict__ pA0,
-                                      cplx* __restrict__ pH0, cplx* __restrict__ pAH0, long long os) {
-  long long idx = (long long)blockIdx.x * NT + threadIdx.x;
-  if (idx >= nn) return;
+// pnp_A = sum f1 A, pnp_H20 = sum f1 H20, pnp_AH20 = sum f2 A over the angles, with
+// H20 = G - G^T: with G = U~^T (h V~ + fd/2 DeltaLR U~) - fd/2 V~^T DeltaRL V~ this is
+// calculate_H20 (module_fields.f90:366-391): U~^T h V~ - (.)^T + fd (U~^T DeltaLR U~
+// - V~^T DeltaRL V~), the two Delta terms being skew.  The sum over the angles comes
+// first, so G - G^T is formed once per state and not per angle.
+// A workgroup takes an 8 x 8 tile and its transposed one, a wave a sixteenth of the angles.
+// State blockIdx.y: items s*na .., sums at pA/pH/pAH + s * os.  Bound by HBM (225 angles of
+// order 336: 155 us, 5.2 TB/s), for small n by the loads in flight (121 of order 140: 20 us,
+// 49 of order 24: 7).  G - G^T per angle and a thread per element over all angles: 347,
+// 83 and 27 us; tiles of 16 x 16 with four sums: 139, 47 and 13.
+constexpr int GMT = 8, GMQ = 16, GMA = 256;   // GMA: angles whose factors are staged
+__global__ void __launch_bounds__(GMT * GMT * GMQ)
+gauge_matrices_kernel(int n, int na, const cplx* __restrict__ f120, const double* __restrict__ mult,
+                      const cplx* __restrict__ Aphi0, const cplx* __restrict__ G0, long long stride,
+                      cplx* __restrict__ pA0, cplx* __restrict__ pH0, cplx* __restrict__ pAH0,
+                      long long os) {
+  __shared__ cplx red[GMQ][3][GMT * GMT], tot[2][GMT * GMT], fm[GMA][2];
+  __shared__ bool pm[GMA];
+  int ti = blockIdx.x, tj = 0;                 // ti <= tj: the pairs of tiles by columns
+  while (ti > tj) ti -= ++tj;
   const long long st = blockIdx.y;
   const cplx* f12 = f120 + st * 2 * na;
   const cplx* Aphi = Aphi0 + st * na * stride;
-  const cplx* H20 = H200 + st * na * stride;
-  cplx* pA = pA0 + st * os;
-  cplx* pH = pH0 + st * os;
-  cplx* pAH = pAH0 + st * os;
-  cplx sa = cmk(0, 0), sh = cmk(0, 0), sah = cmk(0, 0);
-  for (int a = 0; a < na; ++a) {
-    const cplx f1 = f12[2 * a], f2 = f12[2 * a + 1];
-    const cplx av = Aphi[a * stride + idx], hv = H20[a * stride + idx];
-    if (mult[a] > 1.5) {        // conjugate pair: 2 Re(.)
-      const cplx t1 = cmul(av, f1), t2 = cmul(hv, f1), t3 = cmul(av, f2);
-      sa.x += 2.0 * t1.x;
-      sh.x += 2.0 * t2.x;
-      sah.x += 2.0 * t3.x;
-    } else {
-      cfma(sa, av, f1);
-      cfma(sh, hv, f1);
-      cfma(sah, av, f2);
+  const cplx* G = G0 + st * na * stride;
+  const int e = threadIdx.x % (GMT * GMT), q = threadIdx.x / (GMT * GMT);
+  const int r = e % GMT, cc = e / GMT, tr = cc + GMT * r;
+  const int ii[2] = {GMT * ti + r, GMT * tj + r}, jj[2] = {GMT * tj + cc, GMT * ti + cc};
+  const int nt = ti == tj ? 1 : 2;
+  cplx sa[2], sh[2], sah[2];
+#pragma unroll
+  for (int x = 0; x < 2; ++x) sa[x] = sh[x] = sah[x] = cmk(0.0, 0.0);
+  bool in[2];
+  long long idx[2];
+#pragma unroll
+  for (int x = 0; x < 2; ++x) {
+    in[x] = x < nt && ii[x] < n && jj[x] < n;
+    idx[x] = in[x] ? ii[x] + (long long)jj[x] * n : 0;
+  }
+  for (int a0 = 0; a0 < na; a0 += GMA) {
+    const int ma = min(GMA, na - a0);
+    __syncthreads();
+    for (int a = threadIdx.x; a < ma; a += GMT * GMT * GMQ) {
+      fm[a][0] = cscale(f12[2 * (a0 + a)], mult[a0 + a]);     // mult 1 or 2
+      fm[a][1] = cscale(f12[2 * (a0 + a) + 1], mult[a0 + a]);
+      pm[a] = mult[a0 + a] > 1.5;
+    }
+    __syncthreads();
+#pragma unroll 4
+    for (int a = q; a < ma; a += GMQ) {
+      const cplx f1 = fm[a][0], f2 = fm[a][1];
+      const bool pair = pm[a];                 // conjugate pair: 2 Re(.)
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        const long long o = (a0 + a) * stride + idx[x];
+        const cplx av = Aphi[o], hv = G[o];
+        const double ya = sa[x].y, yh = sh[x].y, yah = sah[x].y;
+        cfma(sa[x], av, f1);
+        cfma(sh[x], hv, f1);
+        cfma(sah[x], av, f2);
+        sa[x].y = pair ? ya : sa[x].y;
+        sh[x].y = pair ? yh : sh[x].y;
+        sah[x].y = pair ? yah : sah[x].y;
+      }
     }
   }
-  pA[idx] = sa;
-  pH[idx] = sh;
-  pAH[idx] = sah;
+#pragma unroll
+  for (int x = 0; x < 2; ++x) {
+    if (x >= nt) break;                        // uniform
+    red[q][0][e] = sa[x];
+    red[q][1][e] = sh[x];
+    red[q][2][e] = sah[x];
+    __syncthreads();
+    if (q < 3) {
+      cplx v = red[0][q][e];
+#pragma unroll
+      for (int k = 1; k < GMQ; ++k) v = cadd(v, red[k][q][e]);
+      if (q == 1) tot[x][e] = v;
+      else if (in[x]) (q == 0 ? pA0 : pAH0)[st * os + idx[x]] = v;
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+    if (q == x && in[x]) pH0[st * os + idx[x]] = csub(tot[x][e], tot[nt - 1 - x][tr]);
 }
 
 // calculate_projected_H20 (:729-759); imag[block] = max Im over the block
@@ -800,7 +828,7 @@ struct RunPlan {
   long long nn, os, outs, is;               // strides: overlap set-up, outputs, imag
   bool proj, need_ovl, uniform;
   std::vector<OvlShape> sh;
-  cplx *work, *Akeep, *Hkeep;
+  cplx *work, *Akeep, *Gkeep;
   cplx *d_ph, *d_tr, *d_over, *d_ener, *d_f12, *d_pnp, *d_pre, *d_det, *d_phase, *d_w, *d_pari;
   cplx* d_trp;   // per-band partial traces of one chunk
   double *d_logabs, *d_imag, *d_mult;
@@ -881,7 +909,7 @@ RunPlan make_plan(tg_ctx* c) {
     }
   P.work = c->d_work.as<cplx>();
   P.Akeep = P.work + wsz;
-  P.Hkeep = P.Akeep + (size_t)B * nn;
+  P.Gkeep = P.Akeep + (size_t)B * nn;
   P.d_ph = c->d_scal.as<cplx>();
   P.d_tr = P.d_ph + 2 * A;
   P.d_over = P.d_tr + 9 * (size_t)B;
@@ -1095,7 +1123,7 @@ int project_run(tg_ctx* c) {
 
   auto Wb = [&](int k) { return P.work + (size_t)k * chunk * nn; };
   cplx* Akeep = P.Akeep;                     // A_phi of every item
-  cplx* Hkeep = P.Hkeep;                     // H20_phi of every item
+  cplx* Gkeep = P.Gkeep;                     // G of every item, H20_phi = G - G^T
   const long long os = P.os;
 
   // overlaps <Phi|R|Phi> for the gauge rotation (rot_over) and, when printing,
@@ -1216,8 +1244,7 @@ int project_run(tg_ctx* c) {
     cplx* dRL = Wb(W_DRL);
     cplx* X = Wb(W_X);
     cplx* Y = Wb(W_Y);
-    cplx* Z = Wb(W_Z);
-    cplx* H20 = Hkeep + (size_t)a0 * nn;
+    cplx* G20 = Gkeep + (size_t)a0 * nn;
 
     if (!proj) {
       hipLaunchKernelGGL(fill_cplx_kernel, dim3(nblk(na)), dim3(NT), 0, s, na, cmk(1.0, 0.0),
@@ -1277,7 +1304,7 @@ int project_run(tg_ctx* c) {
       TG_TRY(contraction_run(c, na, rho, kLR, proj ? kRL : nullptr, G, dLR, dRL, proj ? 0 : 1,
                              c->d_H1.as<cplx>(), hsp, split));
     }
-    // H20 (calculate_H20 with U~, V~) as G - G^T,
+    // H20 (calculate_H20 with U~, V~) is G - G^T, formed from the sum over the angles;
     //   X1 = h V~ + fd/2 DeltaLR U~,  X2 = -fd/2 DeltaRL V~,  G = U~^T X1 + V~^T X2
     const cplx hfd = cmk(0.5 * c->factor_delta, 0.0), mhfd = cmk(-0.5 * c->factor_delta, 0.0);
     auto zg = [&](TgOp oa, const cplx* Aa, cplx al, const cplx* Bb, cplx be, cplx* Cc) -> int {
@@ -1305,11 +1332,8 @@ int project_run(tg_ctx* c) {
       if (!split) TG_TRY(zg(OP_N, hsp, one, Vt, zero, X));
       TG_TRY(zg(OP_N, dLR, hfd, Ut, one, X));
       TG_TRY(zg(OP_N, dRL, mhfd, Vt, zero, Y));
-      TG_TRY(zg(OP_T, Ut, one, X, zero, Z));
-      TG_TRY(zg(OP_T, Vt, one, Y, one, Z));
-      hipLaunchKernelGGL(skew_part_kernel, dim3((n + 31) / 32, (n + 31) / 32, na), dim3(256), 0, s,
-                         n, Z, H20);
-      TG_HIP(hipGetLastError());
+      TG_TRY(zg(OP_T, Ut, one, X, zero, G20));
+      TG_TRY(zg(OP_T, Vt, one, Y, one, G20));
     }
   }
 
@@ -1335,8 +1359,9 @@ int project_run(tg_ctx* c) {
   double* H20v = reinterpret_cast<double*>(pAH + nn);
   hipLaunchKernelGGL(gauge_scalars_kernel, dim3(S), dim3(NT), 0, s, A, n, c->H0, P.d_w, P.d_over,
                      P.d_tr, c->iprint ? P.d_pari : nullptr, P.d_mult, P.d_f12, P.d_ener, P.d_pnp);
-  hipLaunchKernelGGL(gauge_matrices_kernel, dim3(nblk(nn), S), dim3(NT), 0, s, nn, A, P.d_f12,
-                     P.d_mult, Akeep, Hkeep, nn, pA, pH, pAH, P.outs);
+  const int gt = (n + GMT - 1) / GMT;
+  hipLaunchKernelGGL(gauge_matrices_kernel, dim3(gt * (gt + 1) / 2, S), dim3(GMT * GMT * GMQ), 0, s, n,
+                     A, P.d_f12, P.d_mult, Akeep, Gkeep, nn, pA, pH, pAH, P.outs);
   hipLaunchKernelGGL(projected_h20_kernel, dim3(nblk(nn), S), dim3(NT), 0, s, n, P.d_pnp, pA, pH,
                      pAH, H20v, P.d_imag, P.outs, P.is);
   TG_HIP(hipGetLastError());
