@@ -1246,14 +1246,25 @@ int project_run(tg_ctx* c) {
     cplx* Y = Wb(W_Y);
     cplx* G20 = Gkeep + (size_t)a0 * nn;
 
-    if (!proj) {
-      hipLaunchKernelGGL(fill_cplx_kernel, dim3(nblk(na)), dim3(NT), 0, s, na, cmk(1.0, 0.0),
-                         P.d_over + a0);
-      TG_HIP(hipGetLastError());
-    } else if (!defer) {
-      TG_TRY(overlap(Pp, Pn, a0, na, P.d_over + a0));
-    }
-    if (c->iprint && !defer) TG_TRY(overlap(R6 + 8 * ks, R6 + 9 * ks, a0, na, P.d_pari + a0));
+    // The overlaps on the second stream.  Inverse and Pfaffian both take a CU per item
+    // above order 64: beside each other while the items of both fit the CUs; with more of
+    // them the inverses would wait for Pfaffians, which then start after the densities and
+    // run beside the contraction (225 items: 80 states 1.09 -> 0.99 ms a projection, 140
+    // states 2.42 -> 2.39).  Larger products fill the chip and lose as much to the Pfaffians
+    // as the inverses do (336 states 16.4 and 16.4; 156 items of 224 states 4.39 -> 4.53).
+    const bool late = n > 64 && n <= 160 && 2 * na > 256;
+    auto overlaps = [&]() -> int {
+      if (!proj) {
+        hipLaunchKernelGGL(fill_cplx_kernel, dim3(nblk(na)), dim3(NT), 0, s, na, cmk(1.0, 0.0),
+                           P.d_over + a0);
+        TG_HIP(hipGetLastError());
+      } else if (!defer) {
+        TG_TRY(overlap(Pp, Pn, a0, na, P.d_over + a0));
+      }
+      if (c->iprint && !defer) TG_TRY(overlap(R6 + 8 * ks, R6 + 9 * ks, a0, na, P.d_pari + a0));
+      return TG_OK;
+    };
+    if (!late) TG_TRY(overlaps());
 
     // Thouless matrix A_phi (calculate_thouless :684-718)
     {
@@ -1295,6 +1306,11 @@ int project_run(tg_ctx* c) {
       TG_TRY(gemm_zd(s, OP_N, OP_T, n, n, n, one, Vt, n, nn, Vc, n, nn, zero, rho, n, nn, na, 1, A));
       TG_TRY(gemm_zd(s, OP_N, OP_T, n, n, n, one, Vt, n, nn, Uc, n, nn, zero, kLR, n, nn, na, 1, A, skew));
       TG_TRY(gemm_dz(s, OP_N, OP_T, n, n, n, one, Vc, n, nn, Ut, n, nn, zero, kRL, n, nn, na, A, 1, skew));
+    }
+    if (late) {
+      TG_HIP(hipEventRecord(c->ev_fork, s));
+      TG_HIP(hipStreamWaitEvent(s2, c->ev_fork, 0));
+      TG_TRY(overlaps());
     }
     // fields; in the projection the pp channel's scatters (third stream) are joined
     // after the first H20 product, which needs only h
