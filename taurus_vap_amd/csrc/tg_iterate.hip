@@ -186,6 +186,151 @@ chol_block_kernel(int n, int k0, int b, const double* __restrict__ A0, double* _
   if (threadIdx.x == 0 && bad && info[blockIdx.x] == 0) info[blockIdx.x] = bad;
 }
 
+// The Cholesky factorisation of a state's matrix and the inverse of its factor in one
+// workgroup (n <= CF_NMAX, state blockIdx.x at + s n^2): A (lower triangle read, destroyed)
+// = L L^T, X = L^-1 (zero above the diagonal), info[s] = 0 or the first non-positive pivot's
+// column (such a pivot is replaced by 1).
+// In steps of 32 columns, k of them done, with L_kk the factor of the diagonal block:
+// column t of Z = L_kk^-1 V is, for t past the block, row t of the panel of L (V: that of
+// A) and, for t up to it, column t of the rows k .. k + 31 of L^-1 (V: what the steps
+// before left there; the unit matrix in the block).  One rank-32 update M(r, c) -= Z_r . Z_c
+// then serves both: M(r, c), r >= c, is A's trailing matrix and M(r, c), r < k + 32,
+// the transposed unfinished rows c of L^-1, in the space above A's diagonal.
+// One wave factors the diagonal block in registers, a row per lane, while the others load
+// V; they solve a column of Z per thread (Z in LDS); all sixteen waves then update
+// 16 x 16 tiles on the matrix cores.
+// Bound by one CU and the chain of its steps (19 us each at order 40, half of it the square
+// roots and quotients of the diagonal block; 35 at 336, where the tiles are as long): orders
+// 40, 224, 336 take 38, 182, 387 us.  A launch per block and product, the block rows of
+// L^-1 on the second stream: 480 us at order 224 in a trace, HFB descent 15.3 -> 14.5 ms; at
+// 336 a descent takes the same 37.2 ms with either, with 50 launches fewer a step here.
+constexpr int CF_B = 32, CF_NW = 16, CF_TH = 64 * CF_NW, CF_NMAX = 512;
+inline int cf_zp(int n) { return (n + 31) / 32 * 32 + 16; }   // rows of Z 16 banks apart
+
+__device__ __forceinline__ double cf_readlane(double v, int lane) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)(unsigned long long)b, lane);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+
+__global__ void __launch_bounds__(CF_TH)
+chol_inverse_kernel(int n, int zp, double* __restrict__ A0, double* __restrict__ X0,
+                    int* __restrict__ info) {
+  typedef double d4 __attribute__((ext_vector_type(4)));
+  extern __shared__ double Z[];                  // CF_B rows of zp
+  __shared__ double Ld[CF_B][CF_B], Rd[CF_B];    // column k of L_kk at Ld[k], 1 / L_kk(k, k)
+  const long long nn = (long long)n * n;
+  double* M = A0 + blockIdx.x * nn;
+  double* X = X0 + blockIdx.x * nn;
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int tv = t - 64;                         // vector of this thread (waves 1 ..)
+  const int nb = (n + 15) / 16;
+  int bad = 0;
+  for (int e = t; e < CF_B * zp; e += CF_TH) Z[e] = 0.0;    // columns past n stay zero
+  __syncthreads();
+  for (int k0 = 0; k0 < n; k0 += CF_B) {
+    const int b = min(CF_B, n - k0), k1 = (k0 + CF_B) / 16;
+    double v[CF_B];
+    if (w == 0) {
+      const int i = lane & 31;                   // the upper half repeats the rows
+      const double* p = M + min(k0 + i, n - 1) + (long long)k0 * n;
+#pragma unroll
+      for (int k = 0; k < CF_B; ++k) v[k] = p[min(k, b - 1) * n];
+      if (b < CF_B)                              // the unit matrix past the last row
+#pragma unroll
+        for (int k = 0; k < CF_B; ++k)
+          if (max(i, k) >= b) v[k] = (i == k) ? 1.0 : 0.0;
+#pragma unroll
+      for (int k = 0; k < CF_B; ++k) {
+        double d = cf_readlane(v[k], k);
+        if (!(d > 0.0)) {
+          if (bad == 0) bad = k0 + k + 1;
+          d = 1.0;
+        }
+        d = sqrt(d);
+        const double l = (i == k) ? d : v[k] / d;
+        if (lane < CF_B) Ld[k][i] = l;           // (rows above k are not read)
+        if (lane == 0) Rd[k] = 1.0 / d;
+#pragma unroll
+        for (int j = k + 1; j < CF_B; ++j) v[j] = fma(-l, cf_readlane(l, j), v[j]);
+#pragma unroll
+        for (int j = k + 1; j < CF_B; ++j) asm volatile("" : "+v"(v[j]));   // here, not at their use
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else if (tv < n) {
+      const double* p = M + tv + (long long)k0 * n;
+#pragma unroll
+      for (int k = 0; k < CF_B; ++k) v[k] = p[min(k, b - 1) * n];
+      if (b < CF_B)
+#pragma unroll
+        for (int k = 0; k < CF_B; ++k) v[k] = (k < b) ? v[k] : 0.0;
+      if (tv >= k0 && tv < k0 + CF_B)
+#pragma unroll
+        for (int k = 0; k < CF_B; ++k) v[k] = (tv - k0 == k) ? 1.0 : 0.0;
+    }
+    __syncthreads();
+    if (w > 0 && tv < n) {
+#pragma unroll
+      for (int k = 0; k < CF_B; ++k) {
+        const double z = v[k] * Rd[k];
+        Z[k * zp + tv] = z;
+#pragma unroll
+        for (int m = k + 1; m < CF_B; ++m) v[m] = fma(-Ld[k][m], z, v[m]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    __syncthreads();
+    for (int e = t; e < CF_B * n; e += CF_TH) {
+      const int k = e % CF_B, c = e / CF_B;
+      if (k < b) X[(k0 + k) + (long long)c * n] = (c < k0 + CF_B) ? Z[k * zp + c] : 0.0;
+    }
+    // column blocks past this one; their rows up to it and from their diagonal on
+    const int lr = lane & 15, lk = lane >> 4;
+    int at = w, cb = k1, rb = 0;
+    auto next = [&]() -> bool {                  // this wave's next tile (rb, cb)
+      while (cb < nb && at >= k1 + nb - cb) {
+        at -= k1 + nb - cb;
+        ++cb;
+      }
+      if (cb >= nb) return false;
+      rb = at < k1 ? at : cb + at - k1;
+      at += CF_NW;
+      return true;
+    };
+    auto load = [&](double (&cv)[4]) {
+      const double* p = M + min(16 * rb + lr, n - 1);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) cv[q] = p[(long long)min(16 * cb + lk + 4 * q, n - 1) * n];
+    };
+    double cv[4], nv[4];
+    bool more = next();
+    if (more) load(cv);
+    while (more) {
+      const int r0 = 16 * rb, c0 = 16 * cb;
+      more = next();
+      if (more) load(nv);
+      d4 acc = {0.0, 0.0, 0.0, 0.0}, acc2 = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int s = 0; s < CF_B / 4; s += 2) {
+        const double* z = Z + (4 * s + lk) * zp + lr;
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(z[c0], z[r0], acc, 0, 0, 0);
+        acc2 = __builtin_amdgcn_mfma_f64_16x16x4f64(z[4 * zp + c0], z[4 * zp + r0], acc2, 0, 0, 0);
+      }
+      const bool fresh = r0 < 16 * k1 && r0 >= k0;            // rows of the unit matrix
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int c = c0 + lk + 4 * q;
+        if (r0 + lr < n && c < n)
+          M[r0 + lr + (long long)c * n] = (fresh ? 0.0 : cv[q]) - (acc[q] + acc2[q]);
+        cv[q] = nv[q];
+      }
+    }
+    __syncthreads();
+  }
+  if (t == 0) info[blockIdx.x] = bad;
+}
+
 // Gaussian elimination with partial pivoting of a small dense system (host);
 // false when singular.
 bool small_solve(int m, std::vector<double> A, std::vector<double>& b) {
@@ -394,7 +539,8 @@ int gram(const Iter& it, const double* c20, const std::vector<int>& states,
 }
 
 // cholesky_factorization + dtrtri of every state: A (n x n per state, destroyed)
-// = L L^T, X = L^-1 (dense, zero above the diagonal).  Right-looking blocked
+// = L L^T, X = L^-1 (dense, zero above the diagonal); one launch up to order CF_NMAX.
+// Above it, where Z does not fit the LDS: right-looking blocked
 // Cholesky with CB-wide panels (diagonal block in LDS, panel and trailing
 // update as GEMMs), then the off-diagonal blocks of L^-1 row block by row
 // block: X(i, :i) = -X(i, i) L(i, :i) X(:i, :i).  L and T are scratch (T:
@@ -407,6 +553,13 @@ int cholesky_inverse(const Iter& it, double* A, double* L, double* X, double* T,
   const int n = it.n, S = it.S;
   const long long nn = it.nn;
   hipStream_t s = it.s;
+  if (n <= CF_NMAX) {
+    const int zp = cf_zp(n);
+    hipLaunchKernelGGL(chol_inverse_kernel, dim3(S), dim3(CF_TH), sizeof(double) * CF_B * zp, s, n, zp,
+                       A, X, info);
+    TG_HIP(hipGetLastError());
+    return TG_OK;
+  }
   hipLaunchKernelGGL(fill_kernel, dim3(nblk(S * nn)), dim3(NT), 0, s, S * nn, 0.0, L);
   hipLaunchKernelGGL(fill_kernel, dim3(nblk(S * nn)), dim3(NT), 0, s, S * nn, 0.0, X);
   hipLaunchKernelGGL(fill_int_kernel, dim3(nblk(S)), dim3(NT), 0, s, S, 0, info);
