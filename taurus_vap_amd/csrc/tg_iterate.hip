@@ -193,18 +193,20 @@ chol_block_kernel(int n, int k0, int b, const double* __restrict__ A0, double* _
 // In steps of 32 columns, k of them done, with L_kk the factor of the diagonal block:
 // column t of Z = L_kk^-1 V is, for t past the block, row t of the panel of L (V: that of
 // A) and, for t up to it, column t of the rows k .. k + 31 of L^-1 (V: what the steps
-// before left there; the unit matrix in the block).  One rank-32 update M(r, c) -= Z_r . Z_c
+// before left there; L_kk^-1 itself in the block).  One rank-32 update M(r, c) -= Z_r . Z_c
 // then serves both: M(r, c), r >= c, is A's trailing matrix and M(r, c), r < k + 32,
 // the transposed unfinished rows c of L^-1, in the space above A's diagonal.
-// One wave factors the diagonal block in registers, a row per lane, while the others load
-// V; they solve a column of Z per thread (Z in LDS); all sixteen waves then update
-// 16 x 16 tiles on the matrix cores.
-// Bound by one CU and the chain of its steps (19 us each at order 40, half of it the square
-// roots and quotients of the diagonal block; 35 at 336, where the tiles are as long): orders
-// 40, 224, 336 take 38, 182, 387 us.  A launch per block and product, the block rows of
-// L^-1 on the second stream: 480 us at order 224 in a trace, HFB descent 15.3 -> 14.5 ms; at
-// 336 a descent takes the same 37.2 ms with either, with 50 launches fewer a step here.
-constexpr int CF_B = 32, CF_NW = 16, CF_TH = 64 * CF_NW, CF_NMAX = 512;
+// Wave 0 factors the diagonal block and inverts the factor in registers, lane i holding
+// row i of the block and lane 32 + i row i of the inverse; Z and the update are 16 x 16
+// tiles on the matrix cores, Z in LDS.  Wave 0 takes the next diagonal block's tiles
+// first and factors that block while the other waves update the rest.
+// Bound by one CU and the chain of its steps (15 us each, the square roots and quotients of
+// the diagonal block, where the tiles do not take longer): orders 40, 224, 336 take 37, 156,
+// 366 us, without the look-ahead 38, 182, 387 (the diagonal block and a thread per column
+// of Z in turn).  A launch per block and product, the block rows of L^-1 on the second
+// stream: 480 us at order 224 in a trace, HFB descent 15.3 -> 14.2 ms; at 336 a descent
+// takes the same 37 ms with either, with 50 launches fewer a step here.
+constexpr int CF_B = 32, CF_NW = 8, CF_TH = 64 * CF_NW, CF_NMAX = 512;
 inline int cf_zp(int n) { return (n + 31) / 32 * 32 + 16; }   // rows of Z 16 banks apart
 
 __device__ __forceinline__ double cf_readlane(double v, int lane) {
@@ -214,102 +216,99 @@ __device__ __forceinline__ double cf_readlane(double v, int lane) {
   return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
 }
 
+// Wave 0: factor of the diagonal block at k0 (b of its 32 rows inside the matrix, the
+// unit matrix past them), its inverse to Xd (Xd[i][j] = L_kk^-1(i, j), zero above the diagonal)
+__device__ __forceinline__ void cf_diagonal(const double* M, int n, int k0, int lane,
+                                            double (*Xd)[CF_B + 1], int& bad) {
+  const int b = min(CF_B, n - k0), i = lane & 31;
+  const bool up = lane >= CF_B;                  // a row of the inverse
+  const double* p = M + min(k0 + i, n - 1) + (long long)k0 * n;
+  double v[CF_B];
+#pragma unroll
+  for (int k = 0; k < CF_B; ++k) v[k] = p[min(k, b - 1) * n];
+  if (b < CF_B || up)
+#pragma unroll
+    for (int k = 0; k < CF_B; ++k)
+      if (up || max(i, k) >= b) v[k] = (i == k) ? 1.0 : 0.0;
+  double scale = 1.0;                            // 1 / L(i, i)
+#pragma unroll
+  for (int k = 0; k < CF_B; ++k) {
+    double d = cf_readlane(v[k], k);
+    if (!(d > 0.0)) {
+      if (bad == 0) bad = k0 + k + 1;
+      d = 1.0;
+    }
+    d = sqrt(d);
+    const double rd = 1.0 / d;
+    const double l = v[k] / d;                   // column k of L (lanes 0 .. 31)
+    if (i == k) scale = rd;
+    // rows past k: row i of the block less l_i l_j (j > k), of the inverse less
+    // l_i / d times row k as it stands (j <= k), which is scaled at the end
+    const double li = __shfl(l, i, 64);
+    const double ma = up ? 0.0 : -l, mb = (up && i > k) ? -li * rd : 0.0;
+#pragma unroll
+    for (int j = 0; j < CF_B; ++j)
+      v[j] = (j > k) ? fma(ma, cf_readlane(l, j), v[j])
+                     : fma(mb, cf_readlane(v[j], CF_B + k), v[j]);
+#pragma unroll
+    for (int j = 0; j < CF_B; ++j) asm volatile("" : "+v"(v[j]));   // here, not at their use
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if (up)
+#pragma unroll
+    for (int j = 0; j < CF_B; ++j) Xd[i][j] = v[j] * scale;
+}
+
 __global__ void __launch_bounds__(CF_TH)
 chol_inverse_kernel(int n, int zp, double* __restrict__ A0, double* __restrict__ X0,
                     int* __restrict__ info) {
   typedef double d4 __attribute__((ext_vector_type(4)));
   extern __shared__ double Z[];                  // CF_B rows of zp
-  __shared__ double Ld[CF_B][CF_B], Rd[CF_B];    // column k of L_kk at Ld[k], 1 / L_kk(k, k)
+  __shared__ double Xd[CF_B][CF_B + 1];
   const long long nn = (long long)n * n;
   double* M = A0 + blockIdx.x * nn;
   double* X = X0 + blockIdx.x * nn;
   const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int tv = t - 64;                         // vector of this thread (waves 1 ..)
+  const int lr = lane & 15, lk = lane >> 4;
   const int nb = (n + 15) / 16;
   int bad = 0;
-  for (int e = t; e < CF_B * zp; e += CF_TH) Z[e] = 0.0;    // columns past n stay zero
+  if (w == 0) cf_diagonal(M, n, 0, lane, Xd, bad);
   __syncthreads();
   for (int k0 = 0; k0 < n; k0 += CF_B) {
     const int b = min(CF_B, n - k0), k1 = (k0 + CF_B) / 16;
-    double v[CF_B];
-    if (w == 0) {
-      const int i = lane & 31;                   // the upper half repeats the rows
-      const double* p = M + min(k0 + i, n - 1) + (long long)k0 * n;
+    // Z = L_kk^-1 V, 32 x 16 at a time: lane: columns 16 tb + lr, rows lk + 4 q (+ 16)
+    for (int tb = w; tb < nb; tb += CF_NW) {
+      const bool diag = 16 * tb >= k0 && tb < k1;
+      const int c = 16 * tb + lr;
+      d4 z0 = {0.0, 0.0, 0.0, 0.0}, z1 = {0.0, 0.0, 0.0, 0.0};
+      if (diag) {
 #pragma unroll
-      for (int k = 0; k < CF_B; ++k) v[k] = p[min(k, b - 1) * n];
-      if (b < CF_B)                              // the unit matrix past the last row
-#pragma unroll
-        for (int k = 0; k < CF_B; ++k)
-          if (max(i, k) >= b) v[k] = (i == k) ? 1.0 : 0.0;
-#pragma unroll
-      for (int k = 0; k < CF_B; ++k) {
-        double d = cf_readlane(v[k], k);
-        if (!(d > 0.0)) {
-          if (bad == 0) bad = k0 + k + 1;
-          d = 1.0;
+        for (int q = 0; q < 4; ++q) {
+          z0[q] = Xd[lk + 4 * q][c - k0];
+          z1[q] = Xd[16 + lk + 4 * q][c - k0];
         }
-        d = sqrt(d);
-        const double l = (i == k) ? d : v[k] / d;
-        if (lane < CF_B) Ld[k][i] = l;           // (rows above k are not read)
-        if (lane == 0) Rd[k] = 1.0 / d;
+      } else {
+        const double* p = M + min(c, n - 1) + (long long)k0 * n;
+        double v[8];
 #pragma unroll
-        for (int j = k + 1; j < CF_B; ++j) v[j] = fma(-l, cf_readlane(l, j), v[j]);
+        for (int s = 0; s < 8; ++s) v[s] = p[(long long)min(4 * s + lk, b - 1) * n];
 #pragma unroll
-        for (int j = k + 1; j < CF_B; ++j) asm volatile("" : "+v"(v[j]));   // here, not at their use
-        __builtin_amdgcn_sched_barrier(0);
+        for (int s = 0; s < 8; ++s) {
+          const double vs = (4 * s + lk < b) ? v[s] : 0.0;
+          if (s < 4) z0 = __builtin_amdgcn_mfma_f64_16x16x4f64(Xd[lr][4 * s + lk], vs, z0, 0, 0, 0);
+          z1 = __builtin_amdgcn_mfma_f64_16x16x4f64(Xd[16 + lr][4 * s + lk], vs, z1, 0, 0, 0);
+        }
       }
-    } else if (tv < n) {
-      const double* p = M + tv + (long long)k0 * n;
 #pragma unroll
-      for (int k = 0; k < CF_B; ++k) v[k] = p[min(k, b - 1) * n];
-      if (b < CF_B)
-#pragma unroll
-        for (int k = 0; k < CF_B; ++k) v[k] = (k < b) ? v[k] : 0.0;
-      if (tv >= k0 && tv < k0 + CF_B)
-#pragma unroll
-        for (int k = 0; k < CF_B; ++k) v[k] = (tv - k0 == k) ? 1.0 : 0.0;
-    }
-    __syncthreads();
-    if (w > 0 && tv < n) {
-#pragma unroll
-      for (int k = 0; k < CF_B; ++k) {
-        const double z = v[k] * Rd[k];
-        Z[k * zp + tv] = z;
-#pragma unroll
-        for (int m = k + 1; m < CF_B; ++m) v[m] = fma(-Ld[k][m], z, v[m]);
-        __builtin_amdgcn_sched_barrier(0);
+      for (int q = 0; q < 4; ++q) {              // (rows past b, columns past n: zero)
+        const int r = lk + 4 * q;
+        Z[r * zp + c] = (r < b && c < n) ? z0[q] : 0.0;
+        Z[(16 + r) * zp + c] = (16 + r < b && c < n) ? z1[q] : 0.0;
       }
     }
     __syncthreads();
-    for (int e = t; e < CF_B * n; e += CF_TH) {
-      const int k = e % CF_B, c = e / CF_B;
-      if (k < b) X[(k0 + k) + (long long)c * n] = (c < k0 + CF_B) ? Z[k * zp + c] : 0.0;
-    }
-    // column blocks past this one; their rows up to it and from their diagonal on
-    const int lr = lane & 15, lk = lane >> 4;
-    int at = w, cb = k1, rb = 0;
-    auto next = [&]() -> bool {                  // this wave's next tile (rb, cb)
-      while (cb < nb && at >= k1 + nb - cb) {
-        at -= k1 + nb - cb;
-        ++cb;
-      }
-      if (cb >= nb) return false;
-      rb = at < k1 ? at : cb + at - k1;
-      at += CF_NW;
-      return true;
-    };
-    auto load = [&](double (&cv)[4]) {
-      const double* p = M + min(16 * rb + lr, n - 1);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) cv[q] = p[(long long)min(16 * cb + lk + 4 * q, n - 1) * n];
-    };
-    double cv[4], nv[4];
-    bool more = next();
-    if (more) load(cv);
-    while (more) {
+    auto update = [&](int rb, int cb, const double (&cv)[4]) {
       const int r0 = 16 * rb, c0 = 16 * cb;
-      more = next();
-      if (more) load(nv);
       d4 acc = {0.0, 0.0, 0.0, 0.0}, acc2 = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
       for (int s = 0; s < CF_B / 4; s += 2) {
@@ -323,7 +322,61 @@ chol_inverse_kernel(int n, int zp, double* __restrict__ A0, double* __restrict__
         const int c = c0 + lk + 4 * q;
         if (r0 + lr < n && c < n)
           M[r0 + lr + (long long)c * n] = (fresh ? 0.0 : cv[q]) - (acc[q] + acc2[q]);
-        cv[q] = nv[q];
+      }
+    };
+    auto load = [&](int rb, int cb, double (&cv)[4]) {
+      const double* p = M + min(16 * rb + lr, n - 1);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) cv[q] = p[(long long)min(16 * cb + lk + 4 * q, n - 1) * n];
+    };
+    // wave 0: the next diagonal block (its lower tiles), then its factor
+    if (w == 0 && k0 + CF_B < n) {
+      double ca[3][4];
+      const int last = min(k1 + 1, nb - 1);      // (one block column left: tile k1 alone)
+      load(k1, k1, ca[0]);
+      if (last > k1) {
+        load(last, k1, ca[1]);
+        load(last, last, ca[2]);
+      }
+      update(k1, k1, ca[0]);
+      if (last > k1) {
+        update(last, k1, ca[1]);
+        update(last, last, ca[2]);
+      }
+      __threadfence_block();
+    }
+    // Xd is read by every wave up to the barrier above, so the next one may be written
+    if (w == 0) {
+      if (k0 + CF_B < n) cf_diagonal(M, n, k0 + CF_B, lane, Xd, bad);
+    } else {
+      for (int e = t - 64; e < CF_B * n; e += CF_TH - 64) {
+        const int k = e % CF_B, c = e / CF_B;
+        if (k < b) X[(k0 + k) + (long long)c * n] = (c < k0 + CF_B) ? Z[k * zp + c] : 0.0;
+      }
+      // column blocks past this one; their rows up to it and from their diagonal on
+      int at = w - 1, cb = k1, rb = 0;
+      auto next = [&]() -> bool {                // this wave's next tile (rb, cb)
+        while (true) {
+          while (cb < nb && at >= k1 + nb - cb) {
+            at -= k1 + nb - cb;
+            ++cb;
+          }
+          if (cb >= nb) return false;
+          rb = at < k1 ? at : cb + at - k1;
+          at += CF_NW - 1;
+          if (cb > k1 + 1 || rb < k1 || rb > k1 + 1) return true;   // (wave 0's tiles)
+        }
+      };
+      double cv[4], nv[4];
+      bool more = next();
+      if (more) load(rb, cb, cv);
+      while (more) {
+        const int rc = rb, cc = cb;
+        more = next();
+        if (more) load(rb, cb, nv);
+        update(rc, cc, cv);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) cv[q] = nv[q];
       }
     }
     __syncthreads();
