@@ -35,6 +35,7 @@
 #include <algorithm>
 #include <atomic>
 #include <map>
+#include <memory>
 #include <new>
 #include <system_error>
 #include <thread>
@@ -529,6 +530,30 @@ Reduced reduce_class(const tg_ctx* c, bool pp, const std::vector<int>& el, const
   return R;
 }
 
+// f(g) for every class g, by up to eight threads; std::bad_alloc where one ran out of memory
+template <typename F>
+void parallel_classes(int nc, const F& f) {
+  std::atomic<int> next(0);
+  std::atomic<bool> nomem(false);
+  auto work = [&] {
+    try {
+      for (int g; (g = next.fetch_add(1)) < nc;) f(g);
+    } catch (const std::bad_alloc&) {      // nothing may leave a thread
+      nomem = true;
+    }
+  };
+  const int nt = std::max(1, std::min({8, (int)std::thread::hardware_concurrency(), nc}));
+  std::vector<std::thread> pool;
+  pool.reserve(nt);
+  try {
+    for (int k = 1; k < nt; ++k) pool.emplace_back(work);
+  } catch (const std::system_error&) {     // the threads there are take the work
+  }
+  work();
+  for (std::thread& th : pool) th.join();
+  if (nomem) throw std::bad_alloc();
+}
+
 int build_blocks(tg_ctx* c, int64_t ntb, const int16_t* abcd, const void* H2, int h2_bytes,
                  const int8_t* trperm) {
   const int n = c->n;
@@ -625,56 +650,50 @@ int build_blocks(tg_ctx* c, int64_t ntb, const int16_t* abcd, const void* H2, in
     Full& f = F[q];
     const int nc = (int)f.el.size();
     std::vector<Reduced> red(nc);
-    std::atomic<int> next(0);
-    std::atomic<bool> nomem(false);
-    auto work = [&] {
-      try {
-        for (int g; (g = next.fetch_add(1)) < nc;) {
-          if (c->w_fp32)
-            for (double& v : f.B[g]) v = (double)(float)v;
-          red[g] = reduce_class(c, q == 1, f.el[g], f.B[g]);
-          std::vector<double>().swap(f.B[g]);
-        }
-      } catch (const std::bad_alloc&) {      // nothing may leave a thread
-        nomem = true;
-      }
-    };
-    const int nt = std::max(1, std::min({8, (int)std::thread::hardware_concurrency(), nc}));
-    std::vector<std::thread> pool;
-    pool.reserve(nt);
-    try {
-      for (int k = 1; k < nt; ++k) pool.emplace_back(work);
-    } catch (const std::system_error&) {     // the threads there are take the work
-    }
-    work();
-    for (std::thread& th : pool) th.join();
-    if (nomem) throw std::bad_alloc();
+    parallel_classes(nc, [&](int g) {
+      if (c->w_fp32)
+        for (double& v : f.B[g]) v = (double)(float)v;
+      red[g] = reduce_class(c, q == 1, f.el[g], f.B[g]);
+      std::vector<double>().swap(f.B[g]);
+    });
 
     std::vector<GroupDesc> groups;
     std::vector<Orbit> orb;
-    std::vector<char> W;
+    std::vector<size_t> first(nc);      // group of each class's first block
+    size_t bytes = 0;
     int off = 0;
     for (int g = 0; g < nc; ++g) {
       for (Orbit& o : red[g].orb) {
         for (int i = 0; i < o.m; ++i) o.pos[i] += off;
         orb.push_back(o);
       }
+      first[g] = groups.size();
       const bool f32 = c->w_fp32 && !red[g].split;
-      size_t w0 = 0;
+      for (int sz : red[g].size) {
+        if (sz == 0) continue;
+        bytes = (bytes + 15) / 16 * 16;
+        groups.push_back({off, sz, (long long)bytes, f32 ? 1 : 0});
+        bytes += (size_t)sz * sz * (f32 ? sizeof(float) : sizeof(double));
+        off += sz;
+      }
+    }
+    // (not set to zero first: every byte that a kernel reads is written)
+    std::unique_ptr<char[]> W(new char[std::max<size_t>(bytes, 16)]);
+    parallel_classes(nc, [&](int g) {
+      size_t w0 = 0, k = first[g];
       for (int sz : red[g].size) {
         if (sz == 0) continue;
         const size_t cnt = (size_t)sz * sz;
-        const size_t at = (W.size() + 15) / 16 * 16;
-        W.resize(at + cnt * (f32 ? sizeof(float) : sizeof(double)));
-        for (size_t k = 0; k < cnt; ++k)
-          if (f32) reinterpret_cast<float*>(W.data() + at)[k] = (float)red[g].W[w0 + k];
-          else reinterpret_cast<double*>(W.data() + at)[k] = red[g].W[w0 + k];
-        groups.push_back({off, sz, (long long)at, f32 ? 1 : 0});
-        off += sz;
+        char* to = W.get() + groups[k].woff;
+        if (groups[k].fp32)
+          for (size_t e = 0; e < cnt; ++e) reinterpret_cast<float*>(to)[e] = (float)red[g].W[w0 + e];
+        else
+          std::copy_n(red[g].W.data() + w0, cnt, reinterpret_cast<double*>(to));
         w0 += cnt;
+        ++k;
       }
       red[g] = Reduced();
-    }
+    });
     ch.npos = off;
     ch.ngroups = (int)groups.size();
     ch.norb = (int)orb.size();
@@ -709,7 +728,7 @@ int build_blocks(tg_ctx* c, int64_t ntb, const int16_t* abcd, const void* H2, in
     };
     TG_TRY(up(ch.d_orb, orb.data(), sizeof(Orbit) * orb.size()));
     TG_TRY(up(ch.d_groups, groups.data(), sizeof(GroupDesc) * groups.size()));
-    TG_TRY(up(ch.d_W, W.data(), W.size()));
+    TG_TRY(up(ch.d_W, W.get(), bytes));
     TG_TRY(up(ch.d_tile_group, tg.data(), sizeof(int) * tg.size()));
     TG_TRY(up(ch.d_tile_n0, tn.data(), sizeof(int) * tn.size()));
   }
