@@ -229,6 +229,8 @@ struct tg_ctx {
   hipStream_t stream = nullptr;
   hipStream_t stream2 = nullptr;                  // overlaps, concurrent with the Thouless chain
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+  void* stage = nullptr;                          // pinned memory for results on their way out
+  size_t stage_bytes = 0;
   hipStream_t stream3 = nullptr;                  // the pp contraction beside the ph one
   hipEvent_t ev_fork3 = nullptr, ev_join3 = nullptr;
   // basis

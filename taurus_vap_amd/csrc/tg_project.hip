@@ -1594,6 +1594,23 @@ void assign_angles(tg_ctx* c, bool conj) {
   c->A = (int)c->phip.size();
 }
 
+// The context's pinned memory, at least `bytes` of it (nullptr: none to be had)
+constexpr size_t TG_STAGE_BYTES = 2 << 20;
+char* stage_memory(tg_ctx* c, size_t bytes) {
+  if (c->stage_bytes < bytes) {
+    if (c->stage) (void)hipHostFree(c->stage);
+    c->stage = nullptr;
+    c->stage_bytes = 0;
+    if (hipHostMalloc(&c->stage, bytes, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      c->stage = nullptr;
+      return nullptr;
+    }
+    c->stage_bytes = bytes;
+  }
+  return static_cast<char*>(c->stage);
+}
+
 int fetch_results(tg_ctx* c, int state, double* scal, double* pA, double* pH, double* pAH,
                   double* H20v, double* imag) {
   const int n = c->n;
@@ -1602,21 +1619,47 @@ int fetch_results(tg_ctx* c, int state, double* scal, double* pA, double* pH, do
     tg_set_error("results: state index out of range");
     return TG_E_ARG;
   }
-  TG_HIP(hipStreamSynchronize(c->stream));
   const RunPlan P = make_plan(c);
   const cplx* d_out = c->d_out.as<cplx>() + (size_t)state * P.outs;
-  const cplx* d_pnp = P.d_pnp + 8 * (size_t)state;
-  const double* d_imag = P.d_imag + (size_t)state * P.is;
-  if (scal) TG_HIP(hipMemcpy(scal, d_pnp, sizeof(cplx) * 7, hipMemcpyDeviceToHost));
-  if (pA) TG_HIP(hipMemcpy(pA, d_out, sizeof(cplx) * nn, hipMemcpyDeviceToHost));
-  if (pH) TG_HIP(hipMemcpy(pH, d_out + nn, sizeof(cplx) * nn, hipMemcpyDeviceToHost));
-  if (pAH) TG_HIP(hipMemcpy(pAH, d_out + 2 * nn, sizeof(cplx) * nn, hipMemcpyDeviceToHost));
-  if (H20v)
-    TG_HIP(hipMemcpy(H20v, reinterpret_cast<const double*>(d_out + 3 * nn), sizeof(double) * nn,
-                     hipMemcpyDeviceToHost));
   const int nb = (int)((nn + NT - 1) / NT);
+  struct Part {
+    void* to;
+    const void* from;
+    size_t bytes;
+  };
   std::vector<double> im(nb);
-  TG_HIP(hipMemcpy(im.data(), d_imag, sizeof(double) * nb, hipMemcpyDeviceToHost));
+  const Part parts[6] = {{scal, P.d_pnp + 8 * (size_t)state, sizeof(cplx) * 7},
+                         {im.data(), P.d_imag + (size_t)state * P.is, sizeof(double) * nb},
+                         {pA, d_out, sizeof(cplx) * nn},
+                         {pH, d_out + nn, sizeof(cplx) * nn},
+                         {pAH, d_out + 2 * nn, sizeof(cplx) * nn},
+                         {H20v, d_out + 3 * nn, sizeof(double) * nn}};
+  size_t total = 0;
+  for (const Part& q : parts)
+    if (q.to) total += q.bytes;
+  // A copy to pageable memory is waited for by itself, 40 us and more each: up to
+  // TG_STAGE_BYTES the parts go to pinned memory, with one wait, and from there
+  // (projection of 24 states 0.51 -> 0.41 ms, of 140 states, 1.1 MB, 1.76 -> 1.70).
+  // Larger ones gain as much by the runtime's own pipelining as by this (224 states,
+  // 2.8 MB: 2.98 and 3.0; 336 states 16.3 and 16.3).
+  char* stage = total <= TG_STAGE_BYTES ? stage_memory(c, total) : nullptr;
+  if (!stage) TG_HIP(hipStreamSynchronize(c->stream));
+  size_t at = 0;
+  for (const Part& q : parts) {
+    if (!q.to) continue;
+    if (stage) TG_HIP(hipMemcpyAsync(stage + at, q.from, q.bytes, hipMemcpyDeviceToHost, c->stream));
+    else TG_HIP(hipMemcpy(q.to, q.from, q.bytes, hipMemcpyDeviceToHost));
+    at += q.bytes;
+  }
+  if (stage) {
+    TG_HIP(hipStreamSynchronize(c->stream));
+    at = 0;
+    for (const Part& q : parts) {
+      if (!q.to) continue;
+      std::memcpy(q.to, stage + at, q.bytes);
+      at += q.bytes;
+    }
+  }
   double mx = -INFINITY;
   for (double v : im) mx = std::max(mx, v);
   if (imag) *imag = mx;
@@ -1804,6 +1847,7 @@ int tg_finalize(tg_ctx* c) {
       b->release();
   if (c->stream2) (void)hipStreamSynchronize(c->stream2);
   if (c->stream3) (void)hipStreamSynchronize(c->stream3);
+  if (c->stage) (void)hipHostFree(c->stage);
   if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
   if (c->ev_join) (void)hipEventDestroy(c->ev_join);
   if (c->ev_fork3) (void)hipEventDestroy(c->ev_fork3);
