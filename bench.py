@@ -53,17 +53,20 @@ def log(msg):
     print("[bench] " + msg, file=sys.stderr, flush=True)
 
 
-def algorithmic_flops(ctx_info, n, A, nb):
+def algorithmic_flops(ctx_info, n, A, nb, fp32):
     """Algorithmic FP64 flops per step (one projection of all A angles) of the
     timed kernels (real flops; complex multiply-add = 8, real x complex = 4)."""
+    # the blocks split by the interaction's symmetries, when the elements are kept in
+    # FP32, leave a third (ph) and two thirds (pp) of the multiply-adds
+    ph, pp = (1.0 / 3.0, 2.0 / 3.0) if fp32 else (1.0, 1.0)
     return {
-        "kernel:grouped_ph": 4.0 * ctx_info["wph"] * A,
-        "kernel:grouped_pp": 4.0 * ctx_info["wpp"] * 2 * A,
+        "kernel:grouped_ph": 4.0 * ctx_info["wph"] * A * ph,
+        "kernel:grouped_pp": 4.0 * ctx_info["wpp"] * 2 * A * pp,
         "kernel:gj_inverse": 8.0 * n ** 3 * A,
         "kernel:pfaffian": (4.0 / 3.0) * nb ** 3 * A,
-        # complex batched GEMMs of the loop body on the main stream: A_phi (n^3),
-        # the two H20 products over the inner dimension 2n and the one over n
-        "kernel:zgemm": 8.0 * A * 6 * n ** 3,
+        # complex batched GEMMs of the loop body on the main stream: A_phi (skew, half
+        # of n^3) and the five H20 products
+        "kernel:zgemm": 8.0 * A * 5.5 * n ** 3,
         # the reduced overlap's angle-independent parts of K on the second stream:
         # three real nb x nb x nb products per state (the per-angle combination is
         # element-wise)
@@ -451,7 +454,7 @@ def main():
     # either stream
     n, A, nb = main_run["n"], main_run["A"], main_run["nb"]
     M = int(fix["Mphip"])
-    fl = algorithmic_flops(sizes, n, A, nb)
+    fl = algorithmic_flops(sizes, n, A, nb, fp32)
     kern = {k: v for k, v in main_run["timing"].items() if k.startswith("kernel:") and v[1] > 0}
     roofline = None
     by_kernel = {}
