@@ -92,7 +92,9 @@ enum TgOp { OP_N = 0, OP_T = 1, OP_C = 2 };
 // What the complex products do as they store C, in place of passes of their own.
 struct GemmEpi {
   int skew = 0;                  // C is skew: tiles on and below the diagonal, -C^T above
-                                 // it, zero on it (M == N, beta = 0)
+                                 // it, zero on it (M == N, beta = 0) ...
+  const double* exact = nullptr; // ... where exact[b / divExact] != 0 for element b (device;
+  int divExact = 1;              // null: everywhere), whole elsewhere
   int conj = 0;                  // conj(C)
   const double* add = nullptr;   // + a real matrix, element b's at add + (b / divAdd) * sAdd
   long long sAdd = 0;            // (leading dimension ldc)

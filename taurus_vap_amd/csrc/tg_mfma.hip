@@ -43,7 +43,9 @@ constexpr int XCDS = 8;
 // Rows and columns past the edge repeat the last one and are not stored; k past the
 // end is masked in the last chunk only.
 // A skew product (GemmEpi) forms the tiles that reach the diagonal or lie below it, 44 of
-// 77 of 48 x 32 at order 336, and stores each element at its transposed place as well.
+// 77 of 48 x 32 at order 336, and stores each element at its transposed place as well.  The
+// tiles above the diagonal follow those of all elements: they end at once, or, where the
+// element is not skew to rounding (GemmEpi::exact), form the rest of its product.
 // Complex x complex is three real products (Gauss): cr = sum Ar Br, ci = sum Ai Bi,
 // c3 = sum (Ar + Ai)(Br + Bi); C = (cr - ci, c3 - cr - ci).
 // Bound by the matrix cores, the load latency covered by the steps in flight and 2-4
@@ -62,20 +64,36 @@ __global__ void __launch_bounds__(256, OCC)
 mfma_batched_kernel(int M, int N, int K, cplx alpha, const TA* __restrict__ A, int lda,
                     long long sA, const TB* __restrict__ B, int ldb, long long sB, cplx beta,
                     int use_beta, cplx* __restrict__ C, int ldc, long long sC, int batch,
-                    int tiles_m, int tiles, int per, int divA, int divB, GemmEpi ep) {
+                    int tiles_m, int tiles, int upper, int per, int divA, int divB, GemmEpi ep) {
   constexpr bool CA = IsC<TA>::v, CB = IsC<TB>::v, CC = CA && CB;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // the batch * tiles (element, tile) pairs are cut into 8 contiguous runs, one per XCD
   // (workgroup ids are dealt round-robin to the XCDs), so the tiles of one element share
   // an L2 and every XCD gets the same number
-  const unsigned g = (blockIdx.x % XCDS * (unsigned)per + blockIdx.x / XCDS) * 4 + w;
-  if (g >= (unsigned)batch * (unsigned)tiles) return;
-  const int b = (int)(g / (unsigned)tiles), tile = (int)(g - (unsigned)b * (unsigned)tiles);
-  int ti = tile % tiles_m, tj = tile / tiles_m;
-  if (ep.skew) {        // the tiles that reach the diagonal or lie below it, by columns
-    ti = tile;
-    for (tj = 0; ti >= tiles_m - tj * TN / TM; ++tj) ti -= tiles_m - tj * TN / TM;
-    ti += tj * TN / TM;
+  const unsigned first = XCDS * (unsigned)per;    // workgroups of the tiles counted by `tiles`
+  int b, ti, tj;
+  bool mirror = ep.skew != 0;
+  if (blockIdx.x < first) {
+    const unsigned g = (blockIdx.x % XCDS * (unsigned)per + blockIdx.x / XCDS) * 4 + w;
+    if (g >= (unsigned)batch * (unsigned)tiles) return;
+    b = (int)(g / (unsigned)tiles);
+    const int tile = (int)(g - (unsigned)b * (unsigned)tiles);
+    ti = tile % tiles_m;
+    tj = tile / tiles_m;
+    if (ep.skew) {        // the tiles that reach the diagonal or lie below it, by columns
+      ti = tile;
+      for (tj = 0; ti >= tiles_m - tj * TN / TM; ++tj) ti -= tiles_m - tj * TN / TM;
+      ti += tj * TN / TM;
+      if (ep.exact) mirror = ep.exact[b / ep.divExact] != 0.0;
+    }
+  } else {                // those above it, of products that are not skew to rounding
+    const unsigned g = (blockIdx.x - first) * 4 + w;
+    if (g >= (unsigned)batch * (unsigned)upper) return;
+    b = (int)(g / (unsigned)upper);
+    if (ep.exact[b / ep.divExact] != 0.0) return;
+    mirror = false;
+    ti = (int)(g - (unsigned)b * (unsigned)upper);
+    for (tj = 0; ti >= tj * TN / TM; ++tj) ti -= tj * TN / TM;
   }
   const int m0 = ti * 16 * TM, n0 = tj * 16 * TN;
   const int lr = lane & 15, lk = lane >> 4;
@@ -178,7 +196,7 @@ mfma_batched_kernel(int M, int N, int K, cplx alpha, const TA* __restrict__ A, i
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int gj = n0 + 16 * y + lk + 4 * r;
-        if (gj >= N || (ep.skew && gi < gj)) continue;
+        if (gj >= N || (mirror && gi < gj)) continue;
         cplx* cp = Cb + gi + (long long)gj * ldc;
         cplx p;
         if constexpr (CC)
@@ -189,7 +207,7 @@ mfma_batched_kernel(int M, int N, int K, cplx alpha, const TA* __restrict__ A, i
         if (use_beta) v = cadd(v, cmul(beta, *cp));
         if (ep.conj) v.y = -v.y;
         if (add) v.x += add[gi + (long long)gj * ldc];
-        if (ep.skew) {
+        if (mirror) {
           if (gi == gj) v = cmk(0.0, 0.0);
           else Cb[gj + (long long)gi * ldc] = cmk(-v.x, -v.y);
         }
@@ -443,7 +461,7 @@ int launch_batched(hipStream_t s, int M, int N, int K, cplx alpha, const TA* A, 
                    cplx* C, int ldc, long long sC, int batch, int divA, int divB,
                    const GemmEpi& ep) {
   const int tiles_m = (M + 16 * TM - 1) / (16 * TM), tiles_n = (N + 16 * TN - 1) / (16 * TN);
-  int tiles = tiles_m * tiles_n;
+  int tiles = tiles_m * tiles_n, upper = 0;
   if (ep.skew) {
     if (M != N || use_beta) {
       tg_set_error("mfma gemm: a skew product is square and written, not added");
@@ -451,9 +469,11 @@ int launch_batched(hipStream_t s, int M, int N, int K, cplx alpha, const TA* A, 
     }
     tiles = 0;
     for (int j = 0; j < tiles_n; ++j) tiles += tiles_m - j * TN / TM;
+    if (ep.exact) upper = tiles_m * tiles_n - tiles;
   }
   const long long wgs = ((long long)batch * tiles + 3) / 4;      // four waves, a tile each
-  const long long per = (wgs + XCDS - 1) / XCDS, grid = (long long)XCDS * per;
+  const long long per = (wgs + XCDS - 1) / XCDS;
+  const long long grid = (long long)XCDS * per + ((long long)batch * upper + 3) / 4;
   if (grid > 0x1fffffffLL) {          // tile numbers in 32 bits
     tg_set_error("mfma gemm: grid too large");
     return TG_E_ARG;
@@ -461,7 +481,7 @@ int launch_batched(hipStream_t s, int M, int N, int K, cplx alpha, const TA* A, 
   if (grid == 0) return TG_OK;
   hipLaunchKernelGGL((mfma_batched_kernel<TA, TB, OPA, OPB, TM, TN, KS, OCC>), dim3((unsigned)grid),
                      dim3(256), 0, s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, use_beta, C, ldc,
-                     sC, batch, tiles_m, tiles, (int)per, divA, divB, ep);
+                     sC, batch, tiles_m, tiles, upper, (int)per, divA, divB, ep);
   TG_HIP(hipGetLastError());
   return TG_OK;
 }

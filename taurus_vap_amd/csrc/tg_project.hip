@@ -83,11 +83,19 @@ inline unsigned nblk(long long tot) { return (unsigned)((tot + NT - 1) / NT); }
 // of state (b0 + a) / A.  A thread takes one element for UV_AG consecutive
 // items, so the real matrices (two of them read transposed) are loaded once per
 // state rather than once per item.
+//
+// exact[s] becomes 0 where state s is not a Bogoliubov transformation to rounding, that is
+// where an element of U^T U + V^T V - 1 or V^T U + (V^T U)^T exceeds TG_EXACT_TOL.
+// A_phi and the pairing tensors of such a state are not skew, and what takes half of them
+// for the whole would change the results by a hundred to a thousand times its error (80
+// angles, noise of 1e-8 on U and V: 7e-7 on H20).  States read, evolved or built by this library
+// stay below 1e-14 (seeds 2e-15, after 400 steps 6e-15).
+constexpr double TG_EXACT_TOL = 2.8e-14;
 constexpr int UV_AG = 16;
 __global__ void build_uv_phi_kernel(int n, int na, long long b0, int A, int S,
                                     const double* __restrict__ R6, const cplx* __restrict__ ph,
                                     cplx* __restrict__ Uphi, cplx* __restrict__ Vphi,
-                                    long long stride) {
+                                    long long stride, double* __restrict__ exact) {
   const long long nn = (long long)n * n;
   const long long r = (long long)blockIdx.x * NT + threadIdx.x;
   if (r >= nn) return;
@@ -108,6 +116,10 @@ __global__ void build_uv_phi_kernel(int n, int na, long long b0, int A, int S,
       kp = Kp + Lp; km = Kp - Lp; kn = Kn + Ln; knm = Kn - Ln;
       mp = Mp + Mpt; mpm = Mp - Mpt; mn = Mn + Mnt; mnm = Mn - Mnt;
       cur = st;
+      // (one item of a state is its first angle; every thread that stores, stores the same)
+      if (ang == 0 && !(fabs(kp + kn - (i == j ? 1.0 : 0.0)) <= TG_EXACT_TOL &&
+                        fabs(mp + mn) <= TG_EXACT_TOL))
+        exact[st] = 0.0;
     }
     const cplx ep = ph[2 * ang], en = ph[2 * ang + 1];
     cplx u, v;
@@ -145,7 +157,8 @@ __global__ void add_h1_kernel(long long nn, int na, const cplx* __restrict__ H1,
 // A workgroup sums the elements (i, j) of one band of 32 rows i of one angle,
 // 32 columns j at a time; rho(j, i) comes from a 32 x 32 tile of rho staged in
 // LDS, so every global read is coalesced; kLR, kRL and DeltaLR are skew, so the
-// elements below the diagonal count twice.  225 angles of
+// elements below the diagonal count twice, but for a state that is not exact (item a0 + a is
+// of state (a0 + a) / A), whose kLR and kRL are read whole.  225 angles of
 // order 336 0.33 ms (whole matrices 0.42).  part[(a * bands + band) * 9 + k];
 // traces_sum_kernel adds the bands.
 constexpr int TRT = 32;
@@ -153,7 +166,7 @@ __global__ void __launch_bounds__(NT)
 traces_kernel(int n, const cplx* __restrict__ H1, const cplx* __restrict__ rho,
               const cplx* __restrict__ kLR, const cplx* __restrict__ kRL,
               const cplx* __restrict__ G, const cplx* __restrict__ dLR, long long stride,
-              cplx* __restrict__ part) {
+              long long a0, int A, const double* __restrict__ exact, cplx* __restrict__ part) {
   const int band = blockIdx.x, bands = gridDim.x;
   const long long a = blockIdx.y;
   const int i0 = band * TRT, h = n / 2;
@@ -168,7 +181,7 @@ traces_kernel(int n, const cplx* __restrict__ H1, const cplx* __restrict__ rho,
 #pragma unroll
   for (int k = 0; k < 9; ++k) acc[k] = cmk(0.0, 0.0);
   const int i = i0 + tx;
-  const bool pi = i < h;
+  const bool pi = i < h, half = exact[(a0 + a) / A] != 0.0;
   for (int j0 = 0; j0 < n; j0 += TRT) {
     for (int ii = ty; ii < TRT; ii += NT / TRT) {
       const int jr = j0 + tx, ir = i0 + ii;
@@ -186,7 +199,7 @@ traces_kernel(int n, const cplx* __restrict__ H1, const cplx* __restrict__ rho,
         if (pi == pj) cfma(acc[pi ? 2 : 4], r_[idx], rji);
         cfma(acc[6], H1[idx], rji);
         cfma(acc[7], g_[idx], rji);
-        if (i > j) {
+        if (i > j || !half) {
           const cplx k = kr[idx];
           if (pi == pj) cfma(acc[pi ? 3 : 5], k, kl[idx]);
           cfma(acc[8], dl[idx], k);
@@ -194,9 +207,10 @@ traces_kernel(int n, const cplx* __restrict__ H1, const cplx* __restrict__ rho,
       }
     __syncthreads();
   }
-  acc[3] = cscale(acc[3], 2.0);
-  acc[5] = cscale(acc[5], 2.0);
-  acc[8] = cscale(acc[8], 2.0);
+  const double twice = half ? 2.0 : 1.0;
+  acc[3] = cscale(acc[3], twice);
+  acc[5] = cscale(acc[5], twice);
+  acc[8] = cscale(acc[8], twice);
   // sums of the waves by lane moves, one barrier (a tree in LDS per trace, 90 barriers: 49
   // angles of order 24 12.6 -> 9.4 us, 121 of order 140 60 -> 56)
   __shared__ cplx red[NT / 64][9];
@@ -489,12 +503,13 @@ gauge_matrices_kernel(int n, int na, const cplx* __restrict__ f120, const double
     if (q == x && in[x]) pH0[st * os + idx[x]] = csub(tot[x][e], tot[nt - 1 - x][tr]);
 }
 
-// calculate_projected_H20 (:729-759); imag[block] = max Im over the block
+// calculate_projected_H20 (:729-759); imag[block] = max Im over the block.  The last reader
+// of a projection's matrices, it sets exact[s] for the next one.
 __global__ void __launch_bounds__(NT)
 projected_h20_kernel(int n, const cplx* __restrict__ pnp0, const cplx* __restrict__ pA0,
                      const cplx* __restrict__ pH0, const cplx* __restrict__ pAH0,
                      double* __restrict__ H20v0, double* __restrict__ imag0, long long os,
-                     long long is) {
+                     long long is, double* __restrict__ exact) {
   // state blockIdx.y: sums at pnp + 8 s, matrices at + s * os (complex), imag at + s * is
   const long long st = blockIdx.y;
   const cplx* pnp = pnp0 + 8 * st;
@@ -505,6 +520,7 @@ projected_h20_kernel(int n, const cplx* __restrict__ pnp0, const cplx* __restric
   double* imag = imag0 + st * is;
   const long long nn = (long long)n * n;
   long long idx = (long long)blockIdx.x * NT + threadIdx.x;
+  if (idx == 0) exact[st] = 1.0;
   const cplx over = pnp[0];
   const cplx oinv = cinv(over);
   const cplx ener = cmul(pnp[1], oinv);
@@ -840,6 +856,7 @@ struct RunPlan {
   cplx *d_ph, *d_tr, *d_over, *d_ener, *d_f12, *d_pnp, *d_pre, *d_det, *d_phase, *d_w, *d_pari;
   cplx* d_trp;   // per-band partial traces of one chunk
   double *d_logabs, *d_imag, *d_mult;
+  double* d_exact;                          // per state, 1 between projections
   int *d_info, *d_zero, *d_perm;
   double *d_T, *d_sg, *d_ovac, *d_vou;      // overlap set-up of state 0 (state s at + s * os)
   cplx* d_pre0;                             // state s at + s * os / 2
@@ -884,11 +901,11 @@ RunPlan make_plan(tg_ctx* c) {
   P.work_bytes = sizeof(cplx) * (wsz + 2 * (size_t)B * nn);
   // scalars: ph (2A) | traces (9B) | over (B) | ener (B) | f12 (2B) | pnp (8S) | pre (B)
   //          | det (B) | phase (B) | w (A) | pari (B) | logabs (B doubles)
-  //          | imag (S * is doubles) | mult (A doubles) | pad to 16 bytes
+  //          | imag (S * is doubles) | mult (A doubles) | exact (S doubles) | pad to 16 bytes
   //          | partial traces (9 * chunk * bands)
   const size_t bands = (n + TRT - 1) / TRT;
   P.scal_bytes = sizeof(cplx) * (3 * (size_t)A + 17 * (size_t)B + 8 * (size_t)S) +
-                 sizeof(double) * ((size_t)B + (size_t)S * P.is + A + 1) +
+                 sizeof(double) * ((size_t)B + (size_t)S * P.is + A + S + 1) +
                  sizeof(cplx) * 9 * (size_t)P.chunk * bands;
   P.int_bytes = sizeof(int) * ((size_t)B * (n + 2) + 8);
   // overlap set-up per state: T (n) | sg (n) | ovac (2) | pre0 (cplx) | v/u (n)
@@ -932,8 +949,9 @@ RunPlan make_plan(tg_ctx* c) {
   P.d_logabs = reinterpret_cast<double*>(P.d_pari + B);
   P.d_imag = P.d_logabs + B;
   P.d_mult = P.d_imag + (size_t)S * P.is;
+  P.d_exact = P.d_mult + A;
   {
-    const size_t end = (size_t)((const char*)(P.d_mult + A) - (const char*)c->d_scal.p);
+    const size_t end = (size_t)((const char*)(P.d_exact + S) - (const char*)c->d_scal.p);
     P.d_trp = reinterpret_cast<cplx*>((char*)c->d_scal.p + ((end + 15) / 16) * 16);
   }
   P.d_info = c->d_int.as<int>();
@@ -1013,10 +1031,12 @@ int project_upload(tg_ctx* c) {
     hph[2 * a + 1] = cmk(cos(c->phin[a]), sin(c->phin[a]));
     hw[a] = c->weight[a];
   }
+  std::vector<double> hm(c->mult);           // | exact: 1 until a projection finds it is not
+  hm.insert(hm.end(), S, 1.0);
   std::vector<double> ovl = overlap_setup(c, P);
   TG_HIP(hipMemcpyAsync(P.d_ph, hph.data(), sizeof(cplx) * 2 * A, hipMemcpyHostToDevice, s));
   TG_HIP(hipMemcpyAsync(P.d_w, hw.data(), sizeof(cplx) * A, hipMemcpyHostToDevice, s));
-  TG_HIP(hipMemcpyAsync(P.d_mult, c->mult.data(), sizeof(double) * A, hipMemcpyHostToDevice, s));
+  TG_HIP(hipMemcpyAsync(P.d_mult, hm.data(), sizeof(double) * hm.size(), hipMemcpyHostToDevice, s));
   TG_HIP(hipMemcpyAsync(P.d_T, ovl.data(), sizeof(double) * ovl.size(), hipMemcpyHostToDevice, s));
   TG_HIP(hipStreamSynchronize(s));   // host vectors go out of scope
 
@@ -1279,7 +1299,7 @@ int project_run(tg_ctx* c) {
       ScopedTiming tm(c, "thouless_inverse");
       hipLaunchKernelGGL(build_uv_phi_kernel, dim3(nblk(nn), (na + UV_AG - 1) / UV_AG), dim3(NT), 0,
                          s, n, na, (long long)a0,
-                         A, S, R6, P.d_ph, Uphi, Vphi, nn);
+                         A, S, R6, P.d_ph, Uphi, Vphi, nn, P.d_exact);
       TG_HIP(hipGetLastError());
       ScopedTiming tk(c, "kernel:gj_inverse");
       TG_TRY(batched_inverse(s, n, Uphi, n, nn, na, P.d_det, P.d_info, P.d_perm));
@@ -1291,11 +1311,13 @@ int project_run(tg_ctx* c) {
       ScopedTiming tm(c, "gemm");
       const double* Uc = U + (size_t)(a0 / A) * nn;
       const double* Vc = V + (size_t)(a0 / A) * nn;
-      // A_phi = conj(V_phi U_phi^-1) and the pairing tensors are skew, so half of each
-      // product gives it; U and V are added, and A_phi conjugated, as the products are
-      // stored (225 angles, 336 states: 17.6 -> 16.8 ms a projection)
+      // A_phi = conj(V_phi U_phi^-1) and the pairing tensors of an exact state are skew, so
+      // half of each product gives it; U and V are added, and A_phi conjugated, as the
+      // products are stored (225 angles, 336 states: 17.6 -> 16.8 ms a projection)
       GemmEpi skew, aphi;
       skew.skew = aphi.skew = aphi.conj = 1;
+      skew.exact = aphi.exact = P.d_exact + a0 / A;
+      skew.divExact = aphi.divExact = S == 1 ? na : A;
       auto plus = [&](const double* W) {
         GemmEpi e;
         e.add = W;
@@ -1346,7 +1368,7 @@ int project_run(tg_ctx* c) {
     {
       const int bands = (n + TRT - 1) / TRT;
       hipLaunchKernelGGL(traces_kernel, dim3(bands, na), dim3(NT), 0, s, n, c->d_H1.as<cplx>(), rho,
-                         kLR, kRL, G, dLR, nn, P.d_trp);
+                         kLR, kRL, G, dLR, nn, (long long)a0, A, P.d_exact, P.d_trp);
       hipLaunchKernelGGL(traces_sum_kernel, dim3(nblk(9LL * na)), dim3(NT), 0, s, na, bands, P.d_trp,
                          P.d_tr + 9 * (size_t)a0);
     }
@@ -1387,7 +1409,7 @@ int project_run(tg_ctx* c) {
   hipLaunchKernelGGL(gauge_matrices_kernel, dim3(gt * (gt + 1) / 2, S), dim3(GMT * GMT * GMQ), 0, s, n,
                      A, P.d_f12, P.d_mult, Akeep, Gkeep, nn, pA, pH, pAH, P.outs);
   hipLaunchKernelGGL(projected_h20_kernel, dim3(nblk(nn), S), dim3(NT), 0, s, n, P.d_pnp, pA, pH,
-                     pAH, H20v, P.d_imag, P.outs, P.is);
+                     pAH, H20v, P.d_imag, P.outs, P.is, P.d_exact);
   TG_HIP(hipGetLastError());
   if (c->grad_on) {
     // Z buffers: [Zi | Zim1 | lambda | partial sums], S states each; the new Z
