@@ -30,14 +30,16 @@ template <> __device__ inline double zero_v<double>() { return 0.0; }
 template <> __device__ inline cplx zero_v<cplx>() { return cmk(0.0, 0.0); }
 
 constexpr int XCDS = 8;
+constexpr int KP = 2;   // k of a lane that follow each other (mfma_batched_kernel)
 
 // One (TM x 16) x (TN x 16) tile of C per wave, operands straight from global memory
 // (L1 / L2) into the matrix-core registers: a lane loads the element of op(A) and op(B)
 // that it feeds, so there is no LDS, no barrier and no wave waits for another.  KS steps
 // of 4 k each are in flight: a step's operands are loaded as soon as its registers are
 // free, KS - 1 steps of products before they are needed.  Lane quarter lk
-// takes k = k0 + KS lk + s in step s (any assignment serves, the same for both operands):
-// an operand contiguous in k is then read as whole runs of 4 KS elements.
+// takes k = 4 KP (t / KP) + KP lk + t mod KP in step t, whatever KS is, so every tile shape adds
+// the products of an element in the same order: the tuner's choice, a matter of timing,
+// leaves the bits alone.
 // The products are formed transposed (MFMA rows = columns of C), so that lanes 0..15
 // hold 16 consecutive rows of a column and loads and stores of C are unit-stride.
 // Rows and columns past the edge repeat the last one and are not stored; k past the
@@ -100,17 +102,17 @@ mfma_batched_kernel(int M, int N, int K, cplx alpha, const TA* __restrict__ A, i
   const TA* Ab = A + (long long)(b / divA) * sA;
   const TB* Bb = B + (long long)(b / divB) * sB;
   constexpr bool AN = OPA == OP_N, BN = OPB == OP_N;
-  // element offsets of the lane's rows / columns at k = KS lk (32 bits: one matrix)
+  // element offsets of the lane's rows / columns at k = KP lk (32 bits: one matrix)
   unsigned ao[TM], bo[TN];
 #pragma unroll
   for (int x = 0; x < TM; ++x) {
     const unsigned i = min(m0 + 16 * x + lr, M - 1);
-    ao[x] = AN ? i + KS * lk * (unsigned)lda : KS * lk + i * (unsigned)lda;
+    ao[x] = AN ? i + KP * lk * (unsigned)lda : KP * lk + i * (unsigned)lda;
   }
 #pragma unroll
   for (int y = 0; y < TN; ++y) {
     const unsigned j = min(n0 + 16 * y + lr, N - 1);
-    bo[y] = BN ? KS * lk + j * (unsigned)ldb : j + KS * lk * (unsigned)ldb;
+    bo[y] = BN ? KP * lk + j * (unsigned)ldb : j + KP * lk * (unsigned)ldb;
   }
   const long long ka = AN ? lda : 1, kb = BN ? 1 : ldb;   // elements per k
   d4 cr[TM][TN], ci[TM][TN], c3[CC ? TM : 1][CC ? TN : 1];
@@ -124,10 +126,11 @@ mfma_batched_kernel(int M, int N, int K, cplx alpha, const TA* __restrict__ A, i
     }
   TA va[KS][TM];
   TB vb[KS][TN];
-  auto load = [&](int s, int k0, bool mask) {
-    const TA* pa = Ab + (k0 + s) * ka;
-    const TB* pb = Bb + (k0 + s) * kb;
-    const bool in = !mask || k0 + KS * lk + s < K;
+  auto load = [&](int s, int t, bool mask) {                // step t to the registers s
+    const int k = t / KP * (4 * KP) + t % KP;
+    const TA* pa = Ab + k * ka;
+    const TB* pb = Bb + k * kb;
+    const bool in = !mask || k + KP * lk < K;
 #pragma unroll
     for (int x = 0; x < TM; ++x) {
       if (mask) va[s][x] = zero_v<TA>();
@@ -159,28 +162,29 @@ mfma_batched_kernel(int M, int N, int K, cplx alpha, const TA* __restrict__ A, i
         }
       }
   };
-  // step s of the next chunk is loaded as soon as step s of this one is multiplied
-  const int kf = K / (4 * KS) * (4 * KS);    // whole chunks
-  if (kf > 0) {
+  // a step's registers are loaded for the step KS further on as soon as it is multiplied
+  const int tf = K / (4 * KP) * KP / KS * KS;               // steps in whole chunks of KS
+  const int te = (K + 4 * KP - 1) / (4 * KP) * KP;
+  if (tf > 0) {
 #pragma unroll
-    for (int s = 0; s < KS; ++s) load(s, 0, false);
-    int k0 = 4 * KS;
+    for (int s = 0; s < KS; ++s) load(s, s, false);
 #pragma unroll 1
-    for (; k0 < kf; k0 += 4 * KS) {
+    for (int t = KS; t < tf; t += KS) {
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
         multiply(s);
         __builtin_amdgcn_sched_barrier(0);
-        load(s, k0, false);
+        load(s, t + s, false);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
 #pragma unroll
     for (int s = 0; s < KS; ++s) multiply(s);
   }
-  if (kf < K) {
+#pragma unroll 1
+  for (int t = tf; t < te; t += KS) {
 #pragma unroll
-    for (int s = 0; s < KS; ++s) load(s, kf, true);
+    for (int s = 0; s < KS; ++s) load(s, t + s, true);
 #pragma unroll
     for (int s = 0; s < KS; ++s) multiply(s);
   }
