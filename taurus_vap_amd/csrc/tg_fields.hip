@@ -33,15 +33,13 @@
 // 5.7e10; the products alone 3.39 -> 1.04 ms and 1.83 -> 0.95 ms, a projection 21.5 ->
 // 18.7 ms.  One set of densities (two products bound by reading W, 0.7 GB) 1.47 -> 0.2 ms.
 #include <algorithm>
-#include <atomic>
 #include <map>
 #include <memory>
 #include <new>
-#include <system_error>
-#include <thread>
 #include <tuple>
 
 #include "tg_internal.h"
+#include "tg_parallel.h"
 
 namespace {
 
@@ -530,30 +528,6 @@ Reduced reduce_class(const tg_ctx* c, bool pp, const std::vector<int>& el, const
   return R;
 }
 
-// f(g) for every class g, by up to eight threads; std::bad_alloc where one ran out of memory
-template <typename F>
-void parallel_classes(int nc, const F& f) {
-  std::atomic<int> next(0);
-  std::atomic<bool> nomem(false);
-  auto work = [&] {
-    try {
-      for (int g; (g = next.fetch_add(1)) < nc;) f(g);
-    } catch (const std::bad_alloc&) {      // nothing may leave a thread
-      nomem = true;
-    }
-  };
-  const int nt = std::max(1, std::min({8, (int)std::thread::hardware_concurrency(), nc}));
-  std::vector<std::thread> pool;
-  pool.reserve(nt);
-  try {
-    for (int k = 1; k < nt; ++k) pool.emplace_back(work);
-  } catch (const std::system_error&) {     // the threads there are take the work
-  }
-  work();
-  for (std::thread& th : pool) th.join();
-  if (nomem) throw std::bad_alloc();
-}
-
 int build_blocks(tg_ctx* c, int64_t ntb, const int16_t* abcd, const void* H2, int h2_bytes,
                  const int8_t* trperm) {
   const int n = c->n;
@@ -650,7 +624,7 @@ int build_blocks(tg_ctx* c, int64_t ntb, const int16_t* abcd, const void* H2, in
     Full& f = F[q];
     const int nc = (int)f.el.size();
     std::vector<Reduced> red(nc);
-    parallel_classes(nc, [&](int g) {
+    parallel_for(nc, [&](int g) {
       if (c->w_fp32)
         for (double& v : f.B[g]) v = (double)(float)v;
       red[g] = reduce_class(c, q == 1, f.el[g], f.B[g]);
@@ -679,7 +653,7 @@ int build_blocks(tg_ctx* c, int64_t ntb, const int16_t* abcd, const void* H2, in
     }
     // (not set to zero first: every byte that a kernel reads is written)
     std::unique_ptr<char[]> W(new char[std::max<size_t>(bytes, 16)]);
-    parallel_classes(nc, [&](int g) {
+    parallel_for(nc, [&](int g) {
       size_t w0 = 0, k = first[g];
       for (int sz : red[g].size) {
         if (sz == 0) continue;
