@@ -286,6 +286,72 @@ mfma_dd_kernel(int M, int N, int K, double alpha, const double* __restrict__ A, 
   }
 }
 
+// The same for many tiles (the matrices of many states): 32 x 32 of C per workgroup, one
+// 16 x 16 block per wave, both operands staged 16 k at a time through LDS, so an element is
+// read for 32 rows or columns instead of 16.  The chain of its 2 K / 16 barriers sets
+// its time (12.5 us at K = 224, 5 at 64) until its workgroups no longer fit the chip at once;
+// mfma_dd_kernel's grows with the tiles from a few hundred on.  32 products A^T B of order 224 33.7
+// against 100 us, 64 of order 140 23.8 against 51, medians inside an iteration.
+template <int OPA, int OPB>
+__global__ void __launch_bounds__(256)
+mfma_dd_lds_kernel(int M, int N, int K, double alpha, const double* __restrict__ A, int lda,
+                   long long sA, const double* __restrict__ B, int ldb, long long sB, double beta,
+                   int use_beta, double* __restrict__ C, int ldc, long long sC, int tiles_m,
+                   int divA, int divB) {
+  constexpr int BT = 32, BK = 16, LD = BT + 1;
+  __shared__ double As[BK][LD], Bs[BK][LD];     // As[k][i] = op(A)(i,k), Bs[k][j] = op(B)(k,j)
+  const int b = blockIdx.y;
+  const double* Ab = A + (long long)(b / divA) * sA;
+  const double* Bb = B + (long long)(b / divB) * sB;
+  double* Cb = C + (long long)b * sC;
+  const int m0 = (blockIdx.x % tiles_m) * BT, n0 = (blockIdx.x / tiles_m) * BT;
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int wi = (w & 1) * 16, wj = (w >> 1) * 16;
+  const int lr = lane & 15, lk = lane >> 4;
+  d4 acc = {0.0, 0.0, 0.0, 0.0};
+  for (int k0 = 0; k0 < K; k0 += BK) {
+    // 512 elements of each operand tile, two per thread, contiguous index fastest
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      const int e = t + 256 * r;
+      int i, k;
+      if (OPA == OP_N) { i = e % BT; k = e / BT; } else { k = e % BK; i = e / BK; }
+      const int gi = m0 + i, gk = k0 + k;
+      double v = 0.0;
+      if (gi < M && gk < K) v = (OPA == OP_N) ? Ab[gi + (long long)gk * lda] : Ab[gk + (long long)gi * lda];
+      As[k][i] = v;
+      int j, k2;
+      if (OPB == OP_N) { k2 = e % BK; j = e / BK; } else { j = e % BT; k2 = e / BT; }
+      const int gj = n0 + j, gk2 = k0 + k2;
+      double u = 0.0;
+      if (gj < N && gk2 < K) u = (OPB == OP_N) ? Bb[gk2 + (long long)gj * ldb] : Bb[gj + (long long)gk2 * ldb];
+      Bs[k2][j] = u;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int kk = 0; kk < BK; kk += 4) {
+      const double av = Bs[kk + lk][wj + lr];    // D rows: columns of C
+      const double bv = As[kk + lk][wi + lr];    // D columns: rows of C
+      acc = mfma(av, bv, acc);
+    }
+    __syncthreads();
+  }
+  // lane l, register r: C(m0 + wi + lr, n0 + wj + lk + 4 r)
+  const int gi = m0 + wi + lr;
+  if (gi < M) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int gj = n0 + wj + lk + 4 * r;
+      if (gj < N) {
+        double* cp = Cb + gi + (long long)gj * ldc;
+        double v = alpha * acc[r];
+        if (use_beta) v = fma(beta, *cp, v);
+        *cp = v;
+      }
+    }
+  }
+}
+
 // Grouped contraction: C(j, a) = sum_k W_g(k, j) X(k, a) for every group g; X and C hold
 // a row of `ld` angles per position (angle contiguous), W_g is real, j contiguous.  The
 // scheme of mfma_batched_kernel with both operands contiguous across the lanes: a wave
@@ -610,15 +676,30 @@ int mfma_gemm_dd(hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, double 
                  double beta, int use_beta, double* C, int ldc, long long sC, int batch, int divA,
                  int divB) {
   if (M <= 0 || N <= 0 || batch <= 0) return TG_OK;
-  const int tiles_m = (M + 15) / 16, tiles_n = (N + 15) / 16;
+  const long long tiles = (long long)((M + 15) / 16) * ((N + 15) / 16) * batch;
+  // Both forms were timed at orders 24 to 336 with 1 to 512 matrices, K = the order and half
+  // of it.  A^T B, both read down their columns: from 750 tiles (order 224, 3 matrices 13.0 with
+  // registers, 12.4 through LDS, 4: 16.6, 12.5).  A B^T, both read along their rows: registers
+  // are as good at any number (order 336, 64 matrices 424, 428) but for short products (order 64,
+  // 64 matrices 5.0, 5.3; 128: 6.9, 6.0).  One of each: short ones from 1000 (order 80, 32: 6.0,
+  // 6.6, 48: 7.1, 6.8), long ones, whose second round of workgroups costs more, from 2000 (order
+  // 224, 8: 19, 25; 16: 35, 27).
+  const bool tn = opa != OP_N && opb == OP_N, nt = opa == OP_N && opb != OP_N;
+  const long long most = tn ? 750 : nt ? (K <= 64 ? 1000 : tiles) : (K <= 96 ? 1000 : 2000);
+  const bool many = tiles > most;
+  const int bt = many ? 32 : 16, tiles_m = (M + bt - 1) / bt, tiles_n = (N + bt - 1) / bt;
   const dim3 grid(tiles_m * tiles_n, batch);
 #define TG_DD(OA, OB)                                                                              \
-  hipLaunchKernelGGL((mfma_dd_kernel<OA, OB>), grid, dim3(256), 0, s, M, N, K, alpha, A, lda, sA, \
-                     B, ldb, sB, beta, use_beta, C, ldc, sC, tiles_m, divA, divB)
-  if (opa == OP_N && opb == OP_N) TG_DD(OP_N, OP_N);
-  else if (opa == OP_N) TG_DD(OP_N, OP_T);
-  else if (opb == OP_N) TG_DD(OP_T, OP_N);
-  else TG_DD(OP_T, OP_T);
+  if (many)                                                                                        \
+    hipLaunchKernelGGL((mfma_dd_lds_kernel<OA, OB>), grid, dim3(256), 0, s, M, N, K, alpha, A, lda, \
+                       sA, B, ldb, sB, beta, use_beta, C, ldc, sC, tiles_m, divA, divB);           \
+  else                                                                                             \
+    hipLaunchKernelGGL((mfma_dd_kernel<OA, OB>), grid, dim3(256), 0, s, M, N, K, alpha, A, lda, sA, \
+                       B, ldb, sB, beta, use_beta, C, ldc, sC, tiles_m, divA, divB)
+  if (opa == OP_N && opb == OP_N) { TG_DD(OP_N, OP_N); }
+  else if (opa == OP_N) { TG_DD(OP_N, OP_T); }
+  else if (opb == OP_N) { TG_DD(OP_T, OP_N); }
+  else { TG_DD(OP_T, OP_T); }
 #undef TG_DD
   TG_HIP(hipGetLastError());
   return TG_OK;
