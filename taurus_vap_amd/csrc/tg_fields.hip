@@ -14,30 +14,16 @@
 // element keeps its value, and the angles of a batch become the M dimension of one
 // GEMM per block: the scattered, atomic-prone loop turns into dense FP64 arithmetic.
 //
-// The blocks are reduced further by the symmetries the interaction has, each a signed
-// permutation of a block's elements:
-//   ph: time reversal with hermiticity, (a,c) -> (c~,a~);  pp: time reversal,
-//       (x,y) -> (x~,y~); the signs follow from the elements;
-//   charge reflection, proton <-> neutron of every state (+1 in ph; a stored pp pair
-//       changes its order, -1), and the product of the two.
-// One that maps a block to itself and leaves its matrix the same BIT BY BIT (checked at
-// tg_init on the values as stored, so no element is changed; a charge-dependent
-// interaction, or one whose elements carry different rounding, simply does not pass)
-// commutes with the block: the elements fall into orbits, and the sums
-// a_chi(O) = sum_p c_chi(p) x_p over an orbit, c = +-1, mix only within a character
-// chi.  A block of s elements becomes 2 (or 4) of about s/2 (s/4): half (a quarter) of
-// the multiply-adds.  Their elements are sums of 2 (4) stored ones, scaled by the power
-// of two |O|, and are kept in FP64; they take the bytes of the FP32 block.  A block with
-// no symmetry keeps its elements as stored (FP32 when the TBMEs are FP32).
+// The blocks are reduced further by the symmetries the interaction has (tg_blocks.h): the
+// gathers form the sums over the orbits, the scatters undo them.
 // At 336 states, FP32 TBMEs, 225 angles: ph 1.71e11 -> 5.7e10 flop, pp 8.5e10 ->
 // 5.7e10; the products alone 3.39 -> 1.04 ms and 1.83 -> 0.95 ms, a projection 21.5 ->
 // 18.7 ms.  One set of densities (two products bound by reading W, 0.7 GB) 1.47 -> 0.2 ms.
 #include <algorithm>
-#include <map>
 #include <memory>
 #include <new>
-#include <tuple>
 
+#include "tg_blocks.h"
 #include "tg_internal.h"
 #include "tg_parallel.h"
 
@@ -271,266 +257,10 @@ __global__ void hermitize_kernel(int n, int na, long long nn, cplx* __restrict__
 
 inline unsigned nblk(long long tot) { return (unsigned)((tot + NT - 1) / NT); }
 
-struct KeyCmp {
-  bool operator()(const std::tuple<int, int, int>& a, const std::tuple<int, int, int>& b) const {
-    return a < b;
-  }
-};
-
-typedef std::tuple<int, int, int> ClassKey;
-
-// Elements of a block channel by class, in patches of 8 x 8 (linear indices x + y n)
-std::map<ClassKey, std::vector<int>> channel_classes(const tg_ctx* c, bool pp) {
-  const int n = c->n;
-  const std::vector<int>&m = c->sp_2mj, &t = c->sp_2mt, &l = c->sp_l;
-  // runs of states with the same m, t and parity, and the place of a state in its run
-  std::vector<int> run(n, 0), in(n, 0);
-  for (int i = 1; i < n; ++i) {
-    const bool same = m[i] == m[i - 1] && t[i] == t[i - 1] && (l[i] & 1) == (l[i - 1] & 1);
-    run[i] = run[i - 1] + (same ? 0 : 1);
-    in[i] = same ? in[i - 1] + 1 : 0;
-  }
-  std::map<ClassKey, std::vector<int>> cls;
-  for (int y = 0; y < n; ++y)
-    for (int x = 0; x < n; ++x) {
-      if (pp && x <= y) continue;
-      cls[pp ? ClassKey(m[x] + m[y], t[x] + t[y], (l[x] + l[y]) & 1)
-             : ClassKey(m[x] - m[y], t[x] - t[y], (l[x] + l[y]) & 1)]
-          .push_back(x + y * n);
-    }
-  for (auto& kv : cls)
-    std::sort(kv.second.begin(), kv.second.end(), [&](int p, int q) {
-      auto key = [&](int e) {
-        const int x = e % n, y = e / n;
-        return std::make_tuple(run[x], run[y], in[y] / 8, in[x] / 8, in[y], in[x]);
-      };
-      return key(p) < key(q);
-    });
-  return cls;
-}
-
-// A signed permutation of a class: element k -> to[k] with sign sg[k]
-struct Sym {
-  std::vector<int> to, sg;
-};
-
-// Whether B(to p, to q) = sg_p sg_q B(p, q) for all p, q, bit by bit (B symmetric in
-// meaning, stored at B[q + p s]).  With `find` the signs are found first: +-1 spread
-// over the elements that B connects, an element and its images (imgs) alike.
-bool sym_holds(const std::vector<double>& B, int s, Sym& g, bool find,
-               const std::vector<const std::vector<int>*>& imgs) {
-  if (find) {
-    g.sg.assign(s, 0);
-    std::vector<int> todo;
-    auto visit = [&](int k, int sg) {
-      std::vector<int> st(1, k);
-      while (!st.empty()) {
-        const int e = st.back();
-        st.pop_back();
-        if (g.sg[e] != 0) continue;
-        g.sg[e] = sg;
-        todo.push_back(e);
-        for (const std::vector<int>* im : imgs) st.push_back((*im)[e]);
-      }
-    };
-    for (int r = 0; r < s; ++r) {
-      if (g.sg[r] != 0) continue;
-      visit(r, 1);
-      while (!todo.empty()) {
-        const int p = todo.back();
-        todo.pop_back();
-        const double* bp = B.data() + (size_t)p * s;
-        const double* bt = B.data() + (size_t)g.to[p] * s;
-        for (int q = 0; q < s; ++q)
-          if (g.sg[q] == 0 && bp[q] != 0.0) visit(q, (bp[q] == bt[g.to[q]]) ? g.sg[p] : -g.sg[p]);
-      }
-    }
-  }
-  for (int p = 0; p < s; ++p) {
-    const double* bp = B.data() + (size_t)p * s;
-    const double* bt = B.data() + (size_t)g.to[p] * s;
-    const double sp = g.sg[p];
-    for (int q = 0; q < s; ++q)
-      if (!(bt[g.to[q]] == sp * g.sg[q] * bp[q])) return false;
-  }
-  return true;
-}
-
-// One class of a channel reduced by its symmetries: its orbits (positions relative to
-// the class) and the character blocks W (matrix [in * size + out], one after another).
-struct Reduced {
-  std::vector<Orbit> orb;
-  std::vector<int> size;
-  std::vector<double> W;
-  bool split = false;
-};
-
-Reduced reduce_class(const tg_ctx* c, bool pp, const std::vector<int>& el, const std::vector<double>& B) {
-  const int n = c->n, h = n / 2, s = (int)el.size();
-  std::vector<int> at((size_t)n * n, -1);
-  for (int k = 0; k < s; ++k) at[el[k]] = k;
-  // the proton and the neutron half hold the same states, in the same order
-  bool halves = true;
-  for (int i = 0; i < h && halves; ++i)
-    halves = c->sp_2mj[i] == c->sp_2mj[i + h] && c->sp_l[i] == c->sp_l[i + h] &&
-             c->sp_tr[i] < h && c->sp_tr[i + h] == c->sp_tr[i] + h;
-  bool tr_ok = true;
-  for (int i = 0; i < n && tr_ok; ++i) tr_ok = c->sp_tr[c->sp_tr[i]] == i && c->sp_tr[i] != i;
-  // image of element (x, y): time reversal (and transposition in ph), reflection; the
-  // sign where a pp pair changes its order
-  auto image = [&](int e, bool tr, bool ch, int& sg) {
-    int x = e % n, y = e / n;
-    sg = 1;
-    if (tr) {
-      const int tx = c->sp_tr[x], ty = c->sp_tr[y];
-      x = pp ? tx : ty;
-      y = pp ? ty : tx;
-    }
-    if (ch) {
-      x = (x + h) % n;
-      y = (y + h) % n;
-    }
-    if (pp && x < y) {
-      std::swap(x, y);
-      sg = -1;
-    }
-    return x + y * n;
-  };
-  Sym g[3];               // time reversal, reflection, their product
-  bool ok[3];
-  for (int q = 0; q < 3; ++q) {
-    const bool tr = q != 1, ch = q != 0;
-    ok[q] = (!tr || tr_ok) && (!ch || halves) && s > 1;
-    g[q].to.assign(s, 0);
-    g[q].sg.assign(s, 1);
-    for (int k = 0; k < s && ok[q]; ++k) {
-      g[q].to[k] = at[image(el[k], tr, ch, g[q].sg[k])];
-      ok[q] = g[q].to[k] >= 0;
-    }
-    for (int k = 0; k < s && ok[q]; ++k) ok[q] = g[q].to[g[q].to[k]] == k;
-  }
-  std::vector<const std::vector<int>*> imgs;
-  for (int q = 0; q < 3; ++q)
-    if (ok[q]) imgs.push_back(&g[q].to);
-  // the reflection's signs are known; those with time reversal are found
-  if (ok[1]) ok[1] = sym_holds(B, s, g[1], false, imgs);
-  if (ok[0]) ok[0] = sym_holds(B, s, g[0], true, imgs);
-  if (ok[2] && !(ok[0] && ok[1])) ok[2] = sym_holds(B, s, g[2], true, imgs);
-  // signs of an involution agree on an element and its image
-  for (int q = 0; q < 3; ++q)
-    for (int k = 0; k < s && ok[q]; ++k) ok[q] = g[q].sg[k] == g[q].sg[g[q].to[k]];
-  std::vector<const Sym*> gen;
-  if (ok[0] && ok[1]) {
-    bool commute = true;
-    for (int k = 0; k < s && commute; ++k)
-      commute = g[0].to[g[1].to[k]] == g[1].to[g[0].to[k]] &&
-                g[0].sg[g[1].to[k]] * g[1].sg[k] == g[1].sg[g[0].to[k]] * g[0].sg[k];
-    gen.push_back(&g[0]);
-    if (commute) gen.push_back(&g[1]);
-  } else {
-    for (int q = 0; q < 3; ++q)
-      if (ok[q]) {
-        gen.push_back(&g[q]);
-        break;
-      }
-  }
-  Reduced R;
-  R.split = !gen.empty();
-  const int ng = (int)gen.size(), order = 1 << ng;
-  // orbits: element e_b = (product of the generators in b) of the first one, its sign
-  std::vector<char> seen(s, 0);
-  R.size.assign(order, 0);
-  std::vector<std::vector<int>> members;          // elements of each orbit (class index)
-  std::vector<unsigned> masks;                    // bit 4 j + i: minus of element i in sum j
-  std::vector<std::vector<int>> chars;            // character of each of the orbit's sums
-  for (int k = 0; k < s; ++k) {
-    if (seen[k]) continue;
-    int im[4], sg[4];
-    for (int b = 0; b < order; ++b) {
-      int e = k, sgn = 1;
-      for (int q = 0; q < ng; ++q)
-        if (b >> q & 1) {
-          sgn *= gen[q]->sg[e];
-          e = gen[q]->to[e];
-        }
-      im[b] = e;
-      sg[b] = sgn;
-    }
-    std::vector<int> mem, first;
-    for (int b = 0; b < order; ++b)
-      if (std::find(mem.begin(), mem.end(), im[b]) == mem.end()) {
-        mem.push_back(im[b]);
-        first.push_back(b);
-        seen[im[b]] = 1;
-      }
-    std::vector<int> ch;
-    unsigned mask = 0;
-    for (int x = 0; x < order; ++x) {
-      // character x: sign (-1)^(bits of b & x) of the group element b
-      auto cs = [&](int b) { return (__builtin_popcount(b & x) & 1 ? -1 : 1) * sg[b]; };
-      bool fits = true;
-      for (int b = 0; b < order && fits; ++b)
-        for (int b2 = 0; b2 < b && fits; ++b2)
-          if (im[b] == im[b2]) fits = cs(b) == cs(b2);
-      if (!fits) continue;
-      const int j = (int)ch.size();
-      for (size_t i = 0; i < mem.size(); ++i)
-        if (cs(first[i]) < 0) mask |= 1u << (4 * j + (int)i);
-      ch.push_back(x);
-    }
-    members.push_back(mem);
-    masks.push_back(mask);
-    chars.push_back(ch);
-    for (int x : ch) ++R.size[x];
-  }
-  // positions: character blocks one after another, orbits in order inside each
-  std::vector<int> base(order, 0), fill(order, 0);
-  std::vector<size_t> wbase(order, 0);
-  size_t wsz = 0;
-  for (int x = 0, o = 0; x < order; ++x) {
-    base[x] = o;
-    o += R.size[x];
-    wbase[x] = wsz;
-    wsz += (size_t)R.size[x] * R.size[x];
-  }
-  R.W.assign(wsz, 0.0);
-  const size_t no = members.size();
-  std::vector<std::vector<int>> idx(no);          // index of each of its sums in its block
-  for (size_t o = 0; o < no; ++o) {
-    Orbit ob{};
-    ob.m = (int)members[o].size();
-    ob.mask = masks[o];
-    for (int i = 0; i < ob.m; ++i) {
-      ob.lin[i] = el[members[o][i]];
-      const int x = chars[o][i];
-      idx[o].push_back(fill[x]);
-      ob.pos[i] = base[x] + fill[x]++;
-    }
-    R.orb.push_back(ob);
-  }
-  for (size_t out = 0; out < no; ++out) {
-    const double* row = B.data() + (size_t)members[out][0] * s;
-    for (size_t jo = 0; jo < chars[out].size(); ++jo) {
-      const int x = chars[out][jo];
-      double* w = R.W.data() + wbase[x] + idx[out][jo];
-      for (size_t o = 0; o < no; ++o)
-        for (size_t j = 0; j < chars[o].size(); ++j)
-          if (chars[o][j] == x) {
-            double v = 0.0;
-            for (size_t i = 0; i < members[o].size(); ++i) {
-              const double b = row[members[o][i]];
-              v += (masks[o] >> (4 * j + i) & 1u) ? -b : b;
-            }
-            w[(size_t)idx[o][j] * R.size[x]] = v / (double)members[o].size();
-          }
-    }
-  }
-  return R;
-}
-
 int build_blocks(tg_ctx* c, int64_t ntb, const int16_t* abcd, const void* H2, int h2_bytes,
                  const int8_t* trperm) {
   const int n = c->n;
+  const SpBasis basis{n, c->sp_2mj, c->sp_2mt, c->sp_l, c->sp_tr};
   // per channel: the classes, the class and place of every element, the full matrices
   struct Full {
     std::vector<std::vector<int>> el;
@@ -540,7 +270,7 @@ int build_blocks(tg_ctx* c, int64_t ntb, const int16_t* abcd, const void* H2, in
   for (int q = 0; q < 2; ++q) {
     F[q].cls.assign((size_t)n * n, -1);
     F[q].at.assign((size_t)n * n, -1);
-    for (auto& kv : channel_classes(c, q == 1)) {
+    for (auto& kv : channel_classes(basis, q == 1)) {
       for (size_t k = 0; k < kv.second.size(); ++k) {
         F[q].cls[kv.second[k]] = (int)F[q].el.size();
         F[q].at[kv.second[k]] = (int)k;
@@ -627,7 +357,7 @@ int build_blocks(tg_ctx* c, int64_t ntb, const int16_t* abcd, const void* H2, in
     parallel_for(nc, [&](int g) {
       if (c->w_fp32)
         for (double& v : f.B[g]) v = (double)(float)v;
-      red[g] = reduce_class(c, q == 1, f.el[g], f.B[g]);
+      red[g] = reduce_class(basis, q == 1, f.el[g], f.B[g]);
       std::vector<double>().swap(f.B[g]);
     });
 

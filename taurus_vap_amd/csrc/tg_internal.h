@@ -180,15 +180,6 @@ int batched_pfaffian(hipStream_t s, int n, cplx* A, int lda, long long sA, int b
 // ---------------------------------------------------------------------------
 // Contraction plan (tg_fields.hip)
 // ---------------------------------------------------------------------------
-// An orbit of matrix elements under the symmetries of its block and the sums the
-// contraction takes over it (kernels of tg_fields.hip); m elements and m sums.
-struct Orbit {
-  int lin[4];                   // linear indices x + y*n of the elements
-  int pos[4];                   // positions of the sums
-  unsigned mask;                // bit 4 j + i: element i enters sum j with a minus
-  int m;
-};
-
 struct Channel {
   int npos = 0;                 // number of positions (n*n for ph, n(n-1)/2 for pp)
   int ngroups = 0, norb = 0;
