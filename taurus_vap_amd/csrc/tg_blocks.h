@@ -46,29 +46,24 @@ typedef std::tuple<int, int, int> ClassKey;
 inline std::map<ClassKey, std::vector<int>> channel_classes(const SpBasis& c, bool pp) {
   const int n = c.n;
   const std::vector<int>&m = c.sp_2mj, &t = c.sp_2mt, &l = c.sp_l;
-  // runs of states with the same m, t and parity, and the place of a state in its run
-  std::vector<int> run(n, 0), in(n, 0);
-  for (int i = 1; i < n; ++i) {
-    const bool same = m[i] == m[i - 1] && t[i] == t[i - 1] && (l[i] & 1) == (l[i - 1] & 1);
-    run[i] = run[i - 1] + (same ? 0 : 1);
-    in[i] = same ? in[i - 1] + 1 : 0;
-  }
+  // runs of states with the same m, t and parity; the elements of two runs are of one class
+  std::vector<int> run(1, 0);
+  for (int i = 1; i < n; ++i)
+    if (m[i] != m[i - 1] || t[i] != t[i - 1] || (l[i] & 1) != (l[i - 1] & 1)) run.push_back(i);
+  run.push_back(n);
   std::map<ClassKey, std::vector<int>> cls;
-  for (int y = 0; y < n; ++y)
-    for (int x = 0; x < n; ++x) {
-      if (pp && x <= y) continue;
-      cls[pp ? ClassKey(m[x] + m[y], t[x] + t[y], (l[x] + l[y]) & 1)
-             : ClassKey(m[x] - m[y], t[x] - t[y], (l[x] + l[y]) & 1)]
-          .push_back(x + y * n);
+  for (size_t rx = 0; rx + 1 < run.size(); ++rx)
+    for (size_t ry = 0; ry + 1 < run.size(); ++ry) {
+      const int x0 = run[rx], x1 = run[rx + 1], y0 = run[ry], y1 = run[ry + 1];
+      if (pp && x1 - 1 <= y0) continue;              // (every x > y)
+      std::vector<int>& el = cls[pp ? ClassKey(m[x0] + m[y0], t[x0] + t[y0], (l[x0] + l[y0]) & 1)
+                                    : ClassKey(m[x0] - m[y0], t[x0] - t[y0], (l[x0] + l[y0]) & 1)];
+      for (int yb = y0; yb < y1; yb += 8)
+        for (int xb = x0; xb < x1; xb += 8)
+          for (int y = yb; y < std::min(yb + 8, y1); ++y)
+            for (int x = xb; x < std::min(xb + 8, x1); ++x)
+              if (!pp || x > y) el.push_back(x + y * n);
     }
-  for (auto& kv : cls)
-    std::sort(kv.second.begin(), kv.second.end(), [&](int p, int q) {
-      auto key = [&](int e) {
-        const int x = e % n, y = e / n;
-        return std::make_tuple(run[x], run[y], in[y] / 8, in[x] / 8, in[y], in[x]);
-      };
-      return key(p) < key(q);
-    });
   return cls;
 }
 
@@ -78,9 +73,9 @@ struct Sym {
 };
 
 // Whether B(to p, to q) = sg_p sg_q B(p, q) for all p, q, bit by bit (B symmetric in
-// meaning, stored at B[q + p s]).  With `find` the signs are found first: +-1 spread
+// meaning, stored at B[q + p s], p the input).  With `find` the signs are found first: +-1 spread
 // over the elements that B connects, an element and its images (imgs) alike.
-inline bool sym_holds(const std::vector<double>& B, int s, Sym& g, bool find,
+inline bool sym_holds(const double* B, int s, Sym& g, bool find,
                       const std::vector<const std::vector<int>*>& imgs) {
   if (find) {
     g.sg.assign(s, 0);
@@ -102,16 +97,16 @@ inline bool sym_holds(const std::vector<double>& B, int s, Sym& g, bool find,
       while (!todo.empty()) {
         const int p = todo.back();
         todo.pop_back();
-        const double* bp = B.data() + (size_t)p * s;
-        const double* bt = B.data() + (size_t)g.to[p] * s;
+        const double* bp = B + (size_t)p * s;
+        const double* bt = B + (size_t)g.to[p] * s;
         for (int q = 0; q < s; ++q)
           if (g.sg[q] == 0 && bp[q] != 0.0) visit(q, (bp[q] == bt[g.to[q]]) ? g.sg[p] : -g.sg[p]);
       }
     }
   }
   for (int p = 0; p < s; ++p) {
-    const double* bp = B.data() + (size_t)p * s;
-    const double* bt = B.data() + (size_t)g.to[p] * s;
+    const double* bp = B + (size_t)p * s;
+    const double* bt = B + (size_t)g.to[p] * s;
     const double sp = g.sg[p];
     for (int q = 0; q < s; ++q)
       if (!(bt[g.to[q]] == sp * g.sg[q] * bp[q])) return false;
@@ -120,19 +115,24 @@ inline bool sym_holds(const std::vector<double>& B, int s, Sym& g, bool find,
 }
 
 // One class of a channel reduced by its symmetries: its orbits (positions relative to
-// the class) and the character blocks W (matrix [in * size + out], one after another).
+// the class) and the orders of the character blocks.
 struct Reduced {
   std::vector<Orbit> orb;
   std::vector<int> size;
-  std::vector<double> W;
   bool split = false;
 };
 
-inline Reduced reduce_class(const SpBasis& c, bool pp, const std::vector<int>& el,
-                            const std::vector<double>& B) {
+// Elements a block of order s takes: a whole number of 16 bytes
+inline size_t block_len(size_t s) { return (s * s + 1) / 2 * 2; }
+
+// Reduces a class in place: the blocks (matrix [in * size + out], block_len(size) apart)
+// replace B, which has room for block_len(s).  place(e): index of element e in the
+// class, or -1; tmp: scratch.
+
+template <typename Place>
+Reduced reduce_class(const SpBasis& c, bool pp, const std::vector<int>& el, double* B, const Place& place,
+                     std::vector<double>& tmp) {
   const int n = c.n, h = n / 2, s = (int)el.size();
-  std::vector<int> at((size_t)n * n, -1);
-  for (int k = 0; k < s; ++k) at[el[k]] = k;
   // the proton and the neutron half hold the same states, in the same order
   bool halves = true;
   for (int i = 0; i < h && halves; ++i)
@@ -168,7 +168,7 @@ inline Reduced reduce_class(const SpBasis& c, bool pp, const std::vector<int>& e
     g[q].to.assign(s, 0);
     g[q].sg.assign(s, 1);
     for (int k = 0; k < s && ok[q]; ++k) {
-      g[q].to[k] = at[image(el[k], tr, ch, g[q].sg[k])];
+      g[q].to[k] = place(image(el[k], tr, ch, g[q].sg[k]));
       ok[q] = g[q].to[k] >= 0;
     }
     for (int k = 0; k < s && ok[q]; ++k) ok[q] = g[q].to[g[q].to[k]] == k;
@@ -200,6 +200,17 @@ inline Reduced reduce_class(const SpBasis& c, bool pp, const std::vector<int>& e
   }
   Reduced R;
   R.split = !gen.empty();
+  if (!R.split) {
+    R.size.assign(1, s);
+    R.orb.resize(s);
+    for (int k = 0; k < s; ++k) {
+      R.orb[k] = Orbit{};
+      R.orb[k].lin[0] = el[k];
+      R.orb[k].pos[0] = k;
+      R.orb[k].m = 1;
+    }
+    return R;
+  }
   const int ng = (int)gen.size(), order = 1 << ng;
   // orbits: element e_b = (product of the generators in b) of the first one, its sign
   std::vector<char> seen(s, 0);
@@ -255,9 +266,9 @@ inline Reduced reduce_class(const SpBasis& c, bool pp, const std::vector<int>& e
     base[x] = o;
     o += R.size[x];
     wbase[x] = wsz;
-    wsz += (size_t)R.size[x] * R.size[x];
+    wsz += block_len(R.size[x]);
   }
-  R.W.assign(wsz, 0.0);
+  tmp.assign(wsz, 0.0);
   const size_t no = members.size();
   std::vector<std::vector<int>> idx(no);          // index of each of its sums in its block
   for (size_t o = 0; o < no; ++o) {
@@ -272,22 +283,32 @@ inline Reduced reduce_class(const SpBasis& c, bool pp, const std::vector<int>& e
     }
     R.orb.push_back(ob);
   }
-  for (size_t out = 0; out < no; ++out) {
-    const double* row = B.data() + (size_t)members[out][0] * s;
-    for (size_t jo = 0; jo < chars[out].size(); ++jo) {
-      const int x = chars[out][jo];
-      double* w = R.W.data() + wbase[x] + idx[out][jo];
-      for (size_t o = 0; o < no; ++o)
-        for (size_t j = 0; j < chars[o].size(); ++j)
-          if (chars[o][j] == x) {
-            double v = 0.0;
-            for (size_t i = 0; i < members[o].size(); ++i) {
-              const double b = row[members[o][i]];
-              v += (masks[o] >> (4 * j + i) & 1u) ? -b : b;
-            }
-            w[(size_t)idx[o][j] * R.size[x]] = v / (double)members[o].size();
-          }
+  // the first elements of the orbits of each block, in its order: the outputs of a row
+  std::vector<std::vector<int>> head(order);
+  for (size_t o = 0; o < no; ++o)
+    for (int x : chars[o]) head[x].push_back(members[o][0]);
+  for (size_t o = 0; o < no; ++o)
+    for (size_t j = 0; j < chars[o].size(); ++j) {
+      const int x = chars[o][j], size = R.size[x], m = (int)members[o].size();
+      const int* out = head[x].data();
+      double* w = tmp.data() + wbase[x] + (size_t)idx[o][j] * size;
+      const double* row[4];
+      double sg[4];
+      for (int i = 0; i < m; ++i) {
+        row[i] = B + (size_t)members[o][i] * s;
+        sg[i] = (masks[o] >> (4 * j + i) & 1u) ? -1.0 : 1.0;
+      }
+      const double over = 1.0 / m;             // a power of two
+      // (0.0 +: no element is a negative zero)
+      if (m == 1)
+        for (int k = 0; k < size; ++k) w[k] = 0.0 + sg[0] * row[0][out[k]];
+      else if (m == 2)
+        for (int k = 0; k < size; ++k) w[k] = ((0.0 + sg[0] * row[0][out[k]]) + sg[1] * row[1][out[k]]) * over;
+      else
+        for (int k = 0; k < size; ++k)
+          w[k] = ((((0.0 + sg[0] * row[0][out[k]]) + sg[1] * row[1][out[k]]) + sg[2] * row[2][out[k]]) +
+                  sg[3] * row[3][out[k]]) * over;
     }
-  }
+  std::copy(tmp.begin(), tmp.end(), B);
   return R;
 }

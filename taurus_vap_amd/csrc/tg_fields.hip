@@ -20,6 +20,8 @@
 // 5.7e10; the products alone 3.39 -> 1.04 ms and 1.83 -> 0.95 ms, a projection 21.5 ->
 // 18.7 ms.  One set of densities (two products bound by reading W, 0.7 GB) 1.47 -> 0.2 ms.
 #include <algorithm>
+#include <cstdlib>
+#include <cstring>
 #include <memory>
 #include <new>
 
@@ -262,30 +264,42 @@ int build_blocks(tg_ctx* c, int64_t ntb, const int16_t* abcd, const void* H2, in
   const int n = c->n;
   const SpBasis basis{n, c->sp_2mj, c->sp_2mt, c->sp_l, c->sp_tr};
   // per channel: the classes, the class and place of every element, the full matrices
+  struct Place {
+    int cls, at;
+  };
   struct Full {
     std::vector<std::vector<int>> el;
-    std::vector<int> cls, at;
-    std::vector<std::vector<double>> B;
+    std::vector<Place> place;
+    std::unique_ptr<double, void (*)(void*)> B{nullptr, std::free};   // one class after another
+    std::vector<std::pair<double*, size_t>> mat;                     // a class's matrix and order
+    size_t elements = 0;
   } F[2];
   for (int q = 0; q < 2; ++q) {
-    F[q].cls.assign((size_t)n * n, -1);
-    F[q].at.assign((size_t)n * n, -1);
+    Full& f = F[q];
+    f.place.assign((size_t)n * n, Place{-1, -1});
     for (auto& kv : channel_classes(basis, q == 1)) {
-      for (size_t k = 0; k < kv.second.size(); ++k) {
-        F[q].cls[kv.second[k]] = (int)F[q].el.size();
-        F[q].at[kv.second[k]] = (int)k;
-      }
-      F[q].B.emplace_back(kv.second.size() * kv.second.size(), 0.0);
-      F[q].el.push_back(std::move(kv.second));
+      const size_t s = kv.second.size();
+      for (size_t k = 0; k < s; ++k) f.place[kv.second[k]] = Place{(int)f.el.size(), (int)k};
+      f.mat.emplace_back(nullptr, s);
+      f.el.push_back(std::move(kv.second));
+      f.elements += block_len(s);
+    }
+    // (zero pages, touched where the list has elements)
+    f.B.reset(static_cast<double*>(std::calloc(std::max<size_t>(f.elements, 2), sizeof(double))));
+    if (!f.B) throw std::bad_alloc();
+    double* at = f.B.get();
+    for (auto& m : f.mat) {
+      m.first = at;
+      at += block_len(m.second);
     }
   }
 
   bool bad = false;
-  // B(q, p) of the class holding both elements, stored at q + p * s (p the field's)
+  // B(q, p) of the class holding both elements, stored at q + p * s (q the field's)
   auto add = [&](Full& f, int out, int in, double v) {
-    const int g = f.cls[out];
-    if (g < 0 || f.cls[in] != g) { bad = true; return; }
-    f.B[g][(size_t)f.at[in] + (size_t)f.at[out] * f.el[g].size()] += v;
+    const Place o = f.place[out], i = f.place[in];
+    if (o.cls < 0 || i.cls != o.cls) { bad = true; return; }
+    f.mat[o.cls].first[(size_t)o.at + (size_t)i.at * f.mat[o.cls].second] += v;
   };
   auto add_ph = [&](int a, int cc, int d, int b, double v) { add(F[0], a + cc * n, d + b * n, v); };
   auto add_pp = [&](int x, int y, int u, int w, double v) {
@@ -354,16 +368,20 @@ int build_blocks(tg_ctx* c, int64_t ntb, const int16_t* abcd, const void* H2, in
     Full& f = F[q];
     const int nc = (int)f.el.size();
     std::vector<Reduced> red(nc);
-    parallel_for(nc, [&](int g) {
+    // a thread takes longer to start (20 us) than 64 K elements to look at
+    const int threads = (int)std::min<size_t>(8, 1 + f.elements / 65536);
+    parallel_for<std::vector<double>>(nc, threads, [&](int g, std::vector<double>& tmp) {
+      double* B = f.mat[g].first;
+      const size_t cnt = f.mat[g].second * f.mat[g].second;
       if (c->w_fp32)
-        for (double& v : f.B[g]) v = (double)(float)v;
-      red[g] = reduce_class(basis, q == 1, f.el[g], f.B[g]);
-      std::vector<double>().swap(f.B[g]);
+        for (size_t e = 0; e < cnt; ++e) B[e] = (double)(float)B[e];
+      const auto place = [&](int e) { return f.place[e].cls == g ? f.place[e].at : -1; };
+      red[g] = reduce_class(basis, q == 1, f.el[g], B, place, tmp);
     });
 
     std::vector<GroupDesc> groups;
     std::vector<Orbit> orb;
-    std::vector<size_t> first(nc);      // group of each class's first block
+    char* const W = reinterpret_cast<char*>(f.B.get());
     size_t bytes = 0;
     int off = 0;
     for (int g = 0; g < nc; ++g) {
@@ -371,33 +389,27 @@ int build_blocks(tg_ctx* c, int64_t ntb, const int16_t* abcd, const void* H2, in
         for (int i = 0; i < o.m; ++i) o.pos[i] += off;
         orb.push_back(o);
       }
-      first[g] = groups.size();
+      // the class's blocks move up to those before it (16 bytes aligned, as where they are)
       const bool f32 = c->w_fp32 && !red[g].split;
+      const size_t at = bytes;
       for (int sz : red[g].size) {
         if (sz == 0) continue;
-        bytes = (bytes + 15) / 16 * 16;
         groups.push_back({off, sz, (long long)bytes, f32 ? 1 : 0});
-        bytes += (size_t)sz * sz * (f32 ? sizeof(float) : sizeof(double));
+        bytes += f32 ? ((size_t)sz * sz * sizeof(float) + 15) / 16 * 16 : block_len(sz) * sizeof(double);
         off += sz;
       }
-    }
-    // (not set to zero first: every byte that a kernel reads is written)
-    std::unique_ptr<char[]> W(new char[std::max<size_t>(bytes, 16)]);
-    parallel_for(nc, [&](int g) {
-      size_t w0 = 0, k = first[g];
-      for (int sz : red[g].size) {
-        if (sz == 0) continue;
-        const size_t cnt = (size_t)sz * sz;
-        char* to = W.get() + groups[k].woff;
-        if (groups[k].fp32)
-          for (size_t e = 0; e < cnt; ++e) reinterpret_cast<float*>(to)[e] = (float)red[g].W[w0 + e];
-        else
-          std::copy_n(red[g].W.data() + w0, cnt, reinterpret_cast<double*>(to));
-        w0 += cnt;
-        ++k;
+      const double* B = f.mat[g].first;
+      if (f32) {
+        const size_t cnt = f.mat[g].second * f.mat[g].second;
+        for (size_t e = 0; e < cnt; ++e) {
+          const float v = (float)B[e];
+          std::memcpy(W + at + e * sizeof(float), &v, sizeof(float));
+        }
+      } else {
+        std::memmove(W + at, B, bytes - at);
       }
       red[g] = Reduced();
-    });
+    }
     ch.npos = off;
     ch.ngroups = (int)groups.size();
     ch.norb = (int)orb.size();
@@ -432,7 +444,7 @@ int build_blocks(tg_ctx* c, int64_t ntb, const int16_t* abcd, const void* H2, in
     };
     TG_TRY(up(ch.d_orb, orb.data(), sizeof(Orbit) * orb.size()));
     TG_TRY(up(ch.d_groups, groups.data(), sizeof(GroupDesc) * groups.size()));
-    TG_TRY(up(ch.d_W, W.get(), bytes));
+    TG_TRY(up(ch.d_W, W, bytes));
     TG_TRY(up(ch.d_tile_group, tg.data(), sizeof(int) * tg.size()));
     TG_TRY(up(ch.d_tile_n0, tn.data(), sizeof(int) * tn.size()));
   }

@@ -109,8 +109,10 @@ int main(int, char** argv) {
       for (const P& g : gen) moved = moved || g.to[0] != 0;
       if (moved) largest = 0;             // (which symmetries are left is not followed)
     }
-    const std::vector<double> B0 = B;
-    const Reduced R = reduce_class(basis, pp, el, B);
+    const std::vector<double> B0 = B;      // (B is reduced in place)
+    std::vector<double> tmp;
+    B.resize(block_len(s));
+    const Reduced R = reduce_class(basis, pp, el, B.data(), [&](int e) { return at[e]; }, tmp);
     int got = 1, elements = 0, sums = 0;
     for (const Orbit& o : R.orb) { got = std::max(got, o.m); elements += o.m; }
     for (int z : R.size) sums += z;
@@ -133,9 +135,9 @@ int main(int, char** argv) {
     int off = 0;
     for (int z : R.size) {
       for (int k = 0; k < z; ++k)
-        for (int j = 0; j < z; ++j) C[off + j] += R.W[w0 + (size_t)k * z + j] * X[off + k];
+        for (int j = 0; j < z; ++j) C[off + j] += B[w0 + (size_t)k * z + j] * X[off + k];
       off += z;
-      w0 += (size_t)z * z;
+      w0 += block_len(z);
       if (s > 2) {                        // (two elements can agree by chance)
         reduced += (long long)z * z;
         splits += z && z < s;

@@ -26,7 +26,7 @@ int main(int, char** argv) {
   std::atomic<int> done(0);
   left = k;
   try {
-    parallel_for(200, [&](int g) {
+    parallel_for<int>(200, 8, [&](int g, int&) {
       if (g == item) throw std::bad_alloc();
       ++done;
     });
