@@ -172,6 +172,30 @@ gemm_batched_kernel(int M, int N, int K, typename Scal<TC>::type alpha,
                                   ep.add ? ep.add + (b / ep.divAdd) * ep.sAdd : nullptr, As, Bs);
 }
 
+// The grouped contraction (gemm_grouped, tg_internal.h): C_g (angles x positions) = X_g W_g
+__global__ void __launch_bounds__(NT)
+gemm_grouped_kernel(int M, const cplx* __restrict__ X, cplx* __restrict__ C, int ld,
+                    const char* __restrict__ W, const GroupDesc* __restrict__ groups,
+                    const int* __restrict__ tile_group, const int* __restrict__ tile_j0) {
+  __shared__ cplx As[BK][BM + 1];
+  __shared__ double Bs[BK][BN + 1];
+  const int grp = tile_group[blockIdx.x];
+  if (grp < 0) return;
+  const GroupDesc g = groups[grp];
+  const int m0 = blockIdx.y * BM, j0 = tile_j0[blockIdx.x];
+  const cplx* Xg = X + (long long)g.off * ld;
+  cplx* Cg = C + (long long)g.off * ld;
+  const cplx one = cmk(1.0, 0.0), zero = cmk(0.0, 0.0);
+  if (g.fp32)
+    gemm_tile<cplx, float, cplx, OP_N, OP_T>(M, g.size, g.size, one, Xg, ld,
+                                             reinterpret_cast<const float*>(W + g.woff), g.size, zero,
+                                             false, Cg, ld, m0, j0, GemmEpi(), nullptr, As, Bs);
+  else
+    gemm_tile<cplx, double, cplx, OP_N, OP_T>(M, g.size, g.size, one, Xg, ld,
+                                              reinterpret_cast<const double*>(W + g.woff), g.size, zero,
+                                              false, Cg, ld, m0, j0, GemmEpi(), nullptr, As, Bs);
+}
+
 template <typename TA, typename TB, typename TC, int OPA, int OPB>
 int launch(hipStream_t s, int M, int N, int K, typename Scal<TC>::type alpha, const TA* A,
            int lda, long long sA, const TB* B, int ldb, long long sB,
@@ -412,6 +436,13 @@ int gemm_dd(hipStream_t s, TgOp opa, TgOp opb, int M, int N, int K, double alpha
 int gemm_grouped(hipStream_t s, int M, const cplx* X, cplx* C, int ld, const void* W,
                  const GroupDesc* groups_dev, const int* tile_group_dev, const int* tile_j0_dev,
                  int tag, int ntiles_total) {
+  if (M <= 0 || ntiles_total <= 0) return TG_OK;
+  if (!sel().mfma) {
+    hipLaunchKernelGGL(gemm_grouped_kernel, dim3(ntiles_total, (M + BM - 1) / BM), dim3(NT), 0, s, M, X,
+                       C, ld, (const char*)W, groups_dev, tile_group_dev, tile_j0_dev);
+    TG_HIP(hipGetLastError());
+    return TG_OK;
+  }
   return mfma_gemm_grouped(variant_for(GemmKey{K_GROUPED, tag, 0, M, ntiles_total, 0, 1}), s, M, X, C,
                            ld, W, groups_dev, tile_group_dev, tile_j0_dev, ntiles_total);
 }
