@@ -812,8 +812,7 @@ gradient_kernel(long long nn, double eta0, double mu0, const double* __restrict_
 int sign_pow(long long e) { return (e % 2 == 0) ? 1 : -1; }
 
 // per-item complex buffers of the loop body
-enum { W_UPHI, W_VPHI, W_UT, W_VT, W_RHO, W_KLR, W_KRL, W_G, W_H, W_DLR, W_DRL, W_T, W_X, W_Y,
-       W_Z, W_COUNT };
+enum { W_UPHI, W_VPHI, W_UT, W_VT, W_RHO, W_KLR, W_KRL, W_G, W_H, W_DLR, W_DRL, W_X, W_Y, W_COUNT };
 
 // Overlap shape of one state (calculate_overlap with state 0 = state 1,
 // :803-818): sizes, signfac and the prefactor of the reduced Pfaffian form.
@@ -1041,12 +1040,12 @@ int project_upload(tg_ctx* c) {
   TG_HIP(hipStreamSynchronize(s));   // host vectors go out of scope
 
   // first iteration at this size: autotune the tile shapes of the batched GEMMs
-  // of the loop body on zeroed scratch operands (W_T, W_X -> W_Y)
+  // of the loop body on zeroed scratch operands (W_H, W_X -> W_Y)
   const int chunk = P.chunk;
   if (c->tuned_n != n || c->tuned_chunk != chunk) {
     auto Wb = [&](int k) { return P.work + (size_t)k * chunk * nn; };
     const double* U = c->d_U.as<double>();
-    cplx* Ta = Wb(W_T);
+    cplx* Ta = Wb(W_H);
     cplx* Xa = Wb(W_X);
     cplx* Ya = Wb(W_Y);
     const long long tot = nn * chunk;
@@ -2403,7 +2402,7 @@ int observables_grid(tg_ctx* c, int nobo, const double* obo_ops, int nobos,
     const double* O2 = O + nn;
     cplx* X = Wb(W_X);
     cplx* Y = Wb(W_Y);
-    cplx* Z = Wb(W_Z);
+    cplx* Z = Wb(W_UPHI);                  // (free after the Thouless matrix)
     TG_TRY(gemm_dz(s, OP_N, OP_N, n, n, n, one, O, n, 0, rho, n, nn, zero, X, n, nn, A));
     TG_TRY(gemm_zd(s, OP_N, OP_N, n, n, n, one, kRL, n, nn, O, n, 0, zero, Y, n, nn, A));
     TG_TRY(gemm_dz(s, OP_N, OP_N, n, n, n, one, O, n, 0, kLR, n, nn, zero, Z, n, nn, A));
