@@ -53,15 +53,13 @@ def log(msg):
     print("[bench] " + msg, file=sys.stderr, flush=True)
 
 
-def algorithmic_flops(ctx_info, n, A, nb, fp32):
+def algorithmic_flops(blocks, n, A, nb):
     """Algorithmic FP64 flops per step (one projection of all A angles) of the
-    timed kernels (real flops; complex multiply-add = 8, real x complex = 4)."""
-    # the blocks split by the interaction's symmetries, when the elements are kept in
-    # FP32, leave a third (ph) and two thirds (pp) of the multiply-adds
-    ph, pp = (1.0 / 3.0, 2.0 / 3.0) if fp32 else (1.0, 1.0)
+    timed kernels (real flops; complex multiply-add = 8, real x complex = 4).
+    blocks: elements of the (ph, pp) blocks as the library reduced them."""
     return {
-        "kernel:grouped_ph": 4.0 * ctx_info["wph"] * A * ph,
-        "kernel:grouped_pp": 4.0 * ctx_info["wpp"] * 2 * A * pp,
+        "kernel:grouped_ph": 4.0 * blocks[0] * A,
+        "kernel:grouped_pp": 4.0 * blocks[1] * 2 * A,
         "kernel:gj_inverse": 8.0 * n ** 3 * A,
         "kernel:pfaffian": (4.0 / 3.0) * nb ** 3 * A,
         # complex batched GEMMs of the loop body on the main stream: A_phi (skew, half
@@ -88,19 +86,6 @@ def measured_traffic(workload, angles_per_launch, kernel):
         return None
     k = t.get("kernels", {}).get(kernel)
     return None if k is None else float(k["hbm_bytes_per_launch"])
-
-
-def contraction_sizes(h):
-    """sum of s_g^2 of the ph and pp block channels (as built by tg_init)."""
-    from collections import Counter
-    b = h["basis"]
-    m, t, l = b.sp_2mj.astype(int), b.sp_2mt.astype(int), b.sp_l.astype(int)
-    n = b.dim
-    x, y = np.meshgrid(np.arange(n), np.arange(n), indexing="ij")
-    ph = Counter(zip((m[x] - m[y]).ravel(), (t[x] - t[y]).ravel(), ((l[x] + l[y]) & 1).ravel()))
-    sel = x > y
-    pp = Counter(zip((m[x] + m[y])[sel], (t[x] + t[y])[sel], ((l[x] + l[y]) & 1)[sel]))
-    return dict(wph=float(sum(v * v for v in ph.values())), wpp=float(sum(v * v for v in pp.values())))
 
 
 FIXTURE = os.path.join(ROOT, "tests", "golden", "emax6.npz")
@@ -198,10 +183,11 @@ def iterate_gpu(args, ham, fix, plain, fp32, steps, warmup, timing=True, graph=F
                     "gemm_h20", "overlap", "thouless_inverse", "canonical_basis_beside"):
             kt[key] = ctx.timing(key)
         ctx.enable_timing(False)
+    blocks = ctx.contraction_size()
     ctx.close()
     n = ham["basis"].dim
     M = int(fix["Mphip"])
-    return dict(seconds=t1 - t0, steps=steps, timing=kt,
+    return dict(seconds=t1 - t0, steps=steps, timing=kt, blocks=blocks,
                 E_first=float((first["ener"] / first["over"]).real), first=first, n=n,
                 A=((M * M + 1) // 2 if conj_pairs else M * M),
                 nb=n - cb["nocc"] - cb["nemp"], adjust_steps=nadj, energies=energies,
@@ -430,7 +416,6 @@ def main():
     log("hamiltonian %s: n=%d, %d stored TBMEs (%.1f s), list %s the reference's"
         % (args.workload, ham["basis"].dim, len(ham["trperm"]), time.perf_counter() - t,
            "equal to" if same_list else "DIFFERENT FROM"))
-    sizes = contraction_sizes(ham)
     fp32 = args.tbme == "fp32"
 
     main_run = iterate_gpu(args, ham, fix, plain=False, fp32=fp32, steps=args.steps,
@@ -454,7 +439,7 @@ def main():
     # either stream
     n, A, nb = main_run["n"], main_run["A"], main_run["nb"]
     M = int(fix["Mphip"])
-    fl = algorithmic_flops(sizes, n, A, nb, fp32)
+    fl = algorithmic_flops(main_run["blocks"], n, A, nb)
     kern = {k: v for k, v in main_run["timing"].items() if k.startswith("kernel:") and v[1] > 0}
     roofline = None
     by_kernel = {}

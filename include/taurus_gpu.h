@@ -76,11 +76,18 @@ int tg_finalize(tg_ctx* ctx);
 int tg_set_mode(tg_ctx* ctx, int plain);
 
 /*
+ * tg_contraction_size -- matrix elements of the blocks that the contraction multiplies by,
+ * per channel (particle-hole, particle-particle), after their reduction by the symmetries
+ * that the interaction has: the multiply-adds of one set of densities, complex by real.
+ */
+int tg_contraction_size(tg_ctx* ctx, int64_t* ph, int64_t* pp);
+
+/*
  * tg_set_batch_limit -- at most max_items (state, angle) items per launch
  * sequence of the batched projection (0: no limit, the default).  Independently
  * of it, when the per-item work matrices of all items do not fit into the free
  * device memory, the projection runs the items chunk by chunk and keeps only
- * A_phi and H20_phi of every item for sum_gauge (the memory-short mode).  With
+ * A_phi and G of every item for sum_gauge (the memory-short mode; H20_phi = G - G^T).  With
  * several states a chunk holds whole states.  tg_project_observables needs all
  * angles at once and returns TG_E_NOMEM otherwise.
  */

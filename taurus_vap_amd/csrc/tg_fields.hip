@@ -413,6 +413,8 @@ int build_blocks(tg_ctx* c, int64_t ntb, const int16_t* abcd, const void* H2, in
     ch.npos = off;
     ch.ngroups = (int)groups.size();
     ch.norb = (int)orb.size();
+    ch.elements = 0;
+    for (const GroupDesc& d : groups) ch.elements += (long long)d.size * d.size;
     ch.mo = 1;
     for (const Orbit& o : orb) ch.mo = std::max(ch.mo, o.m);
     // (group, first position) of every 64-position tile, entry t for XCD t % 8: each

@@ -184,6 +184,7 @@ struct Channel {
   int npos = 0;                 // number of positions (n*n for ph, n(n-1)/2 for pp)
   int ngroups = 0, norb = 0;
   int mo = 1;                   // sums of an orbit at most
+  long long elements = 0;       // of all groups' W
   DevBuf d_orb, d_groups, d_W, d_tile_group, d_tile_n0;
   int ntiles_total = 0;
 };

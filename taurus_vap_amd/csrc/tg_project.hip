@@ -1890,6 +1890,16 @@ int tg_finalize(tg_ctx* c) {
   return TG_OK;
 }
 
+int tg_contraction_size(tg_ctx* c, int64_t* ph, int64_t* pp) {
+  if (!c || !ph || !pp) {
+    tg_set_error("tg_contraction_size: invalid argument");
+    return TG_E_ARG;
+  }
+  *ph = c->ph.elements;
+  *pp = c->pp.elements;
+  return TG_OK;
+}
+
 int tg_set_batch_limit(tg_ctx* c, int max_items) {
   if (!c || max_items < 0) {
     tg_set_error("tg_set_batch_limit: invalid argument");

@@ -42,6 +42,7 @@ EXPORTS = [
     "tg_set_batch_limit", "tg_canonical_basis", "tg_set_gradient_type",
     "tg_get_hsp_h11_eigenvalues", "tg_diagonalize_hsp_and_H11", "tg_sym_eigenvalues",
     "tg_zskpfa_noalloc", "tg_inverse", "tg_sym_eigensystem", "tg_iterate_canonical",
+    "tg_contraction_size",
 ]
 
 _lib = None
@@ -96,6 +97,7 @@ def load_library():
     lib.tg_group_iterate_results.argtypes = [P, I, P, P, P, P, P]
     lib.tg_project_observables.argtypes = [P, I, P, I, P, I, P, P, P]
     lib.tg_set_batch_limit.argtypes = [P, I]
+    lib.tg_contraction_size.argtypes = [P, P, P]
     lib.tg_canonical_basis.argtypes = [P, D, P, P, P, P]
     lib.tg_iterate_canonical.argtypes = [P, D, D, P, P, P, P, P, P, P, P, P]
     lib.tg_set_gradient_type.argtypes = [P, I]
@@ -161,6 +163,14 @@ class Context:
             self.close()
         except Exception:
             pass
+
+    def contraction_size(self):
+        """(ph, pp): elements of the contraction's blocks as the symmetries of the
+        interaction leave them (tg_contraction_size)."""
+        out = np.zeros(2, np.int64)
+        _check(load_library().tg_contraction_size(self._h, _p(out[:1]), _p(out[1:])),
+               "tg_contraction_size")
+        return int(out[0]), int(out[1])
 
     def set_batch_limit(self, max_items: int):
         """At most max_items (state, angle) items per launch sequence (0: all)."""
