@@ -1276,12 +1276,14 @@ int project_run(tg_ctx* c) {
     // The overlaps on the second stream.  Inverse and Pfaffian both take a CU per item
     // above order 64: beside each other while the items of both fit the CUs; with more of
     // them the inverses would wait for Pfaffians, which then start after the densities and
-    // run beside the contraction (225 items: 80 states 1.09 -> 0.99 ms a projection, 140
-    // states 2.42 -> 2.39).  Larger products fill the chip and lose as much to the Pfaffians
-    // as the inverses do (336 states 16.4 and 16.4; 156 items of 224 states 4.39 -> 4.53).
-    // A deferred basis keeps the wait: its overlaps, issued after the loop, gain by it alike
-    // (an iteration with 225 angles: 80 states 1.91 ms, without the wait 2.0; 140 states 3.53, 3.59).
-    const bool late = n > 64 && n <= 160 && 2 * na > 256;
+    // run beside the contraction.  A projection called by itself, 144 and 225 angles, first and
+    // after: 80 states 0.86 -> 0.77, 0.95 -> 0.87 ms, 108 1.20 -> 1.07, 1.51 -> 1.39, 140 1.88 ->
+    // 1.75, 2.36 -> 2.25 (the inverse's launches no longer queue behind the overlaps');
+    // projections that follow each other on the device 1 to 3 % longer (80 states 0.552, 0.558;
+    // 140 1.451, 1.493), iterations with a deferred basis 0.5 % shorter.  From 160 on a call gains
+    // nothing (2.20 and 2.17 on average) and the others lose 3 %: larger products fill the
+    // chip and lose to the Pfaffians what the inverses gain (156 angles of 224 states 4.39 -> 4.53).
+    const bool late = n > 64 && n <= 150 && 2 * na > 256;
     auto overlaps = [&]() -> int {
       if (!proj) {
         hipLaunchKernelGGL(fill_cplx_kernel, dim3(nblk(na)), dim3(NT), 0, s, na, cmk(1.0, 0.0),

@@ -1,4 +1,4 @@
-"""Overlaps that start after the densities: orders of 66 to 160 with more than 128 angles at
+"""Overlaps that start after the densities: orders of 66 to 150 with more than 128 angles at
 once.  80 states with 12 x 12 angles against the same with a batch limit of 128 and of 37
 items, where they start first; eager and as a captured graph, with the parity overlaps, and
 with the canonical basis deferred to the second stream.  The runs add the same numbers in
