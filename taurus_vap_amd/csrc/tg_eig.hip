@@ -807,7 +807,8 @@ int tridiag_launch(hipStream_t s, int n, const double* A, int lda, long long sA,
 }
 
 // Eigenvalues of tridiagonal matrices by multisection on Sturm counts, to the
-// resolution of the floating-point numbers.  A group of SG lanes takes one
+// resolution of the floating-point numbers or 2^-261 of the Gershgorin interval (64
+// passes), whichever is coarser.  A group of SG lanes takes one
 // eigenvalue index: each lane counts at one of SG points inside the bracket, so
 // a pass over the matrix leaves 1/(SG+1) of it (4.1 bits for SG = 16 against one
 // for a bisection); the counts are a serial chain of divisions, so the time is
@@ -862,7 +863,8 @@ sturm_kernel(int n, const double* __restrict__ d0, const double* __restrict__ e0
     if (f > 0) lo = fmax(lo, xl);
     if (f < SG) hi = fmin(hi, xh);
   }
-  // the counts do not resolve values within the pivot guard: these are zero
+  // the counts do not resolve values within the pivot guard (an interval of this width, that
+  // of a zero matrix say): these are zero
   const double wv = 0.5 * (lo + hi);
   if (g == 0 && i < n) w0[blockIdx.y * ws + i] = (fabs(wv) <= 2.0 * pivmin) ? 0.0 : wv;
 }

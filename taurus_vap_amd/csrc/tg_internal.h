@@ -64,6 +64,14 @@ __host__ __device__ inline void cfms(cplx& a, cplx b, cplx c) {
   a.y = fma(-b.x, c.y, fma(-b.y, c.x, a.y));
 }
 
+// v of a lane that is the same in the whole wave
+__device__ __forceinline__ double readlane_f64(double v, int lane) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)(unsigned long long)b, lane);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+
 // ---------------------------------------------------------------------------
 // Device buffer helper
 // ---------------------------------------------------------------------------
@@ -370,7 +378,6 @@ inline size_t sym_eigvals_work(int n, int count) { return (size_t)count * ((size
 // The resident U, V, D and c->st of c->ns states are set: the tail of
 // tg_set_states (Z buffers, gauge grid, state marked for the set-up upload).
 int tg_states_ready(tg_ctx* c);
-// releases the rocBLAS handle of the device canonical basis
 
 int contraction_build(tg_ctx* c, int64_t ntb, const int16_t* abcd, const void* H2,
                       int h2_bytes, const int8_t* trperm);

@@ -209,13 +209,6 @@ chol_block_kernel(int n, int k0, int b, const double* __restrict__ A0, double* _
 constexpr int CF_B = 32, CF_NW = 8, CF_TH = 64 * CF_NW, CF_NMAX = 512;
 inline int cf_zp(int n) { return (n + 31) / 32 * 32 + 16; }   // rows of Z 16 banks apart
 
-__device__ __forceinline__ double cf_readlane(double v, int lane) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane((int)(unsigned long long)b, lane);
-  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
-  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
-}
-
 // Wave 0: factor of the diagonal block at k0 (b of its 32 rows inside the matrix, the
 // unit matrix past them), its inverse to Xd (Xd[i][j] = L_kk^-1(i, j), zero above the diagonal)
 __device__ __forceinline__ void cf_diagonal(const double* M, int n, int k0, int lane,
@@ -233,7 +226,7 @@ __device__ __forceinline__ void cf_diagonal(const double* M, int n, int k0, int 
   double scale = 1.0;                            // 1 / L(i, i)
 #pragma unroll
   for (int k = 0; k < CF_B; ++k) {
-    double d = cf_readlane(v[k], k);
+    double d = readlane_f64(v[k], k);
     if (!(d > 0.0)) {
       if (bad == 0) bad = k0 + k + 1;
       d = 1.0;
@@ -248,8 +241,8 @@ __device__ __forceinline__ void cf_diagonal(const double* M, int n, int k0, int 
     const double ma = up ? 0.0 : -l, mb = (up && i > k) ? -li * rd : 0.0;
 #pragma unroll
     for (int j = 0; j < CF_B; ++j)
-      v[j] = (j > k) ? fma(ma, cf_readlane(l, j), v[j])
-                     : fma(mb, cf_readlane(v[j], CF_B + k), v[j]);
+      v[j] = (j > k) ? fma(ma, readlane_f64(l, j), v[j])
+                     : fma(mb, readlane_f64(v[j], CF_B + k), v[j]);
 #pragma unroll
     for (int j = 0; j < CF_B; ++j) asm volatile("" : "+v"(v[j]));   // here, not at their use
     __builtin_amdgcn_sched_barrier(0);

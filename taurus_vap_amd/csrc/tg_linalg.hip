@@ -686,13 +686,6 @@ __device__ __forceinline__ unsigned gj_wave_umax(unsigned v) {
   return __builtin_amdgcn_readlane(v, W - 1);
 }
 
-__device__ __forceinline__ double gj_readlane(double v, int lane) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane((int)(unsigned long long)b, lane);
-  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
-  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
-}
-
 // The lane (of lanes 0 .. W-1) with the largest v, the smallest label on ties; -1 if no
 // v is positive.  Compared by its bits: the upper words decide nearly
 // always, the lower words and the labels are looked at only when they tie.  NaN is no
@@ -799,13 +792,13 @@ gj_small_kernel(int n, cplx* __restrict__ Aall, int lda, long long sA, cplx* __r
         gj_rotate(pr);
         continue;
       }
-      const cplx piv = cmk(gj_readlane(pr[0].x, p), gj_readlane(pr[0].y, p));
+      const cplx piv = cmk(readlane_f64(pr[0].x, p), readlane_f64(pr[0].y, p));
       if (L != k) d = cmk(-d.x, -d.y);
       d = cmul(d, piv);
       cplx r[16];
 #pragma unroll
-      for (int j = 1; j < 16; ++j) r[j] = cmk(gj_readlane(pr[j].x, p), gj_readlane(pr[j].y, p));
-      gj_eliminate(pr, cmk(gj_readlane(mine.x, p), gj_readlane(mine.y, p)), t == p,
+      for (int j = 1; j < 16; ++j) r[j] = cmk(readlane_f64(pr[j].x, p), readlane_f64(pr[j].y, p));
+      gj_eliminate(pr, cmk(readlane_f64(mine.x, p), readlane_f64(mine.y, p)), t == p,
                    [&](int j) { return r[j]; });
     }
     __syncthreads();
@@ -1718,7 +1711,7 @@ int batched_inverse(hipStream_t s, int n, cplx* A, int lda, long long sA, int ba
                      lda, sA, det, info, perm)
     if (rp == 2 && n <= 384)
       TG_GJ_LAUNCH(2, 384, GJ_WIN);
-    // the LDS of a CU holds three matrices of order 48 or two of order 64: past two
+    // the LDS of a CU holds four matrices of order 48 or two of order 64: past two
     // rounds of the latter the 16-column kernel, which shares a CU among more waves, is
     // ahead (order 64, 400 matrices: 142 against 242 us; 1296: 418 against 322)
     else if (rp != 1 && (n <= 48 || (n <= GJ_SMALL && batch <= 2 * CUS)))
