@@ -87,9 +87,9 @@ inline unsigned nblk(long long tot) { return (unsigned)((tot + NT - 1) / NT); }
 // exact[s] becomes 0 where state s is not a Bogoliubov transformation to rounding, that is
 // where an element of U^T U + V^T V - 1 or V^T U + (V^T U)^T exceeds TG_EXACT_TOL.
 // A_phi and the pairing tensors of such a state are not skew, and what takes half of them
-// for the whole would change the results by a hundred to a thousand times its error (80
-// angles, noise of 1e-8 on U and V: 7e-7 on H20).  States read, evolved or built by this library
-// stay below 1e-14 (seeds 2e-15, after 400 steps 6e-15).
+// for the whole would change the results by a hundred to a thousand times its error (24
+// states, noise of 1e-8 on U and V: 7e-7 on H20).  Seeds and evolved states stay below 1e-14
+// (2e-15; after 400 steps 6e-15).
 constexpr double TG_EXACT_TOL = 2.8e-14;
 constexpr int UV_AG = 16;
 __global__ void build_uv_phi_kernel(int n, int na, long long b0, int A, int S,
