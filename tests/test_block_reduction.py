@@ -164,8 +164,9 @@ def program(tmp_path_factory):
     d = tmp_path_factory.mktemp("blocks")
     src, exe = d / "b.cpp", d / "b"
     src.write_text(PROGRAM)
-    subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-fsanitize=undefined", "-fno-sanitize-recover", "-D_GLIBCXX_ASSERTIONS", "-I", CSRC, str(src),
-                    "-o", str(exe)], check=True)
+    flags = ["-std=c++17", "-O1", "-g", "-fsanitize=undefined", "-fno-sanitize-recover",
+             "-D_GLIBCXX_ASSERTIONS", "-I", CSRC]
+    subprocess.run(["g++", *flags, str(src), "-o", str(exe)], check=True)
     return str(exe)
 
 
